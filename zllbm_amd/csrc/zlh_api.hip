@@ -234,6 +234,58 @@ __global__ void k_materialize(BrickLevel<T> lv, const int32_t *node_slot, const 
     for (int q = 0; q < Q; ++q) out[q * n + i] = post_stream_value<D, T, SHIFT>(lv, slot, ai, q, last, aux_f, fresh);
 }
 
+// Post-stream populations of the nodes [i0, i0 + m), [m][Q] double in key order (unshifted), into
+// pinned host memory: the rows go through LDS, so that a wavefront's stores to the host are whole
+// runs.  Bound by the host link (152 B per D3Q19 node).
+template <int D, typename T, bool SHIFT>
+__global__ __launch_bounds__(128) void k_rows_out(BrickLevel<T> lv, const int32_t *node_slot, const int32_t *node_aux,
+                                                  int64_t i0, int64_t m, const T *last, const T *aux_f, int fresh,
+                                                  double *__restrict__ out) {
+    constexpr int Q = Lattice<D>::Q;
+    __shared__ double tile[128 * Q];
+    const int64_t r0 = (int64_t)blockIdx.x * 128;
+    const int64_t r = r0 + threadIdx.x;
+    if (r < m) {
+        const int32_t ai = node_aux[i0 + r];
+        const int64_t slot = node_slot[i0 + r];
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            tile[threadIdx.x * Q + q] = post_stream_value<D, T, SHIFT>(lv, slot, ai, q, last, aux_f, fresh);
+    }
+    __syncthreads();
+    const int ne = (int)(m - r0 < 128 ? m - r0 : 128) * Q;
+    for (int e = threadIdx.x; e < ne; e += 128) out[r0 * Q + e] = tile[e];
+}
+
+// Density and velocity (rho [m], then u [m][D]) of the post-stream populations of the same nodes,
+// into pinned host memory, summed in double in direction order as the reference sums them
+// (CalMacro*, lbm_solver_interface.cpp:477-592).  (1 + D) 8 bytes of a node cross the host link
+// where its populations are 8 Q: the 3.29M nodes of a four-level D3Q19 grid take 8.6 ms, host
+// copy included (12 GB/s, bound by the page faults of a fresh destination), where downloading the
+// populations and summing them on the host took 269 ms.
+template <int D, typename T, bool SHIFT>
+__global__ __launch_bounds__(256) void k_macros_out(BrickLevel<T> lv, const int32_t *node_slot, const int32_t *node_aux,
+                                                    int64_t i0, int64_t m, const T *last, const T *aux_f, int fresh,
+                                                    int compressible, double *__restrict__ rho, double *__restrict__ u) {
+    using L = Lattice<D>;
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (r >= m) return;
+    const int32_t ai = node_aux[i0 + r];
+    const int64_t slot = node_slot[i0 + r];
+    double s = post_stream_value<D, T, SHIFT>(lv, slot, ai, 0, last, aux_f, fresh);
+    double j[3] = {0., 0., 0.};
+#pragma unroll
+    for (int q = 1; q < L::Q; ++q) {
+        const double v = post_stream_value<D, T, SHIFT>(lv, slot, ai, q, last, aux_f, fresh);
+        s += v;
+        j[0] += L::cx[q] * v;
+        j[1] += L::cy[q] * v;
+        if (D == 3) j[2] += L::cz[q] * v;
+    }
+    rho[r] = s;
+    for (int a = 0; a < D; ++a) u[r * D + a] = compressible ? j[a] / s : j[a];
+}
+
 __global__ void k_sum4(const double *fq, int64_t n, int Q, const int *cx, const int *cy, const int *cz,
                        double *acc) {
     __shared__ double sh[4][256];
@@ -418,6 +470,11 @@ struct zlh_ctx {
     double timing_ms[16] = {};       // per level
     int64_t timing_launches[16] = {};
     DevBuf lattice_d;
+    // pinned staging of the downloads (download_nodes): two halves, grown to what a call needs up
+    // to 2 kStageBytes, freed with the context
+    char *stage = nullptr;
+    size_t stage_bytes = 0;
+    hipEvent_t ev_stage[2] = {nullptr, nullptr};
     DevBuf mlp_d;           // MlpDev of the learned closure
     bool mlp_set = false;
     int mlp_train_form = ZLH_MLP_FP32;   // kernel of zlh_mlp_gradient / zlh_mlp_train
@@ -826,6 +883,82 @@ zlh_status do_materialize(zlh_ctx *ctx, int level, double *out_dev) {
                        : dispatch_materialize<3, float, true>(ctx, level, out_dev);
 }
 
+// Downloads of a level's nodes: a kernel writes a chunk of nodes into one half of a pinned buffer
+// while the host copies the other half into the caller's array, so that no device workspace is
+// allocated and the only bytes over the host link are those returned.  kStageBytes: chunks of
+// 4 MiB keep both sides busy and the buffer small.  A 33^2 macros call takes 28 us where
+// allocating, copying and freeing device memory took 82.
+constexpr size_t kStageBytes = 4u << 20;
+
+zlh_status stage_reserve(zlh_ctx *ctx, size_t bytes) {
+    if (ctx->stage_bytes >= bytes) return ZLH_OK;
+    if (ctx->stage) {
+        ZLH_TRY(hipStreamSynchronize(ctx->stream));   // a failed call may have left a chunk in flight
+        (void)hipHostFree(ctx->stage);
+        ctx->stage = nullptr;
+        ctx->stage_bytes = 0;
+    }
+    void *p = nullptr;
+    const hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocCoherent);
+    if (e != hipSuccess) return ctx->fail(ZLH_ENOMEM, "hipHostMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    ctx->stage = static_cast<char *>(p);
+    ctx->stage_bytes = bytes;
+    return ZLH_OK;
+}
+
+template <int D, typename T, bool SHIFT>
+zlh_status download_nodes_t(zlh_ctx *ctx, int level, double *f, double *rho, double *u) {
+    LevelState &L = ctx->lv[level];
+    BrickLevel<T> v = view<T>(L);
+    // the buffer read by the last fused kernel (or, before any step, the uploaded populations)
+    const T *last = L.f_d[L.cur ^ 1].as<T>();
+    const int32_t *slots = L.node_slot_d.as<int32_t>(), *auxs = L.node_aux_d.as<int32_t>();
+    constexpr int Q = Lattice<D>::Q;
+    const int64_t per = f ? Q : 1 + D;                    // doubles per node
+    const int64_t chunk = std::min<int64_t>(L.n, (int64_t)(kStageBytes / 8) / per);
+    const size_t half = ((size_t)(chunk * per) * 8 + 255) & ~(size_t)255;
+    const int64_t nchunk = (L.n + chunk - 1) / chunk;
+    zlh_status s = stage_reserve(ctx, nchunk > 1 ? 2 * half : half);
+    if (s) return s;
+    auto fill = [&](int64_t c) -> hipError_t {
+        const int64_t i0 = c * chunk, m = std::min(chunk, L.n - i0);
+        double *dst = reinterpret_cast<double *>(ctx->stage + (c & 1) * half);
+        if (f)
+            hipLaunchKernelGGL((k_rows_out<D, T, SHIFT>), dim3(blocks(m, 128)), dim3(128), 0, ctx->stream, v, slots, auxs,
+                               i0, m, last, L.aux_f_d.as<T>(), L.fresh ? 1 : 0, dst);
+        else
+            hipLaunchKernelGGL((k_macros_out<D, T, SHIFT>), dim3(blocks(m)), dim3(256), 0, ctx->stream, v, slots, auxs,
+                               i0, m, last, L.aux_f_d.as<T>(), L.fresh ? 1 : 0, ctx->d.compressible, dst, dst + m);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess ? e : hipEventRecord(ctx->ev_stage[c & 1], ctx->stream);
+    };
+    ZLH_TRY(fill(0));
+    for (int64_t c = 0; c < nchunk; ++c) {
+        if (c + 1 < nchunk) ZLH_TRY(fill(c + 1));
+        ZLH_TRY(hipEventSynchronize(ctx->ev_stage[c & 1]));
+        const int64_t i0 = c * chunk, m = std::min(chunk, L.n - i0);
+        const double *src = reinterpret_cast<const double *>(ctx->stage + (c & 1) * half);
+        if (f) {
+            std::memcpy(f + i0 * Q, src, sizeof(double) * m * Q);
+        } else {
+            std::memcpy(rho + i0, src, sizeof(double) * m);
+            std::memcpy(u + i0 * D, src + m, sizeof(double) * m * D);
+        }
+    }
+    return ZLH_OK;
+}
+
+// populations f [n][Q], or (f null) density rho [n] and velocity u [n][dims], in key order
+zlh_status download_nodes(zlh_ctx *ctx, int level, double *f, double *rho, double *u) {
+    if (ctx->d.dims == 2)
+        return ctx->fp64() ? download_nodes_t<2, double, false>(ctx, level, f, rho, u)
+             : ctx->bf16() ? download_nodes_t<2, bf16_t, true>(ctx, level, f, rho, u)
+                           : download_nodes_t<2, float, true>(ctx, level, f, rho, u);
+    return ctx->fp64() ? download_nodes_t<3, double, false>(ctx, level, f, rho, u)
+         : ctx->bf16() ? download_nodes_t<3, bf16_t, true>(ctx, level, f, rho, u)
+                       : download_nodes_t<3, float, true>(ctx, level, f, rho, u);
+}
+
 // feq of given macros (double, unshifted) [n][Q]
 void host_feq(int dims, double rho, const double *u, int compressible, double *feq) {
     const int Q = dims == 2 ? 9 : 19;
@@ -1080,6 +1213,8 @@ zlh_status zlh_create(const zlh_solver_desc *desc, zlh_ctx **out) {
     ctx->ev_join.assign(nl, nullptr);
     ctx->ev_rows.assign(nl, nullptr);
     if (hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess) return ZLH_EDEVICE;
+    for (hipEvent_t &e : ctx->ev_stage)
+        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return ZLH_EDEVICE;
     for (int l = 0; l < nl; ++l)
         if (hipStreamCreate(&ctx->lstream[l]) != hipSuccess ||
             hipEventCreateWithFlags(&ctx->ev_step[l], hipEventDisableTiming) != hipSuccess ||
@@ -1113,6 +1248,9 @@ void zlh_destroy(zlh_ctx *ctx) {
         for (hipEvent_t e : *v)
             if (e) (void)hipEventDestroy(e);
     if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
+    for (hipEvent_t e : ctx->ev_stage)
+        if (e) (void)hipEventDestroy(e);
+    if (ctx->stage) (void)hipHostFree(ctx->stage);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -1549,41 +1687,14 @@ zlh_status zlh_download_populations(zlh_ctx *ctx, int level, double *f) {
     if (!ctx) return ZLH_EINVAL;
     if (!ctx->built) return ctx->fail(ZLH_ESTATE, "not built");
     if (level < 0 || level > ctx->d.max_level || !f) return ctx->fail(ZLH_EINVAL, "bad download arguments");
-    LevelState &L = ctx->lv[level];
-    const int Q = ctx->q;
-    DevBuf tmp;
-    zlh_status s = dalloc(ctx, tmp, sizeof(double) * L.n * Q, false);
-    if (s) return s;
-    if ((s = do_materialize(ctx, level, tmp.as<double>()))) return s;
-    std::vector<double> h((size_t)L.n * Q);
-    ZLH_TRY(hipMemcpyAsync(h.data(), tmp.p, sizeof(double) * L.n * Q, hipMemcpyDeviceToHost, ctx->stream));
-    ZLH_TRY(hipStreamSynchronize(ctx->stream));
-    for (int64_t i = 0; i < L.n; ++i)
-        for (int q = 0; q < Q; ++q) f[i * Q + q] = h[(size_t)q * L.n + i];
-    return ZLH_OK;
+    return download_nodes(ctx, level, f, nullptr, nullptr);
 }
 
 zlh_status zlh_download_macros(zlh_ctx *ctx, int level, double *rho, double *u) {
     if (!ctx) return ZLH_EINVAL;
     if (level < 0 || level > ctx->d.max_level || !rho || !u) return ctx->fail(ZLH_EINVAL, "bad download arguments");
-    LevelState &L = ctx->lv[level];
-    const int Q = ctx->q, dims = ctx->d.dims;
-    std::vector<double> f((size_t)L.n * Q);
-    zlh_status s = zlh_download_populations(ctx, level, f.data());
-    if (s) return s;
-    for (int64_t i = 0; i < L.n; ++i) {
-        double r = f[i * Q], j[3] = {0, 0, 0};
-        for (int q = 1; q < Q; ++q) {
-            const double v = f[i * Q + q];
-            r += v;
-            j[0] += (dims == 2 ? Lattice<2>::cx[q] : Lattice<3>::cx[q]) * v;
-            j[1] += (dims == 2 ? Lattice<2>::cy[q] : Lattice<3>::cy[q]) * v;
-            if (dims == 3) j[2] += Lattice<3>::cz[q] * v;
-        }
-        rho[i] = r;
-        for (int a = 0; a < dims; ++a) u[i * dims + a] = ctx->d.compressible ? j[a] / r : j[a];
-    }
-    return ZLH_OK;
+    if (!ctx->built) return ctx->fail(ZLH_ESTATE, "not built");
+    return download_nodes(ctx, level, nullptr, rho, u);
 }
 
 zlh_status zlh_download_source_table(zlh_ctx *ctx, int level, int32_t *src) {
