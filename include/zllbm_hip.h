@@ -220,12 +220,12 @@ zlh_status zlh_mlp_gradient(zlh_ctx *ctx, const float *params, const float *x, c
                             float *grad, float *loss);
 /* zlh_mlp_gradient without any device allocation.  No counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture, tight training
- * loops, harnesses that forbid hipMalloc).  The parameters, samples, targets and the gradient
- * and loss accumulators are staged in one static device array of the library, 2.6 MiB per GPU,
+ * loops, harnesses that forbid hipMalloc).  The parameters, samples, targets, partial sums and
+ * the gradient and loss are staged in one static device array of the library, 3.9 MiB per GPU,
  * held until the process ends; it holds at most ZLH_MLP_NOALLOC_MAX_SAMPLES samples, and a
  * larger n returns ZLH_EINVAL.  Same arguments, kernel (zlh_mlp_training_form) and results as
  * zlh_mlp_gradient.  Every call on one GPU uses that GPU's one array, which keeps the last
- * call's contents (each call clears its accumulators first): calls that overlap on one GPU,
+ * call's contents (each call writes all that it reads first): calls that overlap on one GPU,
  * from several threads or contexts, race. */
 #define ZLH_MLP_NOALLOC_MAX_SAMPLES 65536
 zlh_status zlh_mlp_gradient_noalloc(zlh_ctx *ctx, const float *params, const float *x, const float *t,
@@ -238,9 +238,9 @@ zlh_status zlh_mlp_train(zlh_ctx *ctx, const float *x, const float *t, int64_t n
 /* network forms: FP32 on the vector units (the FP64 solver's collision) and BF16 operands with
  * FP32 accumulation on the matrix cores, 64 nodes per wavefront (the FP32 solver's collision) */
 enum { ZLH_MLP_FP32 = 0, ZLH_MLP_BF16_MFMA = 1, ZLH_MLP_FP16_MFMA = 2 };
-/* kernel of zlh_mlp_gradient and zlh_mlp_train: ZLH_MLP_FP32 (default; FP32 on the vector units,
- * one thread per sample) or ZLH_MLP_BF16_MFMA (forward and backward of 64 samples per wavefront
- * on the matrix cores, BF16 operands and FP32 accumulation); ZLH_EINVAL for any other form */
+/* kernel of zlh_mlp_gradient and zlh_mlp_train: ZLH_MLP_FP32 (default; FP32 operands, products
+ * and sums) or ZLH_MLP_BF16_MFMA (BF16 operands and FP32 accumulation); ZLH_EINVAL for any other
+ * form.  Without BF16 a gradient depends on its inputs alone, bit for bit. */
 zlh_status zlh_mlp_training_form(zlh_ctx *ctx, int form);
 /* network output (nu_t / nu_scale) of normalised inputs [n][9] with the parameters set by
  * zlh_mlp_set, in the given form */

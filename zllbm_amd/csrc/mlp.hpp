@@ -397,9 +397,16 @@ __global__ __launch_bounds__(256) void k_mlp_eval_wave(const MlpDev *m, const fl
 }
 
 // ---------------------------------------------------------------------------------------------
-// training: one thread per sample, forward + backward in FP32, wavefront-reduced gradients
-// accumulated with atomics; Adam update over the flat parameter vector
+// training: gradient kernels, their reduction, and the Adam update over the flat parameter vector.
+// A gradient workgroup writes the sums of its samples as one row of `part` ([workgroup][kGradRow]:
+// the gradient in parameter order, then the loss); k_grad_reduce adds the rows in workgroup order,
+// so a gradient depends on its inputs alone (no floating-point atomics between workgroups) and no
+// accumulator has to be cleared first.
 // ---------------------------------------------------------------------------------------------
+constexpr int kGradRow = 1412;       // kMlpParams + 1, rounded up to 16 bytes
+constexpr int kGradMaxBlocks = 256;  // rows: one workgroup per CU loops over a larger batch
+static_assert(kGradRow >= kMlpParams + 1, "a row holds the gradient and the loss");
+
 __device__ __forceinline__ float wave_sum_f(float v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
@@ -410,74 +417,214 @@ __device__ __forceinline__ uint32_t hash32(uint32_t x) {
     return x;
 }
 
-// gradient of mean((softplus(net(x)) - t)^2) over a batch; idx == nullptr uses samples 0..batch-1,
-// otherwise sample k of the batch is (hash(seed, k) mod n)
+// sample k of a batch: k itself, or with `random` (hash(seed, k) mod n); n <= 2^26
+__device__ __forceinline__ int64_t batch_sample(int k, uint32_t seed, int random, int64_t n) {
+    return random ? (int64_t)(hash32(seed * 2654435761u + (uint32_t)k) % (uint32_t)n) : (int64_t)k;
+}
+
+__device__ __forceinline__ float dsilu(float z, float sg) { return sg * (1.f + z * (1.f - sg)); }
+
+// orders a wavefront's LDS writes before its later LDS reads of other lanes' values
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Gradient of mean((softplus(net(x)) - t)^2) in FP32: products and sums of every layer as
+// v_mfma_f32_32x32x2f32 (exact FP32 products, FP32 accumulation), activations in FP32.  A
+// wavefront takes 32 samples, one per column; lane l = 32 h + c holds rows mfma_row(h, r) of
+// column c.
+//   forward    H^T[32 x 32 samples] = W . (...)^T: K step r of layer 2 takes units mfma_row(0, r)
+//              and mfma_row(1, r), so that accumulators feed the next product from their registers;
+//              the accumulators start from the biases
+//   backward   D1^T = W2^T . D2 the same way
+//   gradients  dW2 = D2 . H1^T and [dW1 | db1] = D1 . [X | 1] contract over the samples: both
+//              operands are turned around through a per-wavefront LDS tile (row stride 36 floats:
+//              16-byte reads of a row's half); the bias and output-weight gradients are the row
+//              sums of the same reads
+// 69 products of 64 cycles per 32 samples.  A batch of 4,096 takes 11.2 us (32 workgroups, bound by
+// the latency of one tile) and 2^20 samples 0.25 ms (4.1 G samples/s, bound by the matrix pipe and
+// its dependent chains at one wavefront per SIMD); one sample per lane with a wavefront reduction
+// and an atomic per parameter (1,409 of each) took 403 us and 8.4 ms.
+constexpr int kTileStride = 36;
+struct alignas(16) GradTilesF {
+    float d[kMlpH][kTileStride];     // layer delta [hidden][sample]: D2, then D1
+    float h[kMlpH][kTileStride];     // layer-1 activations [hidden][sample], then dz3 h2
+    float x[kMlpF][kTileStride];     // inputs [feature][sample]
+};
+
 __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ params, const float *__restrict__ X,
                                                   const float *__restrict__ T, int64_t n, int batch, uint32_t seed,
-                                                  int random, float *__restrict__ grad, float *__restrict__ loss) {
-    __shared__ float sp[kMlpParams];
-    for (int i = threadIdx.x; i < kMlpParams; i += blockDim.x) sp[i] = params[i];
-    __syncthreads();
-    const float *W1 = sp, *b1 = W1 + kMlpH * kMlpF, *W2 = b1 + kMlpH, *b2 = W2 + kMlpH * kMlpH;
+                                                  int random, float *__restrict__ part) {
+    __shared__ union {
+        GradTilesF tiles[4];
+        float sums[4][kGradRow];   // after the loop
+    } sh;
+    const int lane = __lane_id(), h = lane >> 5, col = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    GradTilesF &tl = sh.tiles[wave];
+    const float *W1 = params, *b1 = W1 + kMlpH * kMlpF, *W2 = b1 + kMlpH, *b2 = W2 + kMlpH * kMlpH;
     const float *w3 = b2 + kMlpH;
+    // A operands: row `col` of W1 (K slots 2 s + h), of W2 and of W2^T (K slots mfma_row(h, r))
+    float a1[5], a2[16], at[16], w3r[16];
+    f32x16_t z1_0, z2_0;
+#pragma unroll
+    for (int s = 0; s < 5; ++s) a1[s] = 2 * s + h < kMlpF ? W1[col * kMlpF + 2 * s + h] : 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int row = mfma_row(h, r);
+        a2[r] = W2[col * kMlpH + row];
+        at[r] = W2[row * kMlpH + col];
+        w3r[r] = w3[row];
+        z1_0[r] = b1[row];
+        z2_0[r] = b2[row];
+    }
     const float b3 = w3[kMlpH];
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool active = k < batch;
-    int64_t s = 0;
-    if (active) s = random ? (int64_t)(hash32(seed * 2654435761u + (uint32_t)k) % (uint64_t)n) : k;
-    float x[kMlpF], z1[kMlpH], h1[kMlpH], z2[kMlpH];
-    for (int i = 0; i < kMlpF; ++i) x[i] = active ? X[s * kMlpF + i] : 0.f;
-    for (int j = 0; j < kMlpH; ++j) {
-        float z = b1[j];
-        for (int i = 0; i < kMlpF; ++i) z += W1[j * kMlpF + i] * x[i];
-        z1[j] = z;
-        h1[j] = z * sigmoidf_(z);
-    }
-    float z3 = b3;
-    for (int j = 0; j < kMlpH; ++j) {
-        float z = b2[j];
-        for (int i = 0; i < kMlpH; ++i) z += W2[j * kMlpH + i] * h1[i];
-        z2[j] = z;
-        z3 += w3[j] * (z * sigmoidf_(z));
-    }
-    const float y = softplusf_(z3);
-    const float t = active ? T[s] : 0.f;
     const float inv_b = 1.f / (float)batch;
-    const float dz3 = active ? 2.f * (y - t) * inv_b * sigmoidf_(z3) : 0.f;
-    const float lsum = wave_sum_f(active ? (y - t) * (y - t) * inv_b : 0.f);
-    const int lane = threadIdx.x & 63;
-    if (lane == 0) atomicAdd(loss, lsum);
-    // layer 3
-    float *gW1 = grad, *gb1 = gW1 + kMlpH * kMlpF, *gW2 = gb1 + kMlpH, *gb2 = gW2 + kMlpH * kMlpH;
-    float *gw3 = gb2 + kMlpH;
-    float g = wave_sum_f(dz3);
-    if (lane == 0) atomicAdd(&gw3[kMlpH], g);
-    float dz2[kMlpH];
-    for (int j = 0; j < kMlpH; ++j) {
-        const float sg = sigmoidf_(z2[j]);
-        const float h2 = z2[j] * sg;
-        g = wave_sum_f(dz3 * h2);
-        if (lane == 0) atomicAdd(&gw3[j], g);
-        dz2[j] = dz3 * w3[j] * sg * (1.f + z2[j] * (1.f - sg));
-        g = wave_sum_f(dz2[j]);
-        if (lane == 0) atomicAdd(&gb2[j], g);
+    f32x16_t gw2 = {}, gw1 = {};
+    float gw3 = 0.f, gb2 = 0.f, gb3 = 0.f, lsum = 0.f;
+    // columns past the batch carry zero inputs and a zero output delta, so they add nothing
+    for (int64_t base = (int64_t)blockIdx.x * 128 + wave * 32; base < batch; base += (int64_t)gridDim.x * 128) {
+        const int64_t k = base + col;
+        const bool active = k < batch;
+        const int64_t s = active ? batch_sample((int)k, seed, random, n) : 0;
+        float xv[5];
+#pragma unroll
+        for (int e = 0; e < 5; ++e) xv[e] = active && 2 * e + h < kMlpF ? X[s * kMlpF + 2 * e + h] : 0.f;
+        const float t = active ? T[s] : 0.f;
+        f32x16_t z1 = z1_0;
+#pragma unroll
+        for (int e = 0; e < 5; ++e) z1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[e], xv[e], z1, 0, 0, 0);
+        float s1[16], g1[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            s1[r] = sigmoidf_(z1[r]);
+            g1[r] = z1[r] * s1[r];
+            tl.h[mfma_row(h, r)][col] = g1[r];
+        }
+#pragma unroll
+        for (int e = 0; e < 5; ++e)
+            if (2 * e + h < kMlpF) tl.x[2 * e + h][col] = xv[e];
+        f32x16_t z2 = z2_0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[r], g1[r], z2, 0, 0, 0);
+        float s2[16], p = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            s2[r] = sigmoidf_(z2[r]);
+            p += w3r[r] * (z2[r] * s2[r]);
+        }
+        // both halves of a column hold the sample's output
+        const float z3 = b3 + (p + swap_halves(p));
+        const float y = softplusf_(z3);
+        const float dz3 = active ? 2.f * (y - t) * inv_b * sigmoidf_(z3) : 0.f;
+        if (h == 0) {
+            lsum += active ? (y - t) * (y - t) * inv_b : 0.f;
+            gb3 += dz3;
+        }
+        float d2[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            d2[r] = dz3 * w3r[r] * dsilu(z2[r], s2[r]);
+            tl.d[mfma_row(h, r)][col] = d2[r];
+        }
+        wave_lds_sync();
+        // row `col`, samples 16 h .. 16 h + 15 (K slot t of both operands is sample 16 h + t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 A = *reinterpret_cast<const float4 *>(&tl.d[col][16 * h + 4 * q]);
+            const float4 B = *reinterpret_cast<const float4 *>(&tl.h[col][16 * h + 4 * q]);
+            gb2 += (A.x + A.y) + (A.z + A.w);
+            gw2 = __builtin_amdgcn_mfma_f32_32x32x2f32(A.x, B.x, gw2, 0, 0, 0);
+            gw2 = __builtin_amdgcn_mfma_f32_32x32x2f32(A.y, B.y, gw2, 0, 0, 0);
+            gw2 = __builtin_amdgcn_mfma_f32_32x32x2f32(A.z, B.z, gw2, 0, 0, 0);
+            gw2 = __builtin_amdgcn_mfma_f32_32x32x2f32(A.w, B.w, gw2, 0, 0, 0);
+        }
+        f32x16_t e1 = {};
+#pragma unroll
+        for (int r = 0; r < 16; ++r) e1 = __builtin_amdgcn_mfma_f32_32x32x2f32(at[r], d2[r], e1, 0, 0, 0);
+        wave_lds_sync();   // D2 and H1 read by every lane before others take their place
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            tl.d[mfma_row(h, r)][col] = e1[r] * dsilu(z1[r], s1[r]);
+            tl.h[mfma_row(h, r)][col] = dz3 * (z2[r] * s2[r]);
+        }
+        wave_lds_sync();
+        const int xr = col < kMlpF ? col : 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 A = *reinterpret_cast<const float4 *>(&tl.d[col][16 * h + 4 * q]);
+            const float4 H = *reinterpret_cast<const float4 *>(&tl.h[col][16 * h + 4 * q]);
+            const float4 V = *reinterpret_cast<const float4 *>(&tl.x[xr][16 * h + 4 * q]);
+            const float o = col == kMlpF ? 1.f : 0.f;   // column 9: the bias; columns 10..31: zero
+            const bool in = col < kMlpF;
+            gw3 += (H.x + H.y) + (H.z + H.w);
+            gw1 = __builtin_amdgcn_mfma_f32_32x32x2f32(A.x, in ? V.x : o, gw1, 0, 0, 0);
+            gw1 = __builtin_amdgcn_mfma_f32_32x32x2f32(A.y, in ? V.y : o, gw1, 0, 0, 0);
+            gw1 = __builtin_amdgcn_mfma_f32_32x32x2f32(A.z, in ? V.z : o, gw1, 0, 0, 0);
+            gw1 = __builtin_amdgcn_mfma_f32_32x32x2f32(A.w, in ? V.w : o, gw1, 0, 0, 0);
+        }
+        wave_lds_sync();   // tiles read before the next samples overwrite them
     }
-    for (int j = 0; j < kMlpH; ++j)
-        for (int i = 0; i < kMlpH; ++i) {
-            g = wave_sum_f(dz2[j] * h1[i]);
-            if (lane == 0) atomicAdd(&gW2[j * kMlpH + i], g);
-        }
-    for (int i = 0; i < kMlpH; ++i) {
-        float dh = 0.f;
-        for (int j = 0; j < kMlpH; ++j) dh += dz2[j] * W2[j * kMlpH + i];
-        const float sg = sigmoidf_(z1[i]);
-        const float dz1 = dh * sg * (1.f + z1[i] * (1.f - sg));
-        g = wave_sum_f(dz1);
-        if (lane == 0) atomicAdd(&gb1[i], g);
-        for (int f = 0; f < kMlpF; ++f) {
-            g = wave_sum_f(dz1 * x[f]);
-            if (lane == 0) atomicAdd(&gW1[i * kMlpF + f], g);
-        }
+    __syncthreads();   // every wavefront is done with its tile
+    float *S = sh.sums[wave];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int row = mfma_row(h, r);
+        S[kMlpH * kMlpF + kMlpH + row * kMlpH + col] = gw2[r];
+        if (col <= kMlpF) S[col < kMlpF ? row * kMlpF + col : kMlpH * kMlpF + row] = gw1[r];
+    }
+    gb2 += swap_halves(gb2);
+    gw3 += swap_halves(gw3);
+    gb3 = wave_sum_f(gb3);
+    lsum = wave_sum_f(lsum);
+    constexpr int kB2 = kMlpH * kMlpF + kMlpH + kMlpH * kMlpH;
+    if (h == 0) {
+        S[kB2 + col] = gb2;
+        S[kB2 + kMlpH + col] = gw3;
+    }
+    if (lane == 0) {
+        S[kMlpParams - 1] = gb3;
+        S[kMlpParams] = lsum;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i <= kMlpParams; i += blockDim.x)
+        part[(int64_t)blockIdx.x * kGradRow + i] = (sh.sums[0][i] + sh.sums[1][i]) + (sh.sums[2][i] + sh.sums[3][i]);
+}
+
+// Sum over the `rows` rows of part: gradient to grad and loss to loss (either may be null), and
+// with ADAM the update of the parameters.  A workgroup takes 32 parameters, 8 groups of threads a
+// share of the rows each.
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_grad_reduce(const float *__restrict__ part, int rows, float *__restrict__ grad,
+                                                     float *__restrict__ loss, float *params, float *m, float *v,
+                                                     float lr, float b1, float b2, float eps, int t) {
+    __shared__ float sh[8][32];
+    const int c = threadIdx.x & 31, grp = threadIdx.x >> 5;
+    const int i = blockIdx.x * 32 + c;
+    float acc = 0.f;
+    if (i <= kMlpParams) {
+#pragma unroll 4
+        for (int b = grp; b < rows; b += 8) acc += part[(int64_t)b * kGradRow + i];
+    }
+    sh[grp][c] = acc;
+    __syncthreads();
+    if (grp != 0 || i > kMlpParams) return;
+    const float g = ((sh[0][c] + sh[1][c]) + (sh[2][c] + sh[3][c])) + ((sh[4][c] + sh[5][c]) + (sh[6][c] + sh[7][c]));
+    if (i == kMlpParams) {
+        if (loss) *loss = g;
+        return;
+    }
+    if (grad) grad[i] = g;
+    if constexpr (ADAM) {
+        const float mi = b1 * m[i] + (1.f - b1) * g;
+        const float vi = b2 * v[i] + (1.f - b2) * g * g;
+        m[i] = mi;
+        v[i] = vi;
+        const float mh = mi / (1.f - powf(b1, (float)t));
+        const float vh = vi / (1.f - powf(b2, (float)t));
+        params[i] -= lr * mh / (sqrtf(vh) + eps);
     }
 }
 
@@ -495,10 +642,9 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ para
 // Rounded to BF16: X, W1, b1, W2, b2, H1, D2 (as operand of both products) and D1.  db2, dw3,
 // db3 and the loss accumulate per lane in FP32 from unrounded values.  A wavefront keeps its
 // sums over all the batches it takes in its accumulators; the workgroup adds its four
-// wavefronts' sums in LDS and then into grad, one atomic per parameter.
+// wavefronts' sums in LDS and writes them as its row of part.
 // ---------------------------------------------------------------------------------------------
 constexpr int kGradTileStride = 72;   // LDS row stride of the transposed tiles, BF16 elements (144 B)
-constexpr int kGradMaxBlocks = 256;
 
 struct alignas(16) GradTiles {
     __bf16 d[kMlpH][kGradTileStride];   // layer delta [hidden][sample]: D2, then D1
@@ -506,12 +652,9 @@ struct alignas(16) GradTiles {
     __bf16 x[16][kGradTileStride];      // inputs [feature][sample]; row 9 = 1, rows 10..15 = 0
 };
 
-__device__ __forceinline__ float dsilu(float z, float sg) { return sg * (1.f + z * (1.f - sg)); }
-
 __global__ __launch_bounds__(256) void k_mlp_grad_mfma(const float *__restrict__ params, const float *__restrict__ X,
                                                        const float *__restrict__ T, int64_t n, int batch,
-                                                       uint32_t seed, int random, float *__restrict__ grad,
-                                                       float *__restrict__ loss) {
+                                                       uint32_t seed, int random, float *__restrict__ part) {
     __shared__ float sp[kMlpParams];
     __shared__ float acc[kMlpParams + 1];   // workgroup sums: gradient, then the loss
     __shared__ GradTiles tiles[4];
@@ -553,8 +696,7 @@ __global__ __launch_bounds__(256) void k_mlp_grad_mfma(const float *__restrict__
     for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < batch; base += (int64_t)gridDim.x * blockDim.x) {
         const int64_t k = base + threadIdx.x;
         const bool active = k < batch;
-        int64_t s = 0;
-        if (active) s = random ? (int64_t)(hash32(seed * 2654435761u + (uint32_t)k) % (uint64_t)n) : k;
+        const int64_t s = active ? batch_sample((int)k, seed, random, n) : 0;
         float xn[kMlpF], px[kMlpF];
 #pragma unroll
         for (int i = 0; i < kMlpF; ++i) xn[i] = active ? X[s * kMlpF + i] : 0.f;
@@ -662,22 +804,7 @@ __global__ __launch_bounds__(256) void k_mlp_grad_mfma(const float *__restrict__
         atomicAdd(&acc[kMlpParams], lsum);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < kMlpParams; i += blockDim.x) atomicAdd(&grad[i], acc[i]);
-    if (threadIdx.x == 0) atomicAdd(loss, acc[kMlpParams]);
-}
-
-__global__ void k_adam(float *params, const float *grad, float *m, float *v, int n, float lr, float b1, float b2,
-                       float eps, int t) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float g = grad[i];
-    const float mi = b1 * m[i] + (1.f - b1) * g;
-    const float vi = b2 * v[i] + (1.f - b2) * g * g;
-    m[i] = mi;
-    v[i] = vi;
-    const float mh = mi / (1.f - powf(b1, (float)t));
-    const float vh = vi / (1.f - powf(b2, (float)t));
-    params[i] -= lr * mh / (sqrtf(vh) + eps);
+    for (int i = threadIdx.x; i <= kMlpParams; i += blockDim.x) part[(int64_t)blockIdx.x * kGradRow + i] = acc[i];
 }
 
 // batch inference (normalised inputs) for tests and evaluation

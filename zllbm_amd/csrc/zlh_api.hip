@@ -415,8 +415,8 @@ __global__ void k_closure_features(const double *fq, int64_t n, double tau0, dou
 }  // namespace zlh
 
 // ==============================================================================================
-// static device array of zlh_mlp_gradient_noalloc: the parameters, the samples and targets,
-// and the gradient and loss accumulators, at fixed float offsets (each a multiple of 64 floats,
+// static device array of zlh_mlp_gradient_noalloc: the parameters, the samples and targets, the
+// workgroups' partial sums, and the gradient and loss, at fixed float offsets (each a multiple of 64 floats,
 // so every region starts 256-byte aligned).  One copy per GPU, at its own address, for the life
 // of the process.  Host code never uses the array's name as an address: the per-device address
 // comes from hipGetSymbolAddress (scratch_setup).
@@ -426,7 +426,8 @@ constexpr int64_t kNoAllocMaxSamples = ZLH_MLP_NOALLOC_MAX_SAMPLES;
 constexpr int64_t kScratchParams = 0;                                     // [kMlpParams]
 constexpr int64_t kScratchGrad = 1536;                                    // [kMlpParams]
 constexpr int64_t kScratchLoss = 3072;                                    // [1]
-constexpr int64_t kScratchT = 3136;                                       // [max samples]
+constexpr int64_t kScratchPart = 3136;                                    // [kGradMaxBlocks][kGradRow]
+constexpr int64_t kScratchT = kScratchPart + (int64_t)zlh::kGradMaxBlocks * zlh::kGradRow;   // [max samples]
 constexpr int64_t kScratchX = kScratchT + kNoAllocMaxSamples;             // [max samples][kMlpF]
 constexpr int64_t kScratchFloats = kScratchX + kNoAllocMaxSamples * zlh::kMlpF;
 static_assert(zlh::kMlpParams <= kScratchGrad - kScratchParams && zlh::kMlpParams <= kScratchLoss - kScratchGrad,
@@ -435,12 +436,6 @@ static_assert(kScratchT % 64 == 0 && kScratchX % 64 == 0, "regions are 256-byte 
 }  // namespace
 
 static __device__ __align__(256) float scratch[kScratchFloats];
-
-// clears the accumulator regions (a kernel, not a memset, so that the call stays capturable)
-__global__ void k_scratch_clear(float *p, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.f;
-}
 
 // ==============================================================================================
 // host context
@@ -1899,17 +1894,26 @@ zlh_status zlh_mlp_set(zlh_ctx *ctx, const float *params, const float *mean, con
     return ZLH_OK;
 }
 
-// gradient kernel of the selected training form: one thread per sample on the vector units, or
-// 64 samples per wavefront on the matrix cores (a grid of at most kGradMaxBlocks workgroups that
-// loop over the batch)
-static void launch_mlp_grad(zlh_ctx *ctx, const float *p, const float *x, const float *t, int64_t n, int nb,
-                            uint32_t seed, int random, float *grad, float *loss) {
-    if (ctx->mlp_train_form == ZLH_MLP_BF16_MFMA)
-        hipLaunchKernelGGL(k_mlp_grad_mfma, dim3(std::min<unsigned>(blocks(nb), kGradMaxBlocks)), dim3(256), 0,
-                           ctx->stream, p, x, t, n, nb, seed, random, grad, loss);
+// gradient kernel of the selected training form (128 samples per workgroup trip in FP32, 256 with
+// BF16 operands; a grid of at most kGradMaxBlocks workgroups that loop over the batch): returns
+// the rows of part it writes
+static int launch_mlp_grad(zlh_ctx *ctx, const float *p, const float *x, const float *t, int64_t n, int nb,
+                           uint32_t seed, int random, float *part) {
+    const bool mfma = ctx->mlp_train_form == ZLH_MLP_BF16_MFMA;
+    const unsigned rows = std::min<unsigned>(blocks(nb, mfma ? 256 : 128), kGradMaxBlocks);
+    if (mfma)
+        hipLaunchKernelGGL(k_mlp_grad_mfma, dim3(rows), dim3(256), 0, ctx->stream, p, x, t, n, nb, seed, random, part);
     else
-        hipLaunchKernelGGL(k_mlp_grad, dim3(blocks(nb)), dim3(256), 0, ctx->stream, p, x, t, n, nb, seed, random, grad,
-                           loss);
+        hipLaunchKernelGGL(k_mlp_grad, dim3(rows), dim3(256), 0, ctx->stream, p, x, t, n, nb, seed, random, part);
+    return (int)rows;
+}
+
+// gradient and loss of all n samples, reduced
+static void launch_full_gradient(zlh_ctx *ctx, const float *p, const float *x, const float *t, int64_t n, float *part,
+                                 float *grad, float *loss) {
+    const int rows = launch_mlp_grad(ctx, p, x, t, n, (int)n, 0u, 0, part);
+    hipLaunchKernelGGL(k_grad_reduce<false>, dim3(blocks(kMlpParams + 1, 32)), dim3(256), 0, ctx->stream, part, rows,
+                       grad, loss, nullptr, nullptr, nullptr, 0.f, 0.f, 0.f, 0.f, 0);
 }
 
 zlh_status zlh_mlp_training_form(zlh_ctx *ctx, int form) {
@@ -1924,21 +1928,22 @@ zlh_status zlh_mlp_gradient(zlh_ctx *ctx, const float *params, const float *x, c
                             float *loss) {
     if (!ctx) return ZLH_EINVAL;
     if (!params || !x || !t || !grad || n < 1 || n > (1 << 26)) return ctx->fail(ZLH_EINVAL, "bad gradient arguments");
-    DevBuf dp, dx, dt, dg, dl;
+    DevBuf dp, dx, dt, dg, dr;
     zlh_status s;
     if ((s = dalloc(ctx, dp, sizeof(float) * kMlpParams, false))) return s;
     if ((s = dalloc(ctx, dx, sizeof(float) * kMlpF * n, false))) return s;
     if ((s = dalloc(ctx, dt, sizeof(float) * n, false))) return s;
-    if ((s = dalloc(ctx, dg, sizeof(float) * kMlpParams))) return s;
-    if ((s = dalloc(ctx, dl, sizeof(float)))) return s;
+    if ((s = dalloc(ctx, dg, sizeof(float) * (kMlpParams + 1), false))) return s;
+    if ((s = dalloc(ctx, dr, sizeof(float) * kGradMaxBlocks * kGradRow, false))) return s;
     ZLH_TRY(hipMemcpyAsync(dp.p, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice, ctx->stream));
     ZLH_TRY(hipMemcpyAsync(dx.p, x, sizeof(float) * kMlpF * n, hipMemcpyHostToDevice, ctx->stream));
     ZLH_TRY(hipMemcpyAsync(dt.p, t, sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
-    launch_mlp_grad(ctx, dp.as<float>(), dx.as<float>(), dt.as<float>(), n, (int)n, 0u, 0, dg.as<float>(),
-                    dl.as<float>());
+    launch_full_gradient(ctx, dp.as<float>(), dx.as<float>(), dt.as<float>(), n, dr.as<float>(), dg.as<float>(),
+                         dg.as<float>() + kMlpParams);
     ZLH_TRY(hipGetLastError());
     ZLH_TRY(hipMemcpyAsync(grad, dg.p, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, ctx->stream));
-    if (loss) ZLH_TRY(hipMemcpyAsync(loss, dl.p, sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
+    if (loss)
+        ZLH_TRY(hipMemcpyAsync(loss, dg.as<float>() + kMlpParams, sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
     ZLH_TRY(hipStreamSynchronize(ctx->stream));
     return ZLH_OK;
 }
@@ -1953,14 +1958,10 @@ zlh_status zlh_mlp_gradient_noalloc(zlh_ctx *ctx, const float *params, const flo
     if (!ctx->scratch_addr) return ctx->fail(ZLH_ESTATE, "no-allocation array not set up");
     float *dp = ctx->scratch_addr + kScratchParams, *dg = ctx->scratch_addr + kScratchGrad;
     float *dl = ctx->scratch_addr + kScratchLoss, *dt = ctx->scratch_addr + kScratchT, *dx = ctx->scratch_addr + kScratchX;
-    // gradient and loss regions (and the gap between them) start at zero
-    const int64_t nclear = kScratchT - kScratchGrad;
-    hipLaunchKernelGGL(k_scratch_clear, dim3(blocks(nclear)), dim3(256), 0, ctx->stream, dg, nclear);
-    ZLH_TRY(hipGetLastError());
     ZLH_TRY(hipMemcpyAsync(dp, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice, ctx->stream));
     ZLH_TRY(hipMemcpyAsync(dx, x, sizeof(float) * kMlpF * n, hipMemcpyHostToDevice, ctx->stream));
     ZLH_TRY(hipMemcpyAsync(dt, t, sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
-    launch_mlp_grad(ctx, dp, dx, dt, n, (int)n, 0u, 0, dg, dl);
+    launch_full_gradient(ctx, dp, dx, dt, n, ctx->scratch_addr + kScratchPart, dg, dl);
     ZLH_TRY(hipGetLastError());
     ZLH_TRY(hipMemcpyAsync(grad, dg, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, ctx->stream));
     if (loss) ZLH_TRY(hipMemcpyAsync(loss, dl, sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
@@ -1973,15 +1974,15 @@ zlh_status zlh_mlp_train(zlh_ctx *ctx, const float *x, const float *t, int64_t n
     if (!ctx) return ZLH_EINVAL;
     if (!params || !x || !t || n < 1 || n > (1 << 26) || steps < 1 || batch < 1 || batch > (1 << 20) || !(lr > 0.))
         return ctx->fail(ZLH_EINVAL, "bad training arguments");
-    DevBuf dp, dx, dt, dg, dm, dv, dl;
+    DevBuf dp, dx, dt, dr, dm, dv, dl;
     zlh_status s;
     if ((s = dalloc(ctx, dp, sizeof(float) * kMlpParams, false))) return s;
     if ((s = dalloc(ctx, dx, sizeof(float) * kMlpF * n, false))) return s;
     if ((s = dalloc(ctx, dt, sizeof(float) * n, false))) return s;
-    if ((s = dalloc(ctx, dg, sizeof(float) * kMlpParams))) return s;
+    if ((s = dalloc(ctx, dr, sizeof(float) * kGradMaxBlocks * kGradRow, false))) return s;
     if ((s = dalloc(ctx, dm, sizeof(float) * kMlpParams))) return s;
     if ((s = dalloc(ctx, dv, sizeof(float) * kMlpParams))) return s;
-    if ((s = dalloc(ctx, dl, sizeof(float) * steps))) return s;
+    if ((s = dalloc(ctx, dl, sizeof(float) * steps, false))) return s;
     ZLH_TRY(hipMemcpyAsync(dp.p, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice, ctx->stream));
     ZLH_TRY(hipMemcpyAsync(dx.p, x, sizeof(float) * kMlpF * n, hipMemcpyHostToDevice, ctx->stream));
     ZLH_TRY(hipMemcpyAsync(dt.p, t, sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
@@ -1990,12 +1991,11 @@ zlh_status zlh_mlp_train(zlh_ctx *ctx, const float *x, const float *t, int64_t n
     const int full = (int64_t)batch >= n;
     const int nb = full ? (int)n : batch;
     for (int it = 1; it <= steps; ++it) {
-        ZLH_TRY(hipMemsetAsync(dg.p, 0, sizeof(float) * kMlpParams, ctx->stream));
-        launch_mlp_grad(ctx, dp.as<float>(), dx.as<float>(), dt.as<float>(), n, nb,
-                        (uint32_t)(seed * 1000003ull + (uint64_t)it), full ? 0 : 1, dg.as<float>(),
-                        dl.as<float>() + (it - 1));
-        hipLaunchKernelGGL(k_adam, dim3(blocks(kMlpParams)), dim3(256), 0, ctx->stream, dp.as<float>(), dg.as<float>(),
-                           dm.as<float>(), dv.as<float>(), kMlpParams, (float)lr, 0.9f, 0.999f, 1e-8f, it);
+        const int rows = launch_mlp_grad(ctx, dp.as<float>(), dx.as<float>(), dt.as<float>(), n, nb,
+                                         (uint32_t)(seed * 1000003ull + (uint64_t)it), full ? 0 : 1, dr.as<float>());
+        hipLaunchKernelGGL(k_grad_reduce<true>, dim3(blocks(kMlpParams + 1, 32)), dim3(256), 0, ctx->stream,
+                           dr.as<float>(), rows, nullptr, dl.as<float>() + (it - 1), dp.as<float>(), dm.as<float>(),
+                           dv.as<float>(), (float)lr, 0.9f, 0.999f, 1e-8f, it);
     }
     ZLH_TRY(hipGetLastError());
     ZLH_TRY(hipMemcpyAsync(params, dp.p, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, ctx->stream));
