@@ -240,7 +240,7 @@ zlh_status zlh_mlp_train(zlh_ctx *ctx, const float *x, const float *t, int64_t n
 enum { ZLH_MLP_FP32 = 0, ZLH_MLP_BF16_MFMA = 1, ZLH_MLP_FP16_MFMA = 2 };
 /* kernel of zlh_mlp_gradient and zlh_mlp_train: ZLH_MLP_FP32 (default; FP32 operands, products
  * and sums) or ZLH_MLP_BF16_MFMA (BF16 operands and FP32 accumulation); ZLH_EINVAL for any other
- * form.  Without BF16 a gradient depends on its inputs alone, bit for bit. */
+ * form.  A gradient depends on its inputs alone, bit for bit. */
 zlh_status zlh_mlp_training_form(zlh_ctx *ctx, int form);
 /* network output (nu_t / nu_scale) of normalised inputs [n][9] with the parameters set by
  * zlh_mlp_set, in the given form */

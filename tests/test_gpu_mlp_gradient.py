@@ -48,3 +48,18 @@ def test_minibatch_loss(n, batch):
     at = np.arange(n) if batch >= n else (x % u(n)).astype(np.int64)
     lref, _ = mo.loss_and_grad(p.astype(np.float64), X[at].astype(np.float64), T[at].astype(np.float64))
     assert abs(hist[0] - lref) <= 1e-5 * lref
+
+
+# BF16 operands: 64 samples a wavefront, 256 a workgroup, at most 256 workgroups.  A difference in
+# the order of an FP32 sum moves an operand to the next BF16 value in about one case of 2^16 per
+# last bit: the bound of the emulation test, 5e-4 of the largest gradient component, for sets large
+# enough that single roundings average out, ten times that below.
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 257, 65536, 65537])
+def test_gradient_bf16_at_tile_edges(n):
+    s = _ctx()
+    X, T = _data(n, seed=n + 7)
+    p = closure.init_params(3)
+    loss, gd = s.mlp_gradient(p, X, T, form=hip.MLP_BF16_MFMA)
+    lemu, gemu = mo.loss_and_grad_lowp(p.astype(np.float64), X.astype(np.float64), T.astype(np.float64), mo.bf16_round)
+    assert abs(loss - lemu) <= 1e-3 * lemu + 1e-6
+    assert np.max(np.abs(gd - gemu)) <= (5e-4 if n > 1000 else 5e-3) * np.max(np.abs(gemu))
