@@ -14,10 +14,16 @@
 //     immersed boundary: the fused kernel pulls their post-collision neighbours (stream) and
 //     immediately applies the next collision, writing post-collision values: 2Q accesses per
 //     node, no per-node tables.
-//   * "aux" nodes (domain boundary nodes and their partners, refinement-interface layers and
-//     interpolation stencils, immersed-boundary supports, nodes with an absent pull source) keep
-//     their post-stream populations in a compact side array, are modified there by the boundary,
-//     transfer and forcing kernels, and are collided at the start of their level's next substep.
+//   * "aux" nodes (refinement-interface layers and interpolation stencils, immersed-boundary
+//     supports, nodes with an absent pull source, and the boundary nodes of a level with
+//     non-equilibrium-extrapolation faces) keep their post-stream populations in a compact side
+//     array, are modified there by the boundary, transfer and forcing kernels, and are collided at
+//     the start of their level's next substep.
+//   * bounce-back and periodic conditions only move post-collision populations: what a boundary
+//     node gets is the population its twin (or the twin's twin, at an edge) pulls, or its own in
+//     the opposite direction.  Where a level has no other conditions the pull of the bricks with
+//     boundary nodes takes its sources from a table ("resolved" boundaries, BoundaryPull): no
+//     boundary launches, and boundary nodes are bulk nodes.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
@@ -59,6 +65,35 @@ __device__ __forceinline__ void store_nt(T v, T *dst) {
     else __builtin_nontemporal_store(v, dst);
 }
 
+// Pull sources of the bricks that hold resolved boundary nodes.  brick[b]: {first row, directions
+// that have a row} (0 directions: no boundary node); src [row][64]: element of the population buffer
+// that the lane pulls for the row's direction (its regular source, or what the boundary conditions
+// resolve to); face (levels with a moving wall only, else null) [row][64]: the wall's face, 0 where
+// none; wall [7][Q]: {6 rho0 w, c . u_w} of a face and direction (BoundaryBounceBack{2D,3D},
+// lbm_bounce_back.cpp:29-91).
+// Rows of 64 lanes for the directions that some lane's conditions set: one coalesced load per such
+// direction and no selection per lane, 5 of 19 directions (1.3 KB beside 4.9 KB of FP32
+// populations) in a brick on one face.  It replaces a launch per face (4.2-4.6 us each) and the
+// deferred collision of the boundary nodes (4-9 us): see k_stream_collide.
+struct BoundaryPull {
+    const int2 *brick;
+    const int32_t *src;
+    const uint8_t *face;
+    const double2 *wall;
+};
+
+// row of direction q in a brick's table
+__host__ __device__ __forceinline__ int32_t bnd_row(int2 brick, int q) {
+    return brick.x + __builtin_popcount((unsigned)brick.y & ((1u << q) - 1u));
+}
+
+// a pulled value behind a moving wall (face > 0)
+template <int Q, typename T>
+__device__ __forceinline__ T wall_value(const double2 *wall, int face, int q, T v) {
+    const double2 k = wall[face * Q + q];
+    return T(__builtin_fma(-k.x, k.y, double(v)));
+}
+
 template <typename T>
 struct BrickLevel {
     int64_t nbrick;
@@ -71,6 +106,7 @@ struct BrickLevel {
     const int32_t *auxbase;   // [nbrick]
     const uint32_t *aux_missing;  // [naux]
     const int32_t *aux_slot;  // [naux]
+    BoundaryPull bnd;         // brick null: no resolved boundary nodes
 };
 
 // shift applied to stored populations: FP32 stores f - w_i
@@ -428,68 +464,154 @@ __device__ __forceinline__ int64_t xcd_group(int64_t ngroups) {
     return g < ngroups ? g : -1;
 }
 
+// Per-lane constants of the pull, fixed by the brick layout and computed once per pull: the
+// offset UNIT lane_of() of the source coordinate along each axis for c = +1, 0, -1, and
+// whether the lane sits on the low / high face of each axis.  lane_of is a sum of one term per
+// axis, so a source slot is the OR of three of these.
+template <int D>
+struct PullLane {
+    uint32_t s[3][3];   // [axis][1 - c]
+    bool lo[3], hi[3];
+};
+
+// UNIT 4: byte offsets of 4-byte populations; 1: elements
+template <int D, int UNIT>
+__device__ __forceinline__ PullLane<D> pull_lane(int lane) {
+    static_assert(UNIT == 4 || UNIT == 1, "bytes of 4-byte populations, or elements");
+    PullLane<D> P;
+    const uint32_t l4 = 4u * (uint32_t)lane;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        constexpr uint32_t kNone = 0u;
+        const uint32_t m4 = a < D ? lane_axis_mask4<D>(a) : kNone;
+        const uint32_t own4 = l4 & m4;
+        // k = 1 - c: the source coordinate along a is l - 1 (k = 0), l (1) or l + 1 (2)
+        P.s[a][0] = a < D ? lane_axis_step4(own4, m4, -1) / (4 / UNIT) : 0u;
+        P.s[a][1] = own4 / (4 / UNIT);
+        P.s[a][2] = a < D ? lane_axis_step4(own4, m4, 1) / (4 / UNIT) : 0u;
+        P.lo[a] = a < D && own4 == 0u;
+        P.hi[a] = a < D && own4 == m4;
+    }
+    return P;
+}
+
+// Calls emit(q, offset) for every direction with the lane's source: nbo holds the offsets of the
+// neighbour bricks (uniform), self the own brick's in a vector register, so that each selection
+// takes one uniform operand and it.  Addresses by selection, no branches: a branch between two of
+// the loads makes the compiler wait on the vector memory counter there.  D2Q9 / D3Q19 directions
+// cross at most two axes: the brick is chosen along the first axis, then the second.  A lane
+// without a node stays inside its own brick.
+template <int D, typename F>
+__device__ __forceinline__ void for_each_source(const PullLane<D> &P, bool has_node,
+                                                const uint32_t (&nbo)[Brick<D>::nnbr], uint32_t self, F emit) {
+    using L = Lattice<D>;
+    constexpr int base = D == 3 ? 13 : 4;
+    bool clo[3], chi[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        clo[a] = P.lo[a] && has_node;
+        chi[a] = P.hi[a] && has_node;
+    }
+#pragma unroll
+    for (int q = 0; q < L::Q; ++q) {
+        const int cx = L::cx[q], cy = L::cy[q], cz = D == 3 ? L::cz[q] : 0;
+        const bool ex = cx == 1 ? clo[0] : (cx == -1 ? chi[0] : false);
+        const bool ey = cy == 1 ? clo[1] : (cy == -1 ? chi[1] : false);
+        const bool ez = cz == 1 ? clo[2] : (cz == -1 ? chi[2] : false);
+        const int dx = -cx, dy = -3 * cy, dz = -9 * cz;
+        uint32_t sel;
+        if (cx != 0 && cy != 0)
+            sel = ey ? (ex ? nbo[base + dx + dy] : nbo[base + dy]) : (ex ? nbo[base + dx] : self);
+        else if (cx != 0 && cz != 0)
+            sel = ez ? (ex ? nbo[base + dx + dz] : nbo[base + dz]) : (ex ? nbo[base + dx] : self);
+        else if (cy != 0 && cz != 0)
+            sel = ez ? (ey ? nbo[base + dy + dz] : nbo[base + dz]) : (ey ? nbo[base + dy] : self);
+        else if (cx != 0)
+            sel = ex ? nbo[base + dx] : self;
+        else if (cy != 0)
+            sel = ey ? nbo[base + dy] : self;
+        else if (cz != 0)
+            sel = ez ? nbo[base + dz] : self;
+        else
+            sel = self;
+        emit(q, sel + (P.s[0][1 - cx] | P.s[1][1 - cy] | P.s[2][1 - cz]));
+    }
+}
+
 // Fused pull-stream + collide of one brick by one wavefront.
 template <int D, typename T, typename C, bool SHIFT, int COLL, int VAR>
 __device__ __forceinline__ void stream_collide_brick(const BrickLevel<T> &lv, const T *__restrict__ fin,
                                                      T *__restrict__ fout, T *__restrict__ aux_f, const StepParams &p,
                                                      int64_t b, const MlpOps *ops) {
     using L = Lattice<D>;
-    using B = Brick<D>;
     constexpr int Q = L::Q;
-    constexpr int E = B::edge;
-    constexpr int NN = B::nnbr;
+    constexpr int NN = Brick<D>::nnbr;
     static_assert(!mlp_on_mfma<C, VAR>(), "the FP32 learned closure runs in k_stream_collide_mlp");
-    constexpr bool kWave = false;
     const int lane = threadIdx.x & 63;
-    const uint64_t occ = lv.occ[b];
-    const bool has_node = (occ >> lane) & 1ull;
-    if (!kWave && !has_node) return;
-    const uint64_t am = lv.auxmask[b];
-    const bool is_aux = (am >> lane) & 1ull;
-    const bool deferred = (lv.defmask[b] >> lane) & 1ull;
-    int64_t ai = 0;
-    uint32_t missing = 0;
-    if (is_aux) {
-        ai = lv.auxbase[b] + __popcll(am & ((1ull << lane) - 1ull));
-        missing = lv.aux_missing[ai];
-    }
+    // the brick's scalars in one batch (the asm makes them all live here): loaded where they are
+    // used, each would wait for the one before it
+    uint64_t occ = lv.occ[b], am = lv.auxmask[b], dm = lv.defmask[b];
+    int32_t base = lv.auxbase[b];
+    int2 bnd = make_int2(0, 0);
+    if (lv.bnd.brick) bnd = lv.bnd.brick[b];
     int32_t nb[NN];
 #pragma unroll
     for (int k = 0; k < NN; ++k) nb[k] = lv.nbr[b * NN + k];
-    const int lx = B::lane_coord(lane, 0), ly = B::lane_coord(lane, 1);
-    const int lz = D == 3 ? B::lane_coord(lane, 2) : 0;
-    C f[Q];
-    const T *__restrict__ own = fin + b * Q * 64 + lane;
-    f[0] = kWave && !has_node ? C(0) : C(own[0]);
+    asm volatile("" : "+s"(occ), "+s"(am), "+s"(dm), "+s"(base), "+s"(bnd.x), "+s"(bnd.y));
 #pragma unroll
-    for (int q = 1; q < Q; ++q) {
-        const int sx = lx - L::cx[q], sy = ly - L::cy[q], sz = lz - L::cz[q];
-        // the source lies in this brick or in the neighbour brick across the faces that c_q
-        // crosses; select among those wave-uniform brick indices (indices fold after unrolling)
-        const bool ex = L::cx[q] != 0 && (sx < 0 || sx >= E);
-        const bool ey = L::cy[q] != 0 && (sy < 0 || sy >= E);
-        const bool ez = D == 3 && L::cz[q] != 0 && (sz < 0 || sz >= E);
-        constexpr int base = D == 3 ? 13 : 4;
-        const int dx = -L::cx[q], dy = -3 * L::cy[q], dz = D == 3 ? -9 * L::cz[q] : 0;
-        const int sb = ez ? (ey ? (ex ? nb[base + dx + dy + dz] : nb[base + dy + dz])
-                                : (ex ? nb[base + dx + dz] : nb[base + dz]))
-                          : (ey ? (ex ? nb[base + dx + dy] : nb[base + dy])
-                                : (ex ? nb[base + dx] : nb[base]));
-        const int sl = B::lane_of(sx & (E - 1), sy & (E - 1), sz & (E - 1));
-        if (kWave && !has_node) f[q] = C(0);
-        else if (missing & (1u << q)) f[q] = aux_f[q * lv.naux + ai];
-        else f[q] = C(fin[((int64_t)sb * Q + q) * 64 + sl]);
+    for (int k = 0; k < NN; ++k) asm volatile("" : "+s"(nb[k]));
+    const bool has_node = (occ >> lane) & 1ull;
+    if (!has_node) return;
+    const bool is_aux = (am >> lane) & 1ull;
+    const bool deferred = (dm >> lane) & 1ull;
+    int64_t ai = 0;
+    uint32_t missing = 0;
+    if (is_aux) {
+        ai = base + __popcll(am & ((1ull << lane) - 1ull));
+        missing = lv.aux_missing[ai];
+    }
+    C f[Q];
+    // elements of fin to pull, then every load, then what no load gives: a branch or a use
+    // between the loads would wait for those before it
+    uint32_t e[Q];
+    {
+        uint32_t nbo[NN];
+#pragma unroll
+        for (int k = 0; k < NN; ++k) nbo[k] = (uint32_t)(nb[k] < 0 ? (int32_t)b : nb[k]) * (uint32_t)(Q * 64);
+        uint32_t self = nbo[D == 3 ? 13 : 4];
+        asm volatile("" : "+v"(self));
+        for_each_source<D>(pull_lane<D, 1>(lane), true, nbo, self, [&](int q, uint32_t o) { e[q] = o + 64u * q; });
+    }
+    if (bnd.y) {   // uniform: a brick with resolved boundary nodes
+#pragma unroll
+        for (int q = 1; q < Q; ++q)
+            if (bnd.y >> q & 1) e[q] = (uint32_t)lv.bnd.src[(int64_t)bnd_row(bnd, q) * 64 + lane];
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) f[q] = C(fin[e[q]]);
+    if (bnd.y && lv.bnd.face) {
+#pragma unroll
+        for (int q = 1; q < Q; ++q) {
+            if (!(bnd.y >> q & 1)) continue;
+            const int w = lv.bnd.face[(int64_t)bnd_row(bnd, q) * 64 + lane];
+            if (w) f[q] = C(wall_value<Q, T>(lv.bnd.wall, w, q, T(f[q])));
+        }
+    }
+    if (missing) {
+        // absent sources that no boundary condition sets keep the earlier values
+#pragma unroll
+        for (int q = 1; q < Q; ++q)
+            if (missing & (1u << q)) f[q] = C(aux_f[q * lv.naux + ai]);
     }
     if (is_aux) {
 #pragma unroll
         for (int q = 0; q < Q; ++q) aux_f[q * lv.naux + ai] = T(f[q]);
         // a recorded node that nothing changes before its next collision collides here
-        if (!kWave && deferred) return;
+        if (deferred) return;
     }
     C F[3] = {C(p.const_force[0]), C(p.const_force[1]), C(p.const_force[2])};
     C rho, u[3];
     collide<D, SHIFT, COLL, C, VAR>(f, F, p, rho, u, ops);
-    if (kWave && (!has_node || deferred)) return;
     // streaming stores: the next substep reads these values through other CUs' caches
     T *__restrict__ dst = fout + b * Q * 64 + lane;
 #pragma unroll
@@ -518,36 +640,9 @@ struct BrickTables {
     const int32_t *__restrict__ auxbase;
     const int32_t *__restrict__ nbr;
     const uint32_t *__restrict__ aux_missing;
+    const int2 *__restrict__ bnd_brick;   // BoundaryPull::brick and ::src (null: no resolved boundaries)
+    const int32_t *__restrict__ bnd_src;
 };
-
-// Per-lane constants of the pull, fixed by the brick layout and computed once per pull: the
-// byte offset 4 lane_of() of the source coordinate along each axis for c = +1, 0, -1, and
-// whether the lane sits on the low / high face of each axis.  lane_of is a sum of one term per
-// axis, so a source slot is the OR of three of these.
-template <int D>
-struct PullLane {
-    uint32_t s4[3][3];   // [axis][1 - c]
-    bool lo[3], hi[3];
-};
-
-template <int D>
-__device__ __forceinline__ PullLane<D> pull_lane(int lane) {
-    PullLane<D> P;
-    const uint32_t l4 = 4u * (uint32_t)lane;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        constexpr uint32_t kNone = 0u;
-        const uint32_t m4 = a < D ? lane_axis_mask4<D>(a) : kNone;
-        const uint32_t own4 = l4 & m4;
-        // k = 1 - c: the source coordinate along a is l - 1 (k = 0), l (1) or l + 1 (2)
-        P.s4[a][0] = a < D ? lane_axis_step4(own4, m4, -1) : 0u;
-        P.s4[a][1] = own4;
-        P.s4[a][2] = a < D ? lane_axis_step4(own4, m4, 1) : 0u;
-        P.lo[a] = a < D && own4 == 0u;
-        P.hi[a] = a < D && own4 == m4;
-    }
-    return P;
-}
 
 // Pull of brick b (every lane, every direction) into a per-wave LDS buffer [Q][64] with one
 // direct-to-LDS dword load per direction (gfx950 global_load_lds_dword: lane i lands at
@@ -556,7 +651,7 @@ __device__ __forceinline__ PullLane<D> pull_lane(int lane) {
 // lane without a node loads the slot its stencil names inside brick b; the consumer drops those values (a deferred node's
 // missing directions keep the boundary / transfer values already in the aux array).  Addresses are 32-bit byte offsets
 // from the direction's base fin + 64 q.  Returns the lane's missing-source mask (deferred nodes).
-template <int D, typename T>
+template <int D, typename T, bool BND>
 __device__ __forceinline__ uint32_t pull_to_lds(const BrickTables &t, const T *__restrict__ fin, int64_t b, int lane,
                                                 T *buf) {
     using L = Lattice<D>;
@@ -564,10 +659,12 @@ __device__ __forceinline__ uint32_t pull_to_lds(const BrickTables &t, const T *_
     constexpr int Q = L::Q;
     constexpr int NN = B::nnbr;
     static_assert(sizeof(T) == 4, "dword staging");
-    const PullLane<D> P = pull_lane<D>(lane);   // per pull: live only while the addresses form
+    const uint64_t am = t.auxmask[b];
+    uint32_t missing = 0;
     // opaque per pull: the direction's LDS destinations are formed here, not hoisted out of the
     // caller's loop into 19 long-lived scalars
     asm volatile("" : "+s"(buf));
+    const PullLane<D> P = pull_lane<D, 4>(lane);   // per pull: live only while the addresses form
     // byte offsets of the neighbour bricks (uniform: scalar multiplies)
     constexpr uint32_t kBrickBytes = (uint32_t)(Q * 64 * sizeof(T));
     uint32_t nbo[NN];
@@ -579,52 +676,33 @@ __device__ __forceinline__ uint32_t pull_to_lds(const BrickTables &t, const T *_
     // a lane crosses into a neighbour brick only if it holds a node: a lane without one loads
     // the slot its stencil names inside its own brick, a line the brick's own pull fetches anyway
     const bool has_node = (t.occ[b] >> lane) & 1ull;
-    bool clo[3], chi[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        clo[a] = P.lo[a] && has_node;
-        chi[a] = P.hi[a] && has_node;
-    }
     constexpr int base = D == 3 ? 13 : 4;
-    // the own brick's offset in a vector register, so that each selection below takes one
-    // uniform operand and this one
     uint32_t self = nbo[base];
     asm volatile("" : "+v"(self));
-    // addresses by selection, no branches: a branch between two of these loads makes the
-    // compiler wait on the vector memory counter there.  D2Q9 / D3Q19 directions cross at most
-    // two axes: the brick is chosen along the first axis, then the second.
+    int2 bnd = make_int2(0, 0);
+    if (BND) bnd = t.bnd_brick[b];
+    if (BND && bnd.y) {
+        // uniform: a brick with resolved boundary nodes; every offset first, then the loads
+        uint32_t o[Q];
+        for_each_source<D>(P, has_node, nbo, self, [&](int q, uint32_t off) { o[q] = off + 256u * q; });
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int cx = L::cx[q], cy = L::cy[q], cz = D == 3 ? L::cz[q] : 0;
-        const bool ex = cx == 1 ? clo[0] : (cx == -1 ? chi[0] : false);
-        const bool ey = cy == 1 ? clo[1] : (cy == -1 ? chi[1] : false);
-        const bool ez = cz == 1 ? clo[2] : (cz == -1 ? chi[2] : false);
-        const int dx = -cx, dy = -3 * cy, dz = -9 * cz;
-        uint32_t sel;
-        if (cx != 0 && cy != 0)
-            sel = ey ? (ex ? nbo[base + dx + dy] : nbo[base + dy]) : (ex ? nbo[base + dx] : self);
-        else if (cx != 0 && cz != 0)
-            sel = ez ? (ex ? nbo[base + dx + dz] : nbo[base + dz]) : (ex ? nbo[base + dx] : self);
-        else if (cy != 0 && cz != 0)
-            sel = ez ? (ey ? nbo[base + dy + dz] : nbo[base + dz]) : (ey ? nbo[base + dy] : self);
-        else if (cx != 0)
-            sel = ex ? nbo[base + dx] : self;
-        else if (cy != 0)
-            sel = ey ? nbo[base + dy] : self;
-        else if (cz != 0)
-            sel = ez ? nbo[base + dz] : self;
-        else
-            sel = self;
-        const uint32_t off = sel + (P.s4[0][1 - cx] | P.s4[1][1 - cy] | P.s4[2][1 - cz]);
+        for (int q = 1; q < Q; ++q)
+            if (bnd.y >> q & 1) o[q] = 4u * (uint32_t)t.bnd_src[(int64_t)bnd_row(bnd, q) * 64 + lane];
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            __builtin_amdgcn_global_load_lds((const void *)(reinterpret_cast<const char *>(fin) + o[q]),
+                                             (__attribute__((address_space(3))) void *)(buf + q * 64), 4, 0, 0);
+        if ((am >> lane) & 1ull) missing = t.aux_missing[t.auxbase[b] + __popcll(am & ((1ull << lane) - 1ull))];
+        return missing;
+    }
+    for_each_source<D>(P, has_node, nbo, self, [&](int q, uint32_t off) {
         // an opaque scalar base, so that the load takes the scalar-base + 32-bit-offset form
         const char *qbase = reinterpret_cast<const char *>(fin + q * 64);
         asm volatile("" : "+s"(qbase));
         const char *src = qbase + off;
         __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)(buf + q * 64),
                                          4, 0, 0);
-    }
-    uint32_t missing = 0;
-    const uint64_t am = t.auxmask[b];
+    });
     if ((am >> lane) & 1ull) missing = t.aux_missing[t.auxbase[b] + __popcll(am & ((1ull << lane) - 1ull))];
     return missing;
 }
@@ -638,14 +716,17 @@ __device__ __forceinline__ uint32_t pull_to_lds(const BrickTables &t, const T *_
 // the next pull, collide, store; the store group is unconditional so that the next round's wait
 // (in-order vector memory counter) covers the pull and not these stores.
 // Register budget: 4 waves per SIMD unforced, 3 forced (whose Guo terms would spill at 4).
-template <int D, typename T, typename C, bool SHIFT, int COLL, int VAR, int ROUNDS>
+// BND: the level has resolved boundary nodes (its own variant: on the other levels the table's two
+// pointers would cost the loop scalar spills, 130.1 against 128.9 us on a 3M-node level).
+template <int D, typename T, typename C, bool SHIFT, int COLL, int VAR, int ROUNDS, bool BND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((VAR & 1) ? 3 : 4)))
 void k_stream_collide_mlp(int64_t nbrick, int64_t naux, const uint64_t *__restrict__ occ,
                           const uint64_t *__restrict__ auxmask, const int32_t *__restrict__ auxbase,
                           const int32_t *__restrict__ nbr, const uint32_t *__restrict__ aux_missing,
+                          const int2 *__restrict__ bnd_brick, const int32_t *__restrict__ bnd_src,
                           const T *__restrict__ fin, T *__restrict__ fout, T *__restrict__ aux_f, StepParams p) {
     static_assert(mlp_on_mfma<C, VAR>(), "kernel of the FP32 learned closure");
-    const BrickTables t{occ, auxmask, auxbase, nbr, aux_missing};
+    const BrickTables t{occ, auxmask, auxbase, nbr, aux_missing, bnd_brick, bnd_src};
     using L = Lattice<D>;
     constexpr int Q = L::Q;
     __shared__ MlpOps ops;
@@ -658,7 +739,7 @@ void k_stream_collide_mlp(int64_t nbrick, int64_t naux, const uint64_t *__restri
     int64_t b = g * per_group + wave;
     // the first pull goes out before the network is staged, so that their latencies overlap
     uint32_t miss = 0;
-    if (b < nbrick) miss = pull_to_lds<D, T>(t, fin, b, threadIdx.x & 63, buf);
+    if (b < nbrick) miss = pull_to_lds<D, T, BND>(t, fin, b, threadIdx.x & 63, buf);
     stage_mlp_ops<((VAR & 15) >> 1) == 4, mrt_on_mfma<C, VAR>()>(ops, p.mlp->ops);
     if (b >= nbrick) return;                 // uniform per wave; no barrier follows
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the first pull has landed
@@ -710,7 +791,7 @@ void k_stream_collide_mlp(int64_t nbrick, int64_t naux, const uint64_t *__restri
         const int64_t bn = b + 4;
         const bool more = r + 1 < ROUNDS && bn < nbrick;
         uint32_t miss_next = 0;
-        if (more) miss_next = pull_to_lds<D, T>(t, fin, bn, lane, buf);
+        if (more) miss_next = pull_to_lds<D, T, BND>(t, fin, bn, lane, buf);
         if (!has_node) {
 #pragma unroll
             for (int q = 0; q < Q; ++q) f[q] = C(0);          // rest state (shifted storage)

@@ -113,10 +113,13 @@ struct IbPlan {
 // Roles of a node on the deferred ("aux") path.  Its post-stream values are kept in the aux array
 // (kAuxRecorded) for the boundary, transfer and forcing kernels to read or change; its collision
 // waits for the next substep's aux collision where they change after the fused kernel: after
-// every substep (kAuxDeferAlways: domain-boundary nodes, immersed-boundary supports, fine-to-
-// coarse targets and sources, nodes with an absent pull source) or only after the substeps that
+// every substep (kAuxDeferAlways: domain-boundary nodes of a level whose conditions are not
+// resolved in the pull, immersed-boundary supports, fine-to-coarse targets and sources, nodes with
+// an absent pull source) or only after the substeps that
 // the transfer into the level follows (kAuxDeferOnTransfer: coarse-to-fine ghost targets).  A
 // recorded node that is not deferred collides in the fused kernel like a bulk node.
+// node_aux of a bulk node: -1, or kResolvedBoundary on a domain face.
+constexpr int32_t kResolvedBoundary = -2;
 constexpr uint8_t kAuxRecorded = 1, kAuxDeferOnTransfer = 2, kAuxDeferAlways = 4;
 
 struct LevelState {
@@ -146,6 +149,13 @@ struct LevelState {
     DevBuf bc_u_d[7];   // [n][3] per-node boundary velocity of a profiled face (empty: uniform)
     int64_t bc_n[7] = {0, 0, 0, 0, 0, 0, 0};
     std::vector<int64_t> bnode[7], bpart[7];
+    // resolved boundaries (BoundaryPull): what each boundary node pulls per direction, as
+    // 8 x (node whose pull or own population it is) + face (0: that node's pull; else its own
+    // population of the opposite direction behind that face), -1: its own pull
+    bool resolved = false;
+    std::vector<int64_t> res_node;    // boundary nodes, ascending
+    std::vector<int64_t> res_code;    // [res_node][Q]
+    DevBuf bnd_brick_d, bnd_src_d, bnd_face_d, bnd_wall_d;
     TransferTables xfer;
     IbTables ibt;
     TransferPlan xplan;

@@ -154,6 +154,60 @@ __global__ void k_source_table(const int32_t *node_slot, int64_t n, const unsign
     }
 }
 
+// element of the population buffer that direction q of slot pulls (post-collision population at
+// x - c_q), or -1 where no node is there
+template <int D>
+__device__ __forceinline__ int32_t pull_element(const unsigned long long *occ, const int32_t *nbr, int64_t slot, int q) {
+    using L = Lattice<D>;
+    using B = Brick<D>;
+    const int64_t b = slot >> 6;
+    const int lane = (int)(slot & 63);
+    const int sx = B::lane_coord(lane, 0) - L::cx[q], sy = B::lane_coord(lane, 1) - L::cy[q];
+    const int sz = D == 3 ? B::lane_coord(lane, 2) - L::cz[q] : 0;
+    const int ox = sx < 0 ? -1 : (sx >= B::edge ? 1 : 0);
+    const int oy = sy < 0 ? -1 : (sy >= B::edge ? 1 : 0);
+    const int oz = D == 3 ? (sz < 0 ? -1 : (sz >= B::edge ? 1 : 0)) : 0;
+    const int k = D == 3 ? (oz + 1) * 9 + (oy + 1) * 3 + (ox + 1) : (oy + 1) * 3 + (ox + 1);
+    const int64_t sb = nbr[b * B::nnbr + k];
+    const int sl = B::lane_of(sx & (B::edge - 1), sy & (B::edge - 1), sz & (B::edge - 1));
+    if (sb < 0 || !((occ[sb] >> sl) & 1ull)) return -1;
+    return (int32_t)pop_at<L::Q>(q, sb * 64 + sl);
+}
+
+// rows of the pull tables (BoundaryPull; row[t]: {brick, direction}): first every lane's regular
+// source (its own slot where there is none), then the entries that the boundary conditions set
+// ({table entry, slot of the node, face}, LevelState::res_code)
+template <int D>
+__global__ void k_bnd_regular(int64_t nrow, const int2 *row, const unsigned long long *occ, const int32_t *nbr,
+                              int32_t *src) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nrow * 64) return;
+    const int2 r = row[t >> 6];
+    const int64_t slot = (int64_t)r.x * 64 + (t & 63);
+    const int32_t e = pull_element<D>(occ, nbr, slot, r.y);
+    src[t] = e >= 0 ? e : (int32_t)pop_at<Lattice<D>::Q>(r.y, slot);
+}
+
+struct BndEntry {
+    int32_t entry, slot, face;
+};
+
+template <int D>
+__global__ void k_bnd_entries(int64_t n, const BndEntry *e, const int2 *row, const unsigned long long *occ,
+                              const int32_t *nbr, int32_t *src, uint8_t *face) {
+    using L = Lattice<D>;
+    constexpr int Q = L::Q;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const BndEntry x = e[i];
+    const int q = row[x.entry >> 6].y;
+    int o = 0;
+    for (int p = 1; p < Q; ++p)
+        if (L::cx[p] == -L::cx[q] && L::cy[p] == -L::cy[q] && L::cz[p] == -L::cz[q]) o = p;
+    src[x.entry] = x.face ? (int32_t)pop_at<Q>(o, x.slot) : pull_element<D>(occ, nbr, x.slot, q);
+    if (face) face[x.entry] = (uint8_t)x.face;
+}
+
 // ----------------------------------------------------------------------------------------------
 // state upload / materialisation
 // ----------------------------------------------------------------------------------------------
@@ -177,6 +231,11 @@ __global__ void k_upload(BrickLevel<T> lv, const double *f_in, int64_t n, const 
     if (ai >= 0) {
 #pragma unroll
         for (int q = 0; q < Q; ++q) aux_f[q * lv.naux + ai] = T(f[q]);
+    }
+    // a boundary node's first collision starts from the stored form of the values, as an aux node's
+    if (ai == kResolvedBoundary) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) f[q] = C(T(f[q]));
     }
     const int64_t slot = active ? node_slot[i] : 0;
     if (active && ai < 0) {
@@ -206,6 +265,12 @@ __device__ __forceinline__ double post_stream_value(const BrickLevel<T> &lv, int
         v = double(aux_f[q * lv.naux + ai]);
     } else if (fresh || q == 0) {
         v = double(last[pop_at<Q>(q, slot)]);
+    } else if (lv.bnd.brick && (lv.bnd.brick[slot >> 6].y >> q & 1)) {
+        // what the fused kernel pulled: a brick with resolved boundary nodes
+        const int64_t e = (int64_t)bnd_row(lv.bnd.brick[slot >> 6], q) * 64 + (slot & 63);
+        T f = last[lv.bnd.src[e]];
+        if (lv.bnd.face && lv.bnd.face[e]) f = wall_value<Q, T>(lv.bnd.wall, lv.bnd.face[e], q, f);
+        v = double(f);
     } else {
         const int64_t b = slot >> 6;
         const int lane = (int)(slot & 63);
@@ -622,6 +687,8 @@ BrickLevel<T> view(const LevelState &L) {
     v.auxbase = L.auxbase_d.as<int32_t>();
     v.aux_missing = L.aux_missing_d.as<uint32_t>();
     v.aux_slot = L.aux_slot_d.as<int32_t>();
+    v.bnd = BoundaryPull{L.bnd_brick_d.as<int2>(), L.bnd_src_d.as<int32_t>(), L.bnd_face_d.as<uint8_t>(),
+                         L.bnd_wall_d.as<double2>()};
     return v;
 }
 
@@ -659,12 +726,12 @@ int64_t find_key(const std::vector<uint64_t> &keys, uint64_t k) {
 namespace {
 
 // learned-closure kernel with R rounds of four bricks per workgroup
-template <int D, typename T, typename C, bool SHIFT, int COLL, int V, int R>
+template <int D, typename T, typename C, bool SHIFT, int COLL, int V, int R, bool BND>
 void launch_mlp_rounds(zlh_ctx *ctx, const BrickLevel<T> &v, T *fa, T *fb, T *aux_f, const StepParams &sp) {
     const int64_t ng = (v.nbrick + 4 * R - 1) / (4 * R);
-    hipLaunchKernelGGL((k_stream_collide_mlp<D, T, C, SHIFT, COLL, V, R>), dim3((unsigned)((ng + 7) / 8 * 8)), dim3(256),
-                       0, ctx->stream, v.nbrick, v.naux, v.occ, v.auxmask, v.auxbase, v.nbr, v.aux_missing, fa, fb,
-                       aux_f, sp);
+    hipLaunchKernelGGL((k_stream_collide_mlp<D, T, C, SHIFT, COLL, V, R, BND>), dim3((unsigned)((ng + 7) / 8 * 8)), dim3(256),
+                       0, ctx->stream, v.nbrick, v.naux, v.occ, v.auxmask, v.auxbase, v.nbr, v.aux_missing,
+                       v.bnd.brick, v.bnd.src, fa, fb, aux_f, sp);
 }
 
 // one round per workgroup while the grid is at most two waves of resident workgroups (the
@@ -674,14 +741,21 @@ template <int D, typename T, typename C, bool SHIFT, int COLL, int V>
 void launch_mlp(zlh_ctx *ctx, const BrickLevel<T> &v, T *fa, T *fb, T *aux_f, const StepParams &sp) {
     static int per_cu = [] {
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_stream_collide_mlp<D, T, C, SHIFT, COLL, V, 1>, 256, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_stream_collide_mlp<D, T, C, SHIFT, COLL, V, 1, false>, 256, 0) !=
                 hipSuccess || n < 1)
             n = 1;
         return n;
     }();
     const int64_t resident = (int64_t)per_cu * ctx->n_cu;
-    if ((v.nbrick + 3) / 4 <= 2 * resident) launch_mlp_rounds<D, T, C, SHIFT, COLL, V, 1>(ctx, v, fa, fb, aux_f, sp);
-    else launch_mlp_rounds<D, T, C, SHIFT, COLL, V, 2>(ctx, v, fa, fb, aux_f, sp);
+    const bool one = (v.nbrick + 3) / 4 <= 2 * resident;
+    if (v.bnd.brick) {
+        if (one) launch_mlp_rounds<D, T, C, SHIFT, COLL, V, 1, true>(ctx, v, fa, fb, aux_f, sp);
+        else launch_mlp_rounds<D, T, C, SHIFT, COLL, V, 2, true>(ctx, v, fa, fb, aux_f, sp);
+    } else if (one) {
+        launch_mlp_rounds<D, T, C, SHIFT, COLL, V, 1, false>(ctx, v, fa, fb, aux_f, sp);
+    } else {
+        launch_mlp_rounds<D, T, C, SHIFT, COLL, V, 2, false>(ctx, v, fa, fb, aux_f, sp);
+    }
 }
 
 // bulk kernel variant: collision operator x (sub-grid model, forcing)
@@ -783,7 +857,7 @@ zlh_status launch_step_kernels(zlh_ctx *ctx, int level, int coll) {
     for (int a = 0; a < dims; ++a) { order[a] = 1 + 2 * a; order[dims + a] = 2 + 2 * a; }
     for (int k = 0; k < 2 * dims; ++k) {
         const int dir = order[k];
-        if (L.bc_n[dir] == 0) continue;
+        if (L.bc_n[dir] == 0 || L.resolved) continue;
         const BcIdx idx = bc_indices(dims, dir);
         const double *bv = ctx->d.bc_value[dir];
         switch (ctx->d.bc_scheme[dir]) {
@@ -977,6 +1051,133 @@ void host_feq(int dims, double rho, const double *u, int compressible, double *f
 // ==============================================================================================
 namespace {
 
+// Resolves the boundary conditions of a level whose faces are all bounce-back or periodic: follows
+// the reference's order of faces and records, for each population a condition sets, the pull of a
+// node or a node's own population of the opposite direction that ends up there.  Each is a copy of
+// one value of the buffer the fused kernel reads (with a moving wall's term), so pulling it there
+// gives the bits that the launches per face give.  Not resolved: a periodic twin whose own source
+// is absent (it keeps an earlier value), and moving walls with the FP32 learned closure (its pull
+// goes straight to LDS).  Resolved populations are no longer missing.
+void resolve_boundaries(const zlh_ctx *ctx, LevelState &L) {
+    const int dims = ctx->d.dims, Q = ctx->q;
+    L.resolved = false;
+    L.res_node.clear();
+    L.res_code.clear();
+    bool any = false;
+    for (int dir = 1; dir <= 2 * dims; ++dir) {
+        if (L.bnode[dir].empty()) continue;
+        any = true;
+        const int scheme = ctx->d.bc_scheme[dir];
+        if (scheme != ZLH_BC_BOUNCE_BACK && scheme != ZLH_BC_PERIODIC) return;
+        if (scheme == ZLH_BC_BOUNCE_BACK && ctx->d.les == ZLH_LES_MLP && ctx->d.precision == ZLH_FP32_SHIFTED)
+            for (int a = 0; a < dims; ++a)
+                if (ctx->d.bc_value[dir][a] != 0.) return;
+    }
+    if (!any) return;
+    std::vector<int32_t> at(L.n, -1);
+    std::vector<int64_t> node, code;
+    for (int dir = 1; dir <= 2 * dims; ++dir)
+        for (int64_t i : L.bnode[dir]) at[i] = 0;
+    for (int64_t i = 0; i < L.n; ++i)
+        if (at[i] == 0) {
+            at[i] = (int32_t)node.size();
+            node.push_back(i);
+        }
+    code.assign(node.size() * Q, -1);
+    for (int k = 0; k < 2 * dims; ++k) {
+        const int dir = k < dims ? 1 + 2 * k : 2 + 2 * (k - dims);
+        const BcIdx idx = bc_indices(dims, dir);
+        for (size_t e = 0; e < L.bnode[dir].size(); ++e) {
+            const int64_t i = L.bnode[dir][e], j = L.bpart[dir][e];
+            for (int m = 0; m < idx.n; ++m) {
+                const int q = idx.ind[m];
+                int64_t &c = code[(size_t)at[i] * Q + q];
+                if (ctx->d.bc_scheme[dir] == ZLH_BC_BOUNCE_BACK) {
+                    c = 8 * i + dir;
+                } else if (j >= 0) {
+                    const int64_t cj = at[j] >= 0 ? code[(size_t)at[j] * Q + q] : -1;
+                    c = cj >= 0 ? cj : 8 * j;
+                }
+            }
+        }
+    }
+    for (size_t e = 0; e < node.size(); ++e)
+        for (int q = 1; q < Q; ++q) {
+            const int64_t c = code[e * Q + q];
+            if (c >= 0 && (c & 7) == 0 && (L.missing_h[c >> 3] >> q & 1u)) return;
+        }
+    for (size_t e = 0; e < node.size(); ++e)
+        for (int q = 1; q < Q; ++q)
+            if (code[e * Q + q] >= 0) L.missing_h[node[e]] &= ~(1u << q);
+    L.res_node = std::move(node);
+    L.res_code = std::move(code);
+    L.resolved = true;
+}
+
+// device tables of the resolved boundary nodes (BoundaryPull)
+zlh_status upload_resolved(zlh_ctx *ctx, int level) {
+    LevelState &L = ctx->lv[level];
+    for (DevBuf *d : {&L.bnd_brick_d, &L.bnd_src_d, &L.bnd_face_d, &L.bnd_wall_d}) *d = DevBuf();
+    if (!L.resolved) return ZLH_OK;
+    const int dims = ctx->d.dims, Q = ctx->q;
+    bool moving = false;
+    std::vector<double2> wall(7 * Q, make_double2(0., 0.));
+    for (int dir = 1; dir <= 2 * dims; ++dir)
+        if (ctx->d.bc_scheme[dir] == ZLH_BC_BOUNCE_BACK) {
+            const double *u = ctx->d.bc_value[dir];
+            for (int a = 0; a < dims; ++a) moving |= u[a] != 0. && !L.bnode[dir].empty();
+            for (int q = 1; q < Q; ++q) {
+                const int o = dims == 2 ? opposite<2>(q) : opposite<3>(q);
+                const double w = dims == 2 ? Lattice<2>::w[o] : Lattice<3>::w[o];
+                const double cu = dims == 2 ? Lattice<2>::cx[o] * u[0] + Lattice<2>::cy[o] * u[1]
+                                            : Lattice<3>::cx[o] * u[0] + Lattice<3>::cy[o] * u[1] + Lattice<3>::cz[o] * u[2];
+                wall[dir * Q + q] = make_double2(6. * ctx->d.rho0 * w, cu);
+            }
+        }
+    std::vector<int2> brick(L.nbrick, make_int2(0, 0)), row;
+    for (size_t e = 0; e < L.res_node.size(); ++e)
+        for (int q = 1; q < Q; ++q)
+            if (L.res_code[e * Q + q] >= 0) brick[L.node_slot_h[L.res_node[e]] >> 6].y |= 1 << q;
+    for (int64_t b = 0; b < L.nbrick; ++b) {
+        brick[b].x = (int32_t)row.size();
+        for (int q = 1; q < Q; ++q)
+            if (brick[b].y >> q & 1) row.push_back(make_int2((int32_t)b, q));
+    }
+    std::vector<BndEntry> entries;
+    for (size_t e = 0; e < L.res_node.size(); ++e) {
+        const int32_t slot = L.node_slot_h[L.res_node[e]];
+        for (int q = 1; q < Q; ++q) {
+            const int64_t c = L.res_code[e * Q + q];
+            if (c >= 0) entries.push_back({bnd_row(brick[slot >> 6], q) * 64 + (slot & 63), L.node_slot_h[c >> 3], (int32_t)(c & 7)});
+        }
+    }
+    const int64_t nrow = (int64_t)row.size();
+    if (nrow == 0) return ZLH_OK;
+    DevBuf rows, ent;
+    zlh_status s;
+    if ((s = upload(ctx, L.bnd_brick_d, brick))) return s;
+    if ((s = upload(ctx, rows, row))) return s;
+    if ((s = upload(ctx, ent, entries))) return s;
+    if ((s = dalloc(ctx, L.bnd_src_d, sizeof(int32_t) * nrow * 64, false))) return s;
+    if (moving) {
+        if ((s = dalloc(ctx, L.bnd_face_d, (size_t)nrow * 64))) return s;
+        if ((s = upload(ctx, L.bnd_wall_d, wall))) return s;
+    }
+    auto build = [&](auto regular, auto set) {
+        hipLaunchKernelGGL(regular, dim3(blocks(nrow * 64)), dim3(256), 0, ctx->stream, nrow, rows.as<int2>(),
+                           L.occ_d.as<unsigned long long>(), L.nbr_d.as<int32_t>(), L.bnd_src_d.as<int32_t>());
+        hipLaunchKernelGGL(set, dim3(blocks((int64_t)entries.size())), dim3(256), 0, ctx->stream,
+                           (int64_t)entries.size(), ent.as<BndEntry>(), rows.as<int2>(),
+                           L.occ_d.as<unsigned long long>(), L.nbr_d.as<int32_t>(), L.bnd_src_d.as<int32_t>(),
+                           L.bnd_face_d.as<uint8_t>());
+    };
+    if (dims == 2) build(k_bnd_regular<2>, k_bnd_entries<2>);
+    else build(k_bnd_regular<3>, k_bnd_entries<3>);
+    ZLH_TRY(hipGetLastError());
+    ZLH_TRY(hipStreamSynchronize(ctx->stream));   // the entries are freed on return
+    return ZLH_OK;
+}
+
 // phase 1: device slot / neighbour tables and the absent-source masks
 zlh_status build_level_slots(zlh_ctx *ctx, int level) {
     LevelState &L = ctx->lv[level];
@@ -1026,10 +1227,7 @@ zlh_status build_level_slots(zlh_ctx *ctx, int level) {
     ZLH_TRY(hipStreamSynchronize(ctx->stream));
     for (int64_t i = 0; i < L.n; ++i)
         if (L.node_slot_h[i] < 0) return ctx->fail(ZLH_EDEVICE, "slot lookup failed for node %lld", (long long)i);
-    // nodes with an absent pull source keep that population from the previous substep
     L.aux_mark.assign(L.n, 0);
-    for (int64_t i = 0; i < L.n; ++i)
-        if (L.missing_h[i]) L.aux_mark[i] = kAuxRecorded | kAuxDeferAlways;
     // domain boundaries (CheckIfNodeOutsideCubicDomain, grid/grid_info.cpp:84-142) and the
     // nodes their conditions read
     for (int d = 0; d < 7; ++d) { L.bnode[d].clear(); L.bpart[d].clear(); }
@@ -1052,12 +1250,21 @@ zlh_status build_level_slots(zlh_ctx *ctx, int level) {
                 }
                 L.bnode[dir].push_back(i);
                 L.bpart[dir].push_back(partner);
-                L.aux_mark[i] |= kAuxRecorded | kAuxDeferAlways;
-                if (partner >= 0) L.aux_mark[partner] |= kAuxRecorded;   // read by the condition
             }
         }
     }
-    return ZLH_OK;
+    resolve_boundaries(ctx, L);
+    if (!L.resolved)
+        for (int dir = 1; dir <= 2 * dims; ++dir)
+            for (size_t k = 0; k < L.bnode[dir].size(); ++k) {
+                L.aux_mark[L.bnode[dir][k]] |= kAuxRecorded | kAuxDeferAlways;
+                if (L.bpart[dir][k] >= 0) L.aux_mark[L.bpart[dir][k]] |= kAuxRecorded;   // read by the condition
+            }
+    // nodes with an absent pull source that no boundary condition sets keep that population from
+    // the previous substep
+    for (int64_t i = 0; i < L.n; ++i)
+        if (L.missing_h[i]) L.aux_mark[i] |= kAuxRecorded | kAuxDeferAlways;
+    return upload_resolved(ctx, level);
 }
 
 // phase 2: deferred-node arrays, boundary tables and population storage
@@ -1077,6 +1284,7 @@ zlh_status build_level_aux(zlh_ctx *ctx, int level) {
     std::vector<int32_t> auxbase(L.nbrick, 0), aux_slot(L.naux);
     std::vector<uint32_t> aux_missing(L.naux);
     L.node_aux_h.assign(L.n, -1);
+    for (int64_t i : L.res_node) L.node_aux_h[i] = kResolvedBoundary;
     for (int64_t k = 0; k < L.naux; ++k) {
         const int64_t i = aux_nodes[k];
         const int32_t slot = L.node_slot_h[i];
