@@ -165,8 +165,8 @@ zlh_status zlh_transfer_to_coarse(zlh_ctx *ctx, int fine_level);
 /* background steps in the coarse-to-fine multi time stepping order (AmrManager::TimeMarching,
  * amr_manager.cpp:279-300; MultiTimeSteppingC2F, grid/grid_manager.cpp:997-1024) */
 zlh_status zlh_time_marching(zlh_ctx *ctx, int nsteps);
-/* zlh_time_marching replays pairs of background steps as captured HIP graphs (default on);
- * off launches every kernel directly (no reference counterpart) */
+/* zlh_time_marching replays pairs of background steps of refined grids as captured HIP graphs
+ * (default on); off launches every kernel directly (no reference counterpart) */
 zlh_status zlh_graphs_enable(zlh_ctx *ctx, int enable);
 /* run each level's substeps of zlh_time_marching on a stream of its own, ordered by events
  * around the transfers, so that coarse levels overlap finer ones (default 1; no reference

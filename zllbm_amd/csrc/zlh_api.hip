@@ -1781,8 +1781,12 @@ zlh_status zlh_time_marching(zlh_ctx *ctx, int nsteps) {
     if (nsteps < 0) return ctx->fail(ZLH_EINVAL, "negative step count");
     // launch-bound multi-level steps replay captured graphs: of two background steps while two
     // remain (level 0's buffer index comes back to where it was), of one step for an odd last
-    // one.  Timing (per-launch events) runs the launches directly.
-    if (!ctx->use_graphs || ctx->timing) return march_launches(ctx, nsteps);
+    // one.  Timing (per-launch events) runs the launches directly, and so does a single level: its
+    // few launches take the host less time each (about 4.8 us a step with resolved boundaries) than
+    // the device, while a graph launch takes 16 us for two steps (a 128^2 FP64 cavity: 5.8 against
+    // 8.2 us a step; one step waited for: 15 against 36 us).  A 7-substep step of three small levels
+    // takes 83 us launched directly and 74 as a graph.
+    if (!ctx->use_graphs || ctx->timing || ctx->d.max_level == 0) return march_launches(ctx, nsteps);
     int t = 0;
     while (t < nsteps) {
         const int n = nsteps - t >= 2 ? 2 : 1;
