@@ -1,0 +1,87 @@
+"""Time marching launches the levels that step together at once; the substep entry points launch
+one level at a time in the reference's order.  Both give the same bits."""
+import numpy as np
+import pytest
+
+from zllbm_amd import grid as g
+from zllbm_amd import hip
+from tests import scenarios as sc
+
+pytestmark = pytest.mark.gpu
+
+
+def _nested(levels):
+    """2D box with `levels` nested levels around its middle (16 cells of each level's spacing)."""
+    boxes, c = [], 13
+    for _ in range(levels - 1):
+        boxes.append(((c - 4, c - 4), (c + 4, c + 4)))
+        c *= 2
+    return g.refined_box_grid(2, (24, 24), boxes)
+
+
+def _reference_order(s, top):
+    count = [0] * (top + 1)
+
+    def step(l):
+        count[l] += 1
+        s.step_level(l, count[l])
+        if l > 0 and count[l] % 2 == 0:
+            s.transfer_levels(l)
+        if l < top:
+            step(l + 1)
+            step(l + 1)
+    step(0)
+
+
+# 8 levels: more than one launch takes
+@pytest.mark.parametrize("levels,graphs", [(2, True), (3, True), (4, True), (8, False)])
+@pytest.mark.parametrize("precision,collision", [(hip.FP64, (hip.MRT,)), (hip.FP32_SHIFTED, (hip.SRT, hip.SRT, hip.MRT)),
+                                                 (hip.BF16_SHIFTED, (hip.MRT, hip.SRT))])
+@pytest.mark.parametrize("scheme", [sc.PER, sc.BB, sc.NEE])
+def test_marching_equals_substeps(levels, graphs, precision, collision, scheme):
+    grid = _nested(levels)
+    kw = dict(nu0=2e-3, bc=sc.all_bc(2, scheme), collision=collision, precision=precision)
+    a, b = hip.Solver(grid, **kw).build(), hip.Solver(grid, **kw).build()
+    a.graphs_enable(graphs)
+    for l in range(levels):
+        rho, u = sc.level_fields(grid, l, u0=0.02)
+        for s in (a, b):
+            s.init_macro(l, rho, u)
+    a.time_marching(3)
+    for _ in range(3):
+        _reference_order(b, levels - 1)
+    for l in range(levels):
+        np.testing.assert_array_equal(a.f(l), b.f(l))
+    a.time_marching(2)
+    for _ in range(2):
+        _reference_order(b, levels - 1)
+    for l in range(levels):
+        np.testing.assert_array_equal(a.f(l), b.f(l))
+
+
+@pytest.mark.parametrize("les,precision", [(hip.LES_SMAGORINSKY, hip.FP32_SHIFTED), (hip.LES_MLP, hip.FP32_SHIFTED)])
+def test_marching_equals_substeps_3d_forced(les, precision):
+    """The learned closure's kernel with a resolved and an unresolved level in one launch, and
+    immersed-boundary markers on the finer one."""
+    import os
+    from zllbm_amd import closure, geometry
+    from tests.test_gpu_mlp import ROOT
+    grid, kw = sc.amr3d()
+    kw.update(collision=(hip.MRT,), les=les, cs=0.1, precision=precision, has_force=True)
+    xyz, area = geometry.fibonacci_sphere_markers((8.5, 8.5, 8.5), 1.5, 0.5)
+    runs = []
+    for _ in range(2):
+        s = hip.Solver(grid, **kw)
+        s.set_ib(1, xyz, area, np.zeros_like(xyz))
+        s.build()
+        if les == hip.LES_MLP:
+            s.mlp_set(closure.ClosureModel.load(os.path.join(ROOT, "zllbm_amd", "data", "closure_turbulence.npz")))
+        for l in range(2):
+            s.init_macro(l, *sc.level_fields(grid, l, u0=0.03))
+        runs.append(s)
+    runs[0].time_marching(4)
+    for _ in range(4):
+        _reference_order(runs[1], 1)
+    for l in range(2):
+        np.testing.assert_array_equal(runs[0].f(l), runs[1].f(l))
+    np.testing.assert_array_equal(runs[0].ib_force(1), runs[1].ib_force(1))

@@ -455,13 +455,63 @@ __device__ __forceinline__ void collide(C (&f)[Lattice<D>::Q], const C *F, const
 }
 
 // workgroup -> brick group mapping that gives each of the 8 XCDs a contiguous range of bricks
-// (Morton order), so neighbouring bricks meet in the same L2
-__device__ __forceinline__ int64_t xcd_group(int64_t ngroups) {
-    const int64_t nb = gridDim.x;
-    const int64_t per = nb >> 3;   // grid is a multiple of 8
-    const int64_t bid = blockIdx.x;
+// (Morton order), so neighbouring bricks meet in the same L2: workgroup bid of nb (a multiple of 8)
+__device__ __forceinline__ int64_t xcd_group(int64_t ngroups, int64_t bid, int64_t nb) {
+    const int64_t per = nb >> 3;
     const int64_t g = (bid & 7) * per + (bid >> 3);
     return g < ngroups ? g : -1;
+}
+__device__ __forceinline__ int64_t xcd_group(int64_t ngroups) { return xcd_group(ngroups, blockIdx.x, gridDim.x); }
+
+// Levels that step at the same time share a launch: the steps of a coarse level and of the first
+// substeps of the levels inside it touch nothing in common, and a small level's launch is all
+// latency (7 to 10 us at a few hundred bricks).  Workgroups [first[i], first[i + 1]) take run i;
+// coarse levels come first, so that their few workgroups are not the tail of the launch.
+// first[i] is a multiple of 8 in the fused kernels (xcd_group).
+constexpr int kMaxBatch = 6;
+template <typename Run>
+struct Batch {
+    int32_t n;
+    uint32_t first[kMaxBatch + 1];
+    Run run[kMaxBatch];
+    // run of this workgroup (uniform)
+    __device__ __forceinline__ int find() const {
+        int k = 0;
+#pragma unroll
+        for (int i = 1; i < kMaxBatch; ++i)
+            if (i < n && blockIdx.x >= first[i]) k = i;
+        return __builtin_amdgcn_readfirstlane(k);
+    }
+};
+
+// one level's fused step: pulls from fin, writes fout and the deferred nodes' values
+template <typename T>
+struct FusedRun {
+    BrickLevel<T> lv;
+    const T *fin;
+    T *fout, *aux_f;
+    StepParams p;
+};
+
+// one level's aux collision: entries of list (or every recorded node, list null) of aux_f into fa,
+// rho and u of the nodes flagged in macro_flag
+template <typename T>
+struct AuxRun {
+    int64_t naux, nlist;
+    const int32_t *list, *aux_slot;
+    const T *aux_f;
+    const double *aux_force;
+    T *fa;
+    double *aux_macro;
+    const uint8_t *macro_flag;
+    StepParams p;
+};
+
+// read-only table entry through the constant address space: a uniform load goes through the
+// scalar cache whatever the kernel stores, so it does not wait on the vector memory counter
+template <typename X>
+__device__ __forceinline__ X table_load(const X *p, int64_t i) {
+    return ((const __attribute__((address_space(4))) X *)(p))[i];
 }
 
 // Per-lane constants of the pull, fixed by the brick layout and computed once per pull: the
@@ -618,31 +668,20 @@ __device__ __forceinline__ void stream_collide_brick(const BrickLevel<T> &lv, co
     for (int q = 0; q < Q; ++q) store_nt(T(f[q]), dst + q * 64);
 }
 
-// Fused pull-stream + collide over all nodes of a level, one wavefront per brick, four bricks
-// per workgroup.
+// Fused pull-stream + collide over all nodes of the levels of a batch, one wavefront per brick,
+// four bricks per workgroup.
 template <int D, typename T, typename C, bool SHIFT, int COLL, int VAR>
-__global__ __launch_bounds__(256) void k_stream_collide(BrickLevel<T> lv, const T *__restrict__ fin,
-                                                        T *__restrict__ fout, T *__restrict__ aux_f,
-                                                        StepParams p) {
-    const int64_t g = xcd_group((lv.nbrick + 3) >> 2);
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(std::is_same<C, float>::value && !(VAR & 1) ? 8 : 1)))
+void k_stream_collide(Batch<FusedRun<T>> B) {
+    const int k = B.find();
+    const FusedRun<T> &R = B.run[k];
+    const int64_t g = xcd_group((R.lv.nbrick + 3) >> 2, blockIdx.x - B.first[k], B.first[k + 1] - B.first[k]);
     if (g < 0) return;
     const int64_t b = g * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (b >= lv.nbrick) return;
-    stream_collide_brick<D, T, C, SHIFT, COLL, VAR>(lv, fin, fout, aux_f, p, b, nullptr);
+    if (b >= R.lv.nbrick) return;
+    stream_collide_brick<D, T, C, SHIFT, COLL, VAR>(R.lv, R.fin, R.fout, R.aux_f, R.p, b, nullptr);
 }
-
-// Read-only brick tables of a level (the kernel takes them as no-alias parameters: it stores into
-// the population arrays inside its loop, and only provably unclobbered tables are read through
-// the scalar cache, whose loads do not wait on the vector memory counter).
-struct BrickTables {
-    const uint64_t *__restrict__ occ;
-    const uint64_t *__restrict__ auxmask;
-    const int32_t *__restrict__ auxbase;
-    const int32_t *__restrict__ nbr;
-    const uint32_t *__restrict__ aux_missing;
-    const int2 *__restrict__ bnd_brick;   // BoundaryPull::brick and ::src (null: no resolved boundaries)
-    const int32_t *__restrict__ bnd_src;
-};
 
 // Pull of brick b (every lane, every direction) into a per-wave LDS buffer [Q][64] with one
 // direct-to-LDS dword load per direction (gfx950 global_load_lds_dword: lane i lands at
@@ -652,14 +691,14 @@ struct BrickTables {
 // missing directions keep the boundary / transfer values already in the aux array).  Addresses are 32-bit byte offsets
 // from the direction's base fin + 64 q.  Returns the lane's missing-source mask (deferred nodes).
 template <int D, typename T, bool BND>
-__device__ __forceinline__ uint32_t pull_to_lds(const BrickTables &t, const T *__restrict__ fin, int64_t b, int lane,
+__device__ __forceinline__ uint32_t pull_to_lds(const BrickLevel<T> &t, const T *__restrict__ fin, int64_t b, int lane,
                                                 T *buf) {
     using L = Lattice<D>;
     using B = Brick<D>;
     constexpr int Q = L::Q;
     constexpr int NN = B::nnbr;
     static_assert(sizeof(T) == 4, "dword staging");
-    const uint64_t am = t.auxmask[b];
+    const uint64_t am = table_load(t.auxmask, b);
     uint32_t missing = 0;
     // opaque per pull: the direction's LDS destinations are formed here, not hoisted out of the
     // caller's loop into 19 long-lived scalars
@@ -670,29 +709,32 @@ __device__ __forceinline__ uint32_t pull_to_lds(const BrickTables &t, const T *_
     uint32_t nbo[NN];
 #pragma unroll
     for (int k = 0; k < NN; ++k) {
-        const int32_t v = t.nbr[b * NN + k];
+        const int32_t v = table_load(t.nbr, b * NN + k);
         nbo[k] = (uint32_t)(v < 0 ? (int32_t)b : v) * kBrickBytes;
     }
     // a lane crosses into a neighbour brick only if it holds a node: a lane without one loads
     // the slot its stencil names inside its own brick, a line the brick's own pull fetches anyway
-    const bool has_node = (t.occ[b] >> lane) & 1ull;
+    const bool has_node = (table_load(t.occ, b) >> lane) & 1ull;
     constexpr int base = D == 3 ? 13 : 4;
     uint32_t self = nbo[base];
     asm volatile("" : "+v"(self));
     int2 bnd = make_int2(0, 0);
-    if (BND) bnd = t.bnd_brick[b];
+    if (BND && t.bnd.brick) {
+        bnd.x = table_load(reinterpret_cast<const int32_t *>(t.bnd.brick), 2 * b);
+        bnd.y = table_load(reinterpret_cast<const int32_t *>(t.bnd.brick), 2 * b + 1);
+    }
     if (BND && bnd.y) {
         // uniform: a brick with resolved boundary nodes; every offset first, then the loads
         uint32_t o[Q];
         for_each_source<D>(P, has_node, nbo, self, [&](int q, uint32_t off) { o[q] = off + 256u * q; });
 #pragma unroll
         for (int q = 1; q < Q; ++q)
-            if (bnd.y >> q & 1) o[q] = 4u * (uint32_t)t.bnd_src[(int64_t)bnd_row(bnd, q) * 64 + lane];
+            if (bnd.y >> q & 1) o[q] = 4u * (uint32_t)t.bnd.src[(int64_t)bnd_row(bnd, q) * 64 + lane];
 #pragma unroll
         for (int q = 0; q < Q; ++q)
             __builtin_amdgcn_global_load_lds((const void *)(reinterpret_cast<const char *>(fin) + o[q]),
                                              (__attribute__((address_space(3))) void *)(buf + q * 64), 4, 0, 0);
-        if ((am >> lane) & 1ull) missing = t.aux_missing[t.auxbase[b] + __popcll(am & ((1ull << lane) - 1ull))];
+        if ((am >> lane) & 1ull) missing = t.aux_missing[table_load(t.auxbase, b) + __popcll(am & ((1ull << lane) - 1ull))];
         return missing;
     }
     for_each_source<D>(P, has_node, nbo, self, [&](int q, uint32_t off) {
@@ -703,7 +745,7 @@ __device__ __forceinline__ uint32_t pull_to_lds(const BrickTables &t, const T *_
         __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)(buf + q * 64),
                                          4, 0, 0);
     });
-    if ((am >> lane) & 1ull) missing = t.aux_missing[t.auxbase[b] + __popcll(am & ((1ull << lane) - 1ull))];
+    if ((am >> lane) & 1ull) missing = t.aux_missing[table_load(t.auxbase, b) + __popcll(am & ((1ull << lane) - 1ull))];
     return missing;
 }
 
@@ -720,19 +762,22 @@ __device__ __forceinline__ uint32_t pull_to_lds(const BrickTables &t, const T *_
 // pointers would cost the loop scalar spills, 130.1 against 128.9 us on a 3M-node level).
 template <int D, typename T, typename C, bool SHIFT, int COLL, int VAR, int ROUNDS, bool BND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((VAR & 1) ? 3 : 4)))
-void k_stream_collide_mlp(int64_t nbrick, int64_t naux, const uint64_t *__restrict__ occ,
-                          const uint64_t *__restrict__ auxmask, const int32_t *__restrict__ auxbase,
-                          const int32_t *__restrict__ nbr, const uint32_t *__restrict__ aux_missing,
-                          const int2 *__restrict__ bnd_brick, const int32_t *__restrict__ bnd_src,
-                          const T *__restrict__ fin, T *__restrict__ fout, T *__restrict__ aux_f, StepParams p) {
+void k_stream_collide_mlp(Batch<FusedRun<T>> B) {
     static_assert(mlp_on_mfma<C, VAR>(), "kernel of the FP32 learned closure");
-    const BrickTables t{occ, auxmask, auxbase, nbr, aux_missing, bnd_brick, bnd_src};
+    const int run = B.find();
+    const FusedRun<T> &R = B.run[run];
+    const BrickLevel<T> &t = R.lv;
+    const T *fin = R.fin;
+    T *fout = R.fout, *aux_f = R.aux_f;
+    const StepParams &p = R.p;
+    const int64_t nbrick = t.nbrick, naux = t.naux;
     using L = Lattice<D>;
     constexpr int Q = L::Q;
     __shared__ MlpOps ops;
     __shared__ T stage[4][Q * 64];
     constexpr int64_t per_group = 4 * ROUNDS;
-    const int64_t g = xcd_group((nbrick + per_group - 1) / per_group);
+    const int64_t g = xcd_group((nbrick + per_group - 1) / per_group, blockIdx.x - B.first[run],
+                                B.first[run + 1] - B.first[run]);
     if (g < 0) return;                       // uniform per workgroup: before the barrier
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     T *buf = stage[wave];
@@ -755,15 +800,15 @@ void k_stream_collide_mlp(int64_t nbrick, int64_t naux, const uint64_t *__restri
         C f[Q];
 #pragma unroll
         for (int q = 0; q < Q; ++q) f[q] = C(buf[q * 64 + lane]);
-        const bool has_node = (t.occ[b] >> lane) & 1ull;
-        const uint64_t am = t.auxmask[b];
+        const bool has_node = (table_load(t.occ, b) >> lane) & 1ull;
+        const uint64_t am = table_load(t.auxmask, b);
         if ((am >> lane) & 1ull) {
             // deferred node: post-stream values to the aux array, except the missing sources
             // (their boundary / transfer values are there already): those go to the spare slot
             // at index Q naux.  Stores take a uniform base and a 32-bit byte offset (the host
             // keeps Q naux 4 below 2^32); a wavefront whose deferred lanes miss no source (a
             // uniform branch) stores without the per-direction selection.
-            const uint32_t ai4 = 4u * (uint32_t)(t.auxbase[b] + __popcll(am & ((1ull << lane) - 1ull)));
+            const uint32_t ai4 = 4u * (uint32_t)(table_load(t.auxbase, b) + __popcll(am & ((1ull << lane) - 1ull)));
             using gchar = __attribute__((address_space(1))) char;
             using gT = __attribute__((address_space(1))) T;
             gchar *base = (gchar *)aux_f;
@@ -810,21 +855,24 @@ void k_stream_collide_mlp(int64_t nbrick, int64_t naux, const uint64_t *__restri
     }
 }
 
-// Collision of the aux nodes (deferred from the previous substep), writing post-collision
+// Collision of the aux nodes of the levels of a batch (deferred from the previous substep), writing post-collision
 // values into the buffer the next fused kernel reads, plus rho/u (GridNodeLbm::rho_/velocity_) of
 // the nodes flagged in macro_flag (the fine-to-coarse sources, the only readers).
 // VAR as in the fused kernel; with the FP32 learned closure the workgroup stages the network in
 // LDS first.
 template <int D, typename T, typename C, bool SHIFT, int COLL, int VAR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(mlp_on_mfma<C, VAR>() ? ((VAR & 1) ? 3 : 4) : 1)))
-void k_aux_collide(BrickLevel<T> lv, const int32_t *__restrict__ list, int64_t nlist,
-                                                     const T *__restrict__ aux_f,
-                                                     const double *__restrict__ aux_force,
-                                                     T *__restrict__ fa, double *__restrict__ aux_macro,
-                                                     const uint8_t *__restrict__ macro_flag, StepParams p) {
+void k_aux_collide(Batch<AuxRun<T>> B) {
+    const int run = B.find();
+    const AuxRun<T> &R = B.run[run];
+    const int32_t *__restrict__ list = R.list;
+    const int64_t nlist = R.nlist, naux = R.naux;
+    const T *__restrict__ aux_f = R.aux_f;
+    const double *__restrict__ aux_force = R.aux_force;
+    const StepParams &p = R.p;
     constexpr int Q = Lattice<D>::Q;
     constexpr bool kWave = mlp_on_mfma<C, VAR>();
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t t = (int64_t)(blockIdx.x - B.first[run]) * blockDim.x + threadIdx.x;
     // lanes past the end run the collision on the rest state (FP32 learned closure is
     // wavefront-wide) and store nothing
     const bool active = t < nlist;
@@ -833,7 +881,7 @@ void k_aux_collide(BrickLevel<T> lv, const int32_t *__restrict__ list, int64_t n
     if (!kWave && !active) return;
     C f[Q];
 #pragma unroll
-    for (int q = 0; q < Q; ++q) f[q] = active ? C(aux_f[q * lv.naux + i]) : C(SHIFT ? 0. : Lattice<D>::w[q]);
+    for (int q = 0; q < Q; ++q) f[q] = active ? C(aux_f[q * naux + i]) : C(SHIFT ? 0. : Lattice<D>::w[q]);
     // the network is staged after the node's loads are out, so that their latencies overlap
     const MlpOps *ops = nullptr;
     if constexpr (kWave) {
@@ -848,10 +896,12 @@ void k_aux_collide(BrickLevel<T> lv, const int32_t *__restrict__ list, int64_t n
     C rho, u[3];
     collide<D, SHIFT, COLL, C, VAR>(f, F, p, rho, u, ops);
     if (!active) return;
-    const int64_t slot = lv.aux_slot[i];
+    T *__restrict__ fa = R.fa;
+    const int64_t slot = R.aux_slot[i];
 #pragma unroll
     for (int q = 0; q < Q; ++q) fa[pop_at<Q>(q, slot)] = T(f[q]);
-    if (macro_flag[i]) {
+    if (R.macro_flag[i]) {
+        double *__restrict__ aux_macro = R.aux_macro;
         aux_macro[i * 4] = double(rho);
         aux_macro[i * 4 + 1] = double(u[0]);
         aux_macro[i * 4 + 2] = double(u[1]);

@@ -369,7 +369,7 @@ class Solver:
         self._chk(lib().zlh_set_moment_transform(self.h, where))
 
     def level_streams_enable(self, on=True):
-        """Run each level's substeps on a stream of its own (default on); results are identical."""
+        """Accepted without effect: levels that step together share launches (zlh_level_streams_enable)."""
         self._chk(lib().zlh_level_streams_enable(self.h, 1 if on else 0))
 
     def synchronize(self):
