@@ -31,67 +31,64 @@ __device__ __forceinline__ void macro_feq_double(const double *f, int compressib
 }
 
 // NodeInfoCoarse2fine (lbm_grid_interface.cpp:570-588) + PostStreamCoarse2Fine
-// (lbm_collision_models.cpp:244-251) for every coarse node that feeds an interpolation stencil,
-// and a plain copy of every fine node that stands in for a missing coarse one.  The rows are
-// stored node-major, [n_src + n_fb][Q], in the populations' storage form (FP64, or FP32 shifted by
-// w), so that each stencil contributor is one contiguous row; both row sets are sorted by aux
-// index, so consecutive threads read neighbouring entries of each direction's plane.  A
-// workgroup's 256 rows go out through LDS as one contiguous, coalesced run.
-// MID (time interpolation after an odd fine substep): each coarse row is the mean of the row
-// computed now and the row `prev` of the last synchronised transfer, i.e. of the coarse state
-// before and after the coarse level's last step; fallback rows stay current copies.
+// (lbm_collision_models.cpp:244-251): the row of a coarse node, in storage form, as an
+// interpolation stencil takes it: feq + tau_ratio (f - feq)
+template <int D, typename T, bool SHIFT>
+__device__ __forceinline__ void rescale_row(T *row, double tau_ratio, int compressible) {
+    constexpr int Q = Lattice<D>::Q;
+    if constexpr (SHIFT) {
+        // FP32 / BF16 storage: in FP32 on the stored deviations f - w, whose equilibrium
+        // feq - w needs no cancellation
+        float f[Q], rho, drho, u[3];
+        load_row<D>(row, 0, f);
+        macro<D, true, float>(f, nullptr, 0.f, 0, compressible, rho, drho, u);
+        const float usq = u[0] * u[0] + u[1] * u[1] + (D == 3 ? u[2] * u[2] : 0.f);
+        const float tr = (float)tau_ratio;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const float feq = feq_stored<D, true, float>(q, rho, drho, u[0], u[1], u[2], usq, compressible);
+            f[q] = __builtin_fmaf(tr, f[q] - feq, feq);
+        }
+        store_row<D>(row, 0, f);
+    } else {
+        double f[Q], feq[Q], rho, u[3];
+        load_row<D>(row, 0, f);
+        macro_feq_double<D>(f, compressible, rho, u, feq);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) f[q] = feq[q] + tau_ratio * (f[q] - feq[q]);
+        store_row<D>(row, 0, f);
+    }
+}
+
+// Time interpolation only: the rows of the interpolation as a table, [n_src + n_fb][S], the
+// rescaled coarse sources and then plain copies of the fine nodes that stand in for missing coarse
+// ones.  MID (after an odd fine substep): each coarse row is the mean of the row computed now and
+// the row `prev` of the last synchronised transfer, i.e. of the coarse state before and after the
+// coarse level's last step; fallback rows stay current copies.
 template <int D, typename T, bool SHIFT, bool MID>
 __global__ __launch_bounds__(256) void k_c2f_sources(int64_t n_src, int64_t n_fb, const int32_t *src_ai,
-                                                     const T *aux_c, int64_t naux_c, const int32_t *fb_ai,
-                                                     const T *aux_f, int64_t naux_f, double tau_ratio,
-                                                     int compressible, const T *__restrict__ prev, T *src_f) {
-    constexpr int Q = Lattice<D>::Q;
-    __shared__ T tile[256 * Q];   // row-major; the odd stride Q keeps the row writes conflict-free
-    const int64_t r0 = (int64_t)blockIdx.x * 256;
-    const int64_t r = r0 + threadIdx.x;
-    const int64_t n = n_src + n_fb;
+                                                     const T *aux_c, const int32_t *fb_ai, const T *aux_f,
+                                                     double tau_ratio, int compressible, const T *__restrict__ prev,
+                                                     T *src_f) {
+    constexpr int Q = Lattice<D>::Q, S = aux_stride<D>();
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (r >= n_src + n_fb) return;
+    RowUnit<T> unit[S / RowUnit<T>::n];
+    T *row = unit[0].v;
+    T v[Q];
+    load_row<D>(r < n_src ? aux_c : aux_f, r < n_src ? src_ai[r] : fb_ai[r - n_src], v);
+    store_row<D>(row, 0, v);
     if (r < n_src) {
-        const int64_t j = src_ai[r];
-        if constexpr (SHIFT) {
-            // FP32 / BF16 storage: in FP32 on the stored deviations f - w, whose equilibrium
-            // feq - w needs no cancellation
-            float f[Q], rho, drho, u[3];
+        rescale_row<D, T, SHIFT>(row, tau_ratio, compressible);
+        if constexpr (MID) {
+            T p[Q];
+            load_row<D>(prev, r, p);
 #pragma unroll
-            for (int q = 0; q < Q; ++q) f[q] = float(aux_c[q * naux_c + j]);
-            macro<D, true, float>(f, nullptr, 0.f, 0, compressible, rho, drho, u);
-            const float usq = u[0] * u[0] + u[1] * u[1] + (D == 3 ? u[2] * u[2] : 0.f);
-            const float tr = (float)tau_ratio;
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                const float feq = feq_stored<D, true, float>(q, rho, drho, u[0], u[1], u[2], usq, compressible);
-                tile[threadIdx.x * Q + q] = T(__builtin_fmaf(tr, f[q] - feq, feq));
-            }
-        } else {
-            double f[Q], feq[Q], rho, u[3];
-#pragma unroll
-            for (int q = 0; q < Q; ++q) f[q] = double(aux_c[q * naux_c + j]);
-            macro_feq_double<D>(f, compressible, rho, u, feq);
-#pragma unroll
-            for (int q = 0; q < Q; ++q) tile[threadIdx.x * Q + q] = T(feq[q] + tau_ratio * (f[q] - feq[q]));
+            for (int q = 0; q < Q; ++q) row[q] = T(0.5 * (double(p[q]) + double(row[q])));
         }
-    } else if (r < n) {
-        const int64_t fi = fb_ai[r - n_src];
-        T v[Q];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) v[q] = aux_f[q * naux_f + fi];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) tile[threadIdx.x * Q + q] = v[q];
     }
-    __syncthreads();
-    const int rows = (int)(n - r0 < 256 ? n - r0 : 256);
-    if constexpr (MID) {
-        // coarse rows [0, n_src) of this workgroup: elements below (n_src - r0) Q
-        const int64_t nc = (n_src - r0) * Q;
-        for (int e = threadIdx.x; e < rows * Q; e += 256)
-            src_f[r0 * Q + e] = e < nc ? T(0.5 * (double(prev[r0 * Q + e]) + double(tile[e]))) : tile[e];
-    } else {
-        for (int e = threadIdx.x; e < rows * Q; e += 256) src_f[r0 * Q + e] = tile[e];
-    }
+    load_row<D>(row, 0, v);
+    store_row<D>(src_f, r, v);
 }
 
 // InterpolationLagrangian{2D,3D} (grid/grid_interpolation.cpp:224-304, 433-525): each ghost node
@@ -100,28 +97,44 @@ __global__ __launch_bounds__(256) void k_c2f_sources(int64_t n_src, int64_t n_fb
 // coordinate, 1 per even one), stably, so the threads of a wavefront loop equally often; inside
 // one count they keep Morton order, so the nodes of a workgroup are neighbours.  A
 // workgroup takes a group of at most 256 / PARTS ghost nodes, as many as keep its staged data
-// within the LDS budget: it first copies the union of their rows of src_f and their contributor
-// words into LDS, then each ghost node is summed from LDS by PARTS threads of 5 directions (D2Q9:
-// 5 and 4).  A contributor is one 32-bit word {LDS row offset, FP16 weight}: the tensor-product
+// within the LDS budget: it first copies the union of their rows and their contributor words into
+// LDS, then each ghost node is summed from LDS by PARTS threads of 5 directions (D2Q9: 5 and 4).
+// DIRECT: a staged row is an aux row, of the coarse level (index >= 0; rescaled in LDS, one thread
+// a row) or of the fine level (~index: a fallback node); rows that several groups stage are
+// rescaled by each, a few hundred operations against a launch over all rows (4.8 us on small
+// levels, 10.8 on a 3M-node one) and their round trip through memory.  Otherwise (time
+// interpolation) a row of the table src_f.  A contributor is one 32-bit word {LDS row offset, FP16 weight}: the tensor-product
 // Lagrange weights are products of -1/16, 9/16, 1/2 and 1, dyadic rationals exact in FP16 (the
 // host checks every one).
 constexpr int kGatherDirs = 5;
 constexpr size_t kGatherLdsBudget = 20 * 1024;
 constexpr int kGatherMaxRows = 768;   // staged rows of one group (row offsets fit the word's 16 bits)
 constexpr int64_t kGatherChunk = 2048;   // ghost nodes sorted by contributor count together
-template <int D, typename T, bool SHIFT>
-__device__ __forceinline__ void gather_group(int64_t gi, unsigned char *lds_raw, const GatherGroup *__restrict__ groups,
-                                             const int32_t *__restrict__ tgt_ai, const int32_t *__restrict__ begin,
-                                             const uint32_t *__restrict__ contrib, const int32_t *__restrict__ rows,
-                                             const T *__restrict__ src_f, T *__restrict__ aux_f, int64_t naux) {
+// what a gather reads: the staged rows' indices and the arrays they name, the fine level's aux rows
+template <typename T>
+struct GatherArgs {
+    const GatherGroup *groups;
+    const int32_t *tgt_ai, *begin;
+    const uint32_t *contrib;
+    const int32_t *rows;      // DIRECT: aux rows; else rows of src_f
+    const T *src_f;           // DIRECT: the coarse level's aux rows; else the table
+    T *aux_f;
+    double tau_ratio;
+    int compressible;
+};
+
+template <int D, typename T, bool SHIFT, bool DIRECT>
+__device__ __forceinline__ void gather_group(int64_t gi, unsigned char *lds_raw, const GatherArgs<T> &a) {
     constexpr int Q = Lattice<D>::Q;
     constexpr int NQ = kGatherDirs;
     constexpr int PARTS = (Q + NQ - 1) / NQ;
-    constexpr int QP = PARTS * NQ;   // LDS row stride: every thread reads NQ entries, pads included
-    const GatherGroup G = groups[gi];
+    constexpr int S = aux_stride<D>();
+    static_assert(PARTS * NQ <= S, "every thread reads NQ entries of a row, pads included");
+    const GatherGroup G = a.groups[gi];
+    T *__restrict__ aux_f = a.aux_f;
     const int32_t nr = G.r1 - G.r0, nc = G.c1 - G.c0;
-    T *rowbuf = reinterpret_cast<T *>(lds_raw);                                  // [nr][QP]
-    uint32_t *cbuf = reinterpret_cast<uint32_t *>(lds_raw + (((size_t)nr * QP * sizeof(T) + 15) & ~(size_t)15));
+    T *rowbuf = reinterpret_cast<T *>(lds_raw);                                  // [nr][S]
+    uint32_t *cbuf = reinterpret_cast<uint32_t *>(lds_raw + (((size_t)nr * S * sizeof(T) + 15) & ~(size_t)15));
     const int local = threadIdx.x / PARTS;
     const int q0 = (threadIdx.x - local * PARTS) * NQ;
     const int32_t t = G.t0 + local;
@@ -130,16 +143,16 @@ __device__ __forceinline__ void gather_group(int64_t gi, unsigned char *lds_raw,
     // an earlier one except a row's data on its entry
     int32_t kb = 0, ke = 0, ai = 0;
     if (active) {
-        kb = begin[t] - G.c0;
-        ke = begin[t + 1] - G.c0;
-        ai = tgt_ai[t];
+        kb = a.begin[t] - G.c0;
+        ke = a.begin[t + 1] - G.c0;
+        ai = a.tgt_ai[t];
     }
     for (int cb = 0; cb < nc; cb += 4 * 256) {
         uint32_t w[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int k = cb + j * 256 + (int)threadIdx.x;
-            w[j] = k < nc ? contrib[G.c0 + k] : 0u;
+            w[j] = k < nc ? a.contrib[G.c0 + k] : 0u;
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -147,32 +160,36 @@ __device__ __forceinline__ void gather_group(int64_t gi, unsigned char *lds_raw,
             if (k < nc) cbuf[k] = w[j];
         }
     }
-    // the rows as one flat run of nr * Q elements, consecutive threads on consecutive elements,
-    // so a wavefront's load covers a few cache lines of src_f instead of 64
-    constexpr int kBatch = 8;
-    const int ne = nr * Q;
-    for (int eb = 0; eb < ne; eb += kBatch * 256) {
+    // the rows in units of 16 bytes (8 in BF16), consecutive threads on consecutive units
+    constexpr int U = S / RowUnit<T>::n, kBatch = 4;
+    const int nu = nr * U;
+    RowUnit<T> *units = reinterpret_cast<RowUnit<T> *>(rowbuf);
+    for (int ub = 0; ub < nu; ub += kBatch * 256) {
         int32_t g[kBatch];
-        T v[kBatch];
+        RowUnit<T> v[kBatch];
 #pragma unroll
         for (int j = 0; j < kBatch; ++j) {
-            const int e = eb + j * 256 + (int)threadIdx.x;
-            g[j] = rows[G.r0 + (e < ne ? e : ne - 1) / Q];
+            const int e = ub + j * 256 + (int)threadIdx.x;
+            g[j] = a.rows[G.r0 + (e < nu ? e : nu - 1) / U];
         }
 #pragma unroll
         for (int j = 0; j < kBatch; ++j) {
-            const int e = eb + j * 256 + (int)threadIdx.x;
-            const int ec = e < ne ? e : ne - 1;
-            v[j] = src_f[(int64_t)g[j] * Q + (ec - (ec / Q) * Q)];
+            const int e = ub + j * 256 + (int)threadIdx.x;
+            const int ec = e < nu ? e : nu - 1;
+            const T *base = DIRECT && g[j] < 0 ? aux_f : a.src_f;
+            const int64_t row = DIRECT && g[j] < 0 ? ~g[j] : g[j];
+            v[j] = reinterpret_cast<const RowUnit<T> *>(base)[row * U + (ec - (ec / U) * U)];
         }
 #pragma unroll
         for (int j = 0; j < kBatch; ++j) {
-            const int e = eb + j * 256 + (int)threadIdx.x;
-            if (e < ne) {
-                const int r = e / Q;
-                rowbuf[r * QP + (e - r * Q)] = v[j];
-            }
+            const int e = ub + j * 256 + (int)threadIdx.x;
+            if (e < nu) units[e] = v[j];
         }
+    }
+    if constexpr (DIRECT) {
+        __syncthreads();
+        for (int r = threadIdx.x; r < nr; r += 256)
+            if (a.rows[G.r0 + r] >= 0) rescale_row<D, T, SHIFT>(rowbuf + r * S, a.tau_ratio, a.compressible);
     }
     __syncthreads();
     if (!active) return;
@@ -183,11 +200,11 @@ __device__ __forceinline__ void gather_group(int64_t gi, unsigned char *lds_raw,
 #pragma unroll
     for (int i = 0; i < NQ; ++i) acc[i] = 0.;
     if constexpr (SHIFT) {
-        // FP32 / BF16 storage holds f - w.  sum c (f~ + w) - w = sum c f~ + w (S - 1) with S =
-        // sum c: the weights are multiples of 2^-12 of magnitude <= 1, so S is exact in FP32.
+        // FP32 / BF16 storage holds f - w.  sum c (f~ + w) - w = sum c f~ + w (sum c - 1): the
+        // weights are multiples of 2^-12 of magnitude <= 1, so their sum is exact in FP32.
         // Runs of four products are summed in FP32 (rounding error a few 2^-24 of the run), the
         // runs in FP64.
-        float S = 0.f;
+        float sum = 0.f;
         int32_t k = kb;
         for (; k + 4 <= ke; k += 4) {
             float c[4];
@@ -198,7 +215,7 @@ __device__ __forceinline__ void gather_group(int64_t gi, unsigned char *lds_raw,
                 c[j] = weight(cw);
                 row[j] = rowbuf + (cw & 0xffffu) + q0;
             }
-            S += (c[0] + c[1]) + (c[2] + c[3]);
+            sum += (c[0] + c[1]) + (c[2] + c[3]);
 #pragma unroll
             for (int i = 0; i < NQ; ++i) {
                 float run = c[0] * float(row[0][i]);
@@ -212,13 +229,13 @@ __device__ __forceinline__ void gather_group(int64_t gi, unsigned char *lds_raw,
             const uint32_t cw = cbuf[k];
             const float c = weight(cw);
             const T *row = rowbuf + (cw & 0xffffu) + q0;
-            S += c;
+            sum += c;
 #pragma unroll
             for (int i = 0; i < NQ; ++i) acc[i] += (double)(c * float(row[i]));
         }
 #pragma unroll
         for (int i = 0; i < NQ; ++i)
-            if (q0 + i < Q) aux_f[(q0 + i) * naux + ai] = T(acc[i] + Lattice<D>::w[q0 + i] * ((double)S - 1.));
+            if (q0 + i < Q) aux_f[(int64_t)ai * S + q0 + i] = T(acc[i] + Lattice<D>::w[q0 + i] * ((double)sum - 1.));
     } else {
         // FP64 storage: every product and sum in FP64, in stencil order
 #pragma unroll 4
@@ -231,102 +248,100 @@ __device__ __forceinline__ void gather_group(int64_t gi, unsigned char *lds_raw,
         }
 #pragma unroll
         for (int i = 0; i < NQ; ++i)
-            if (q0 + i < Q) aux_f[(q0 + i) * naux + ai] = T(acc[i]);
+            if (q0 + i < Q) aux_f[(int64_t)ai * S + q0 + i] = T(acc[i]);
     }
 }
 
-template <int D, typename T, bool SHIFT>
-__global__ __launch_bounds__(256) void k_c2f_gather(int64_t n_groups, const GatherGroup *__restrict__ groups,
-                                                    const int32_t *__restrict__ tgt_ai,
-                                                    const int32_t *__restrict__ begin,
-                                                    const uint32_t *__restrict__ contrib,
-                                                    const int32_t *__restrict__ rows, const T *__restrict__ src_f,
-                                                    T *__restrict__ aux_f, int64_t naux) {
-    extern __shared__ unsigned char lds_raw[];
+template <int D, typename T, bool SHIFT, bool DIRECT>
+__global__ __launch_bounds__(256) void k_c2f_gather(int64_t n_groups, GatherArgs<T> a) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
     const int64_t gi = xcd_group(n_groups);   // groups are in spatial order: an XCD takes a range
     if (gi < 0) return;
-    gather_group<D, T, SHIFT>(gi, lds_raw, groups, tgt_ai, begin, contrib, rows, src_f, aux_f, naux);
+    gather_group<D, T, SHIFT, DIRECT>(gi, lds_raw, a);
 }
 
 // NodeInfoFine2Coarse (lbm_grid_interface.cpp:594-610) + PostStreamFine2Coarse
 // (lbm_collision_models.cpp:259-267): rho, u of the fine node's last collision
+template <typename T>
+struct F2cArgs {
+    int64_t n;
+    const int32_t *coarse_ai, *fine_ai;
+    const T *fine_f;
+    const double *fine_macro;
+    double tau_ratio;
+    int compressible;
+    T *coarse_f;
+};
+
 template <int D, typename T, bool SHIFT>
-__device__ __forceinline__ void f2c_node(int64_t p, const int32_t *coarse_ai, const int32_t *fine_ai, const T *fine_f,
-                                         int64_t naux_f, const double *fine_macro, double tau_ratio, int compressible,
-                                         T *coarse_f, int64_t naux_c) {
+__device__ __forceinline__ void f2c_node(int64_t p, const F2cArgs<T> &a) {
     using L = Lattice<D>;
     constexpr int Q = L::Q;
-    const int64_t i = fine_ai[p], j = coarse_ai[p];
+    const int64_t i = a.fine_ai[p], j = a.coarse_ai[p];
     if constexpr (SHIFT) {
         // FP32 / BF16 storage: in FP32 on the stored deviations f - w
-        const float rho = (float)fine_macro[i * 4], ux = (float)fine_macro[i * 4 + 1];
-        const float uy = (float)fine_macro[i * 4 + 2], uz = D == 3 ? (float)fine_macro[i * 4 + 3] : 0.f;
-        const float drho = (float)(fine_macro[i * 4] - 1.);
+        float f[Q];
+        load_row<D>(a.fine_f, i, f);
+        const float rho = (float)a.fine_macro[i * 4], ux = (float)a.fine_macro[i * 4 + 1];
+        const float uy = (float)a.fine_macro[i * 4 + 2], uz = D == 3 ? (float)a.fine_macro[i * 4 + 3] : 0.f;
+        const float drho = (float)(a.fine_macro[i * 4] - 1.);
         const float usq = ux * ux + uy * uy + (D == 3 ? uz * uz : 0.f);
-        const float tr = (float)tau_ratio;
+        const float tr = (float)a.tau_ratio;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            const float feq = feq_stored<D, true, float>(q, rho, drho, ux, uy, uz, usq, compressible);
-            coarse_f[q * naux_c + j] = T(__builtin_fmaf(tr, float(fine_f[q * naux_f + i]) - feq, feq));
+            const float feq = feq_stored<D, true, float>(q, rho, drho, ux, uy, uz, usq, a.compressible);
+            f[q] = __builtin_fmaf(tr, f[q] - feq, feq);
         }
+        store_row<D>(a.coarse_f, j, f);
         return;
     }
-    const double rho = fine_macro[i * 4], ux = fine_macro[i * 4 + 1], uy = fine_macro[i * 4 + 2];
-    const double uz = D == 3 ? fine_macro[i * 4 + 3] : 0.;
+    double f[Q];
+    load_row<D>(a.fine_f, i, f);
+    const double rho = a.fine_macro[i * 4], ux = a.fine_macro[i * 4 + 1], uy = a.fine_macro[i * 4 + 2];
+    const double uz = D == 3 ? a.fine_macro[i * 4 + 3] : 0.;
     const double usq = ux * ux + uy * uy + (D == 3 ? uz * uz : 0.);
+#pragma unroll
     for (int q = 0; q < Q; ++q) {
         double cu = ux * L::cx[q] + uy * L::cy[q];
         if (D == 3) cu += uz * L::cz[q];
-        const double feq = compressible ? L::w[q] * rho * (1. + 3. * cu + 4.5 * cu * cu - 1.5 * usq)
-                                        : L::w[q] * (rho + 3. * cu + 4.5 * cu * cu - 1.5 * usq);
-        const double ff = double(fine_f[q * naux_f + i]) + (SHIFT ? L::w[q] : 0.);
-        coarse_f[q * naux_c + j] = T(feq + tau_ratio * (ff - feq) - (SHIFT ? L::w[q] : 0.));
+        const double feq = a.compressible ? L::w[q] * rho * (1. + 3. * cu + 4.5 * cu * cu - 1.5 * usq)
+                                          : L::w[q] * (rho + 3. * cu + 4.5 * cu * cu - 1.5 * usq);
+        f[q] = feq + a.tau_ratio * (f[q] - feq);
     }
+    store_row<D>(a.coarse_f, j, f);
 }
 
 template <int D, typename T, bool SHIFT>
-__global__ void k_f2c(int64_t n, const int32_t *coarse_ai, const int32_t *fine_ai, const T *fine_f, int64_t naux_f,
-                      const double *fine_macro, double tau_ratio, int compressible, T *coarse_f, int64_t naux_c) {
+__global__ void k_f2c(F2cArgs<T> a) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    f2c_node<D, T, SHIFT>(p, coarse_ai, fine_ai, fine_f, naux_f, fine_macro, tau_ratio, compressible, coarse_f, naux_c);
+    if (p < a.n) f2c_node<D, T, SHIFT>(p, a);
 }
 
 // The gather and the fine-to-coarse copy of one exchange in one launch, where the host found
-// them independent (no fine node is both a gather target and a fine-to-coarse source; the
-// coarse-to-fine source rows are taken before either): blocks below nb_gather (a multiple of 8)
+// them independent (no fine node is both a gather target and a fine-to-coarse source, no coarse
+// node both a staged source and a fine-to-coarse target): blocks below nb_gather (a multiple of 8)
 // are the gather's, in its XCD-aware order; the blocks after them take 256 fine-to-coarse nodes
 // each.
-template <int D, typename T, bool SHIFT>
-__global__ __launch_bounds__(256) void k_c2f_gather_f2c(int64_t nb_gather, int64_t n_groups,
-                                                        const GatherGroup *__restrict__ groups,
-                                                        const int32_t *__restrict__ tgt_ai,
-                                                        const int32_t *__restrict__ begin,
-                                                        const uint32_t *__restrict__ contrib,
-                                                        const int32_t *__restrict__ rows, const T *__restrict__ src_f,
-                                                        T *__restrict__ aux_f, int64_t naux, int64_t n_f2c,
-                                                        const int32_t *coarse_ai, const int32_t *fine_ai,
-                                                        const double *fine_macro, double tau_ratio, int compressible,
-                                                        T *coarse_f, int64_t naux_c) {
-    extern __shared__ unsigned char lds_raw[];
+template <int D, typename T, bool SHIFT, bool DIRECT>
+__global__ __launch_bounds__(256) void k_c2f_gather_f2c(int64_t nb_gather, int64_t n_groups, GatherArgs<T> g,
+                                                        F2cArgs<T> c) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
     const int64_t bid = blockIdx.x;
     if (bid < nb_gather) {
         const int64_t per = nb_gather >> 3;
         const int64_t gi = (bid & 7) * per + (bid >> 3);
         if (gi >= n_groups) return;
-        gather_group<D, T, SHIFT>(gi, lds_raw, groups, tgt_ai, begin, contrib, rows, src_f, aux_f, naux);
+        gather_group<D, T, SHIFT, DIRECT>(gi, lds_raw, g);
     } else {
         const int64_t p = (bid - nb_gather) * 256 + threadIdx.x;
-        if (p < n_f2c)
-            f2c_node<D, T, SHIFT>(p, coarse_ai, fine_ai, aux_f, naux, fine_macro, tau_ratio, compressible, coarse_f,
-                                  naux_c);
+        if (p < c.n) f2c_node<D, T, SHIFT>(p, c);
     }
 }
 
 // immersed boundary, step 1: zero the force of every supported node and recompute its velocity
 // with the remaining (constant) force (the lazy reset, immersed_boundary.cpp:76-85, 284-296)
 template <int D, typename T, typename C, bool SHIFT>
-__global__ void k_ib_reset(int64_t n, const int32_t *reset_ai, const T *aux_f, int64_t naux, double *aux_force,
+__global__ void k_ib_reset(int64_t n, const int32_t *reset_ai, const T *aux_f, double *aux_force,
                            double *node_u, StepParams p) {
     constexpr int Q = Lattice<D>::Q;
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -336,7 +351,7 @@ __global__ void k_ib_reset(int64_t n, const int32_t *reset_ai, const T *aux_f, i
     aux_force[ai * 3 + 1] = 0.;
     aux_force[ai * 3 + 2] = 0.;
     C f[Q];
-    for (int q = 0; q < Q; ++q) f[q] = C(aux_f[q * naux + ai]);
+    load_row<D>(aux_f, ai, f);
     C F[3] = {C(p.const_force[0]), C(p.const_force[1]), C(p.const_force[2])};
     C rho, drho, u[3];
     macro<D, SHIFT, C>(f, F, C(p.dt), 1, p.compressible, rho, drho, u);
@@ -712,6 +727,17 @@ inline bool exact_half_bits(double w, uint16_t *bits) {
     return true;
 }
 
+// the row tables of time interpolation (when it is switched on after the build: by the rows computed
+// then, before any step)
+inline zlh_status reserve_row_tables(zlh_ctx *ctx, TransferTables &X) {
+    const int64_t stride = ctx->d.dims == 2 ? aux_stride<2>() : aux_stride<3>();
+    const size_t bytes = ctx->tsize() * stride * std::max<int64_t>(X.n_src + X.n_fb, 1);
+    zlh_status s;
+    if (!X.src_f.p && (s = dalloc(ctx, X.src_f, bytes))) return s;
+    if (!X.src_mid.p && (s = dalloc(ctx, X.src_mid, bytes))) return s;
+    return ZLH_OK;
+}
+
 inline zlh_status upload_transfer(zlh_ctx *ctx, int level) {
     LevelState &F = ctx->lv[level], &C = ctx->lv[level - 1];
     TransferPlan &P = F.xplan;
@@ -754,7 +780,8 @@ inline zlh_status upload_transfer(zlh_ctx *ctx, int level) {
     // kGatherChunk; inside a chunk by descending contributor count, then aux index.  A group
     // closes at 256 / PARTS nodes or when its rows and contributor words would pass the budget
     const int Qn = ctx->q;
-    const int parts = (Qn + kGatherDirs - 1) / kGatherDirs, row_stride = parts * kGatherDirs;
+    const int parts = (Qn + kGatherDirs - 1) / kGatherDirs;
+    const int row_stride = ctx->d.dims == 2 ? aux_stride<2>() : aux_stride<3>();
     const size_t lds_budget = kGatherLdsBudget, row_bytes = (size_t)row_stride * ctx->tsize();
     const int group_max = 256 / parts;
     const int64_t nt = (int64_t)tgt.size();
@@ -828,11 +855,21 @@ inline zlh_status upload_transfer(zlh_ctx *ctx, int level) {
     if ((s = upload(ctx, X.c2f_begin, begin2))) return s;
     if ((s = upload(ctx, X.groups, groups))) return s;
     if ((s = upload(ctx, X.group_rows, group_rows))) return s;
+    {
+        // the aux rows of the same entries: coarse, or ~fine
+        std::vector<int32_t> aux_rows(group_rows.size());
+        for (size_t k = 0; k < group_rows.size(); ++k) {
+            const size_t g = (size_t)group_rows[k];
+            aux_rows[k] = g < src_ai.size() ? src_ai[g] : ~fb_ai[g - src_ai.size()];
+        }
+        if ((s = upload(ctx, X.group_aux, aux_rows))) return s;
+    }
     if ((s = upload(ctx, X.c2f_contrib, packed))) return s;
     if ((s = upload(ctx, X.src_coarse_ai, src_ai))) return s;
     if ((s = upload(ctx, X.fb_fine_ai, fb_ai))) return s;
-    if ((s = dalloc(ctx, X.src_f, ctx->tsize() * ctx->q * std::max<int64_t>(X.n_src + X.n_fb, 1)))) return s;
-    if ((s = dalloc(ctx, X.src_mid, ctx->tsize() * ctx->q * std::max<int64_t>(X.n_src + X.n_fb, 1)))) return s;
+    X.src_f = DevBuf();
+    X.src_mid = DevBuf();
+    if (ctx->time_interp && (s = reserve_row_tables(ctx, X))) return s;
     if ((s = upload(ctx, X.f2c_coarse_ai, f2c_c))) return s;
     if ((s = upload(ctx, X.f2c_fine_ai, f2c_f))) return s;
     {
@@ -842,6 +879,11 @@ inline zlh_status upload_transfer(zlh_ctx *ctx, int level) {
         std::vector<int32_t> common;
         std::set_intersection(a.begin(), a.end(), b.begin(), b.end(), std::back_inserter(common));
         X.f2c_apart = common.empty();
+        std::vector<int32_t> c(f2c_c.begin(), f2c_c.end());
+        std::sort(c.begin(), c.end());
+        common.clear();
+        std::set_intersection(src_ai.begin(), src_ai.end(), c.begin(), c.end(), std::back_inserter(common));
+        X.f2c_apart &= common.empty();
     }
     F.xfer_writes = tgt;
     F.xfer_reads = fb_ai;
@@ -947,43 +989,51 @@ zlh_status launch_transfers_t(zlh_ctx *ctx, int level, int parts) {
     const double dtc = 1. / (double)(1u << (level - 1)), dtf = 1. / (double)(1u << level);
     const double c2f = 0.5 * (nu * 3. / dtc * 2. + 0.5) / (nu * 3. / dtc + 0.5);
     const double f2c = 2. * (nu * 3. / dtf / 2 + 0.5) / (nu * 3. / dtf + 0.5);
-    if ((parts & (kTransferC2F | kTransferRows)) && X.n_c2f > 0) {
-        const bool mid = (parts & kTransferMid) != 0;
-        T *rows = mid ? X.src_mid.as<T>() : X.src_f.as<T>();
-        if (X.n_src + X.n_fb > 0) {
-            if (mid)
-                hipLaunchKernelGGL((k_c2f_sources<D, T, SHIFT, true>), dim3(blocks(X.n_src + X.n_fb)),
-                                   dim3(256), 0, ctx->stream, X.n_src, X.n_fb, X.src_coarse_ai.as<int32_t>(),
-                                   C.aux_f_d.as<T>(), C.naux, X.fb_fine_ai.as<int32_t>(), F.aux_f_d.as<T>(), F.naux,
-                                   c2f, comp, X.src_f.as<T>(), rows);
-            else
-                hipLaunchKernelGGL((k_c2f_sources<D, T, SHIFT, false>), dim3(blocks(X.n_src + X.n_fb)),
-                                   dim3(256), 0, ctx->stream, X.n_src, X.n_fb, X.src_coarse_ai.as<int32_t>(),
-                                   C.aux_f_d.as<T>(), C.naux, X.fb_fine_ai.as<int32_t>(), F.aux_f_d.as<T>(), F.naux,
-                                   c2f, comp, nullptr, rows);
-        }
-        const int64_t nb_gather = (X.n_groups + 7) / 8 * 8;
-        if ((parts & kTransferC2F) && (parts & kTransferF2C) && X.n_f2c > 0 && X.f2c_apart) {
-            // one launch for both halves (independent: see k_c2f_gather_f2c)
-            hipLaunchKernelGGL((k_c2f_gather_f2c<D, T, SHIFT>), dim3((unsigned)(nb_gather + blocks(X.n_f2c))), dim3(256),
-                               X.lds_bytes, ctx->stream, nb_gather, X.n_groups, X.groups.as<GatherGroup>(),
-                               X.c2f_target.as<int32_t>(), X.c2f_begin.as<int32_t>(), X.c2f_contrib.as<uint32_t>(),
-                               X.group_rows.as<int32_t>(), rows, F.aux_f_d.as<T>(), F.naux, X.n_f2c,
-                               X.f2c_coarse_ai.as<int32_t>(), X.f2c_fine_ai.as<int32_t>(), F.aux_macro_d.as<double>(),
-                               f2c, comp, C.aux_f_d.as<T>(), C.naux);
-            ZLH_TRY(hipGetLastError());
-            return ZLH_OK;
-        }
-        if (parts & kTransferC2F)
-            hipLaunchKernelGGL((k_c2f_gather<D, T, SHIFT>), dim3((unsigned)nb_gather), dim3(256),
-                               X.lds_bytes, ctx->stream, X.n_groups, X.groups.as<GatherGroup>(),
-                               X.c2f_target.as<int32_t>(), X.c2f_begin.as<int32_t>(), X.c2f_contrib.as<uint32_t>(),
-                               X.group_rows.as<int32_t>(), rows, F.aux_f_d.as<T>(), F.naux);
+    // with time interpolation the rows go through a table, which keeps the earlier ones
+    const bool table = ctx->time_interp;
+    const bool mid = (parts & kTransferMid) != 0;
+    if (table && (parts & (kTransferC2F | kTransferRows)) && X.n_src + X.n_fb > 0) {
+        const zlh_status s = reserve_row_tables(ctx, X);
+        if (s) return s;
+        const dim3 grid(blocks(X.n_src + X.n_fb));
+        if (mid)
+            hipLaunchKernelGGL((k_c2f_sources<D, T, SHIFT, true>), grid, dim3(256), 0, ctx->stream, X.n_src, X.n_fb,
+                               X.src_coarse_ai.as<int32_t>(), C.aux_f_d.as<T>(), X.fb_fine_ai.as<int32_t>(),
+                               F.aux_f_d.as<T>(), c2f, comp, X.src_f.as<T>(), X.src_mid.as<T>());
+        else
+            hipLaunchKernelGGL((k_c2f_sources<D, T, SHIFT, false>), grid, dim3(256), 0, ctx->stream, X.n_src, X.n_fb,
+                               X.src_coarse_ai.as<int32_t>(), C.aux_f_d.as<T>(), X.fb_fine_ai.as<int32_t>(),
+                               F.aux_f_d.as<T>(), c2f, comp, nullptr, X.src_f.as<T>());
     }
-    if ((parts & kTransferF2C) && X.n_f2c > 0)
-        hipLaunchKernelGGL((k_f2c<D, T, SHIFT>), dim3(blocks(X.n_f2c)), dim3(256), 0, ctx->stream, X.n_f2c,
-                           X.f2c_coarse_ai.as<int32_t>(), X.f2c_fine_ai.as<int32_t>(), F.aux_f_d.as<T>(), F.naux,
-                           F.aux_macro_d.as<double>(), f2c, comp, C.aux_f_d.as<T>(), C.naux);
+    const F2cArgs<T> fc{X.n_f2c, X.f2c_coarse_ai.as<int32_t>(), X.f2c_fine_ai.as<int32_t>(), F.aux_f_d.as<T>(),
+                        F.aux_macro_d.as<double>(), f2c, comp, C.aux_f_d.as<T>()};
+    bool copied = false;
+    if ((parts & kTransferC2F) && X.n_c2f > 0) {
+        const GatherArgs<T> ga{X.groups.as<GatherGroup>(), X.c2f_target.as<int32_t>(), X.c2f_begin.as<int32_t>(),
+                               X.c2f_contrib.as<uint32_t>(), table ? X.group_rows.as<int32_t>() : X.group_aux.as<int32_t>(),
+                               table ? (mid ? X.src_mid.as<T>() : X.src_f.as<T>()) : C.aux_f_d.as<T>(), F.aux_f_d.as<T>(),
+                               c2f, comp};
+        const int64_t nb_gather = (X.n_groups + 7) / 8 * 8;
+        if ((parts & kTransferF2C) && X.n_f2c > 0 && X.f2c_apart) {
+            // one launch for both halves (independent: see k_c2f_gather_f2c)
+            const dim3 grid((unsigned)(nb_gather + blocks(X.n_f2c)));
+            if (table)
+                hipLaunchKernelGGL((k_c2f_gather_f2c<D, T, SHIFT, false>), grid, dim3(256), X.lds_bytes, ctx->stream,
+                                   nb_gather, X.n_groups, ga, fc);
+            else
+                hipLaunchKernelGGL((k_c2f_gather_f2c<D, T, SHIFT, true>), grid, dim3(256), X.lds_bytes, ctx->stream,
+                                   nb_gather, X.n_groups, ga, fc);
+            copied = true;
+        } else if (table) {
+            hipLaunchKernelGGL((k_c2f_gather<D, T, SHIFT, false>), dim3((unsigned)nb_gather), dim3(256), X.lds_bytes,
+                               ctx->stream, X.n_groups, ga);
+        } else {
+            hipLaunchKernelGGL((k_c2f_gather<D, T, SHIFT, true>), dim3((unsigned)nb_gather), dim3(256), X.lds_bytes,
+                               ctx->stream, X.n_groups, ga);
+        }
+    }
+    if ((parts & kTransferF2C) && X.n_f2c > 0 && !copied)
+        hipLaunchKernelGGL((k_f2c<D, T, SHIFT>), dim3(blocks(X.n_f2c)), dim3(256), 0, ctx->stream, fc);
     ZLH_TRY(hipGetLastError());
     return ZLH_OK;
 }
@@ -1003,7 +1053,7 @@ zlh_status launch_ib_t(zlh_ctx *ctx, int level) {
     LevelState &L = ctx->lv[level];
     IbTables &B = L.ibt;
     hipLaunchKernelGGL((k_ib_reset<D, T, Cc, SHIFT>), dim3(blocks(B.n_reset)), dim3(256), 0, ctx->stream, B.n_reset,
-                       B.reset_ai.as<int32_t>(), L.aux_f_d.as<T>(), L.naux, L.aux_force_d.as<double>(),
+                       B.reset_ai.as<int32_t>(), L.aux_f_d.as<T>(), L.aux_force_d.as<double>(),
                        B.node_u.as<double>(), L.sp);
     hipLaunchKernelGGL((k_ib_markers<D>), dim3(blocks(B.n_markers * 64)), dim3(256), 0, ctx->stream, B.n_markers,
                        B.support, B.node_ai.as<int32_t>(), B.weight.as<double>(), B.node_u.as<double>(),

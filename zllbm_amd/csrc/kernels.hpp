@@ -54,6 +54,13 @@ __host__ __device__ __forceinline__ int64_t pop_at(int q, int64_t slot) {
     return ((slot >> 6) * Q + q) * 64 + (slot & 63);
 }
 
+// Populations of the aux nodes are node-major, [naux][S] with S = 20 (D3Q19) or 12 (D2Q9): a node's
+// row is whole 16-byte units (8 in BF16), so that the kernels that take a node at a time (aux
+// collision, exchange, forcing) move it in 5 (3) vector accesses instead of 19 (9) and the
+// interpolation stages rows as they are.  The pads hold anything.
+template <int D>
+__host__ __device__ constexpr int aux_stride() { return D == 3 ? 20 : 12; }
+
 // Storage form of ZLH_BF16_SHIFTED: f - w in bfloat16, converted to and from float with
 // round-to-nearest-even (v_cvt_pk_bf16_f32).
 typedef __bf16 bf16_t;
@@ -94,6 +101,39 @@ __device__ __forceinline__ T wall_value(const double2 *wall, int face, int q, T 
     return T(__builtin_fma(-k.x, k.y, double(v)));
 }
 
+// 16 bytes (8 in BF16) of an aux row
+template <typename T>
+struct alignas(sizeof(T) == 2 ? 8 : 16) RowUnit {
+    static constexpr int n = sizeof(T) == 8 ? 2 : 4;
+    T v[n];
+};
+
+template <int D, typename T, typename C>
+__device__ __forceinline__ void load_row(const T *__restrict__ aux_f, int64_t ai, C (&f)[Lattice<D>::Q]) {
+    constexpr int N = RowUnit<T>::n, U = aux_stride<D>() / N;
+    const RowUnit<T> *row = reinterpret_cast<const RowUnit<T> *>(aux_f + ai * aux_stride<D>());
+    RowUnit<T> r[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+        if (k * N < Lattice<D>::Q) r[k] = row[k];
+#pragma unroll
+    for (int q = 0; q < Lattice<D>::Q; ++q) f[q] = C(r[q / N].v[q % N]);
+}
+
+template <int D, typename T, typename C>
+__device__ __forceinline__ void store_row(T *__restrict__ aux_f, int64_t ai, const C (&f)[Lattice<D>::Q]) {
+    constexpr int N = RowUnit<T>::n, U = aux_stride<D>() / N;
+    RowUnit<T> *row = reinterpret_cast<RowUnit<T> *>(aux_f + ai * aux_stride<D>());
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+        if (k * N >= Lattice<D>::Q) continue;
+        RowUnit<T> r;
+#pragma unroll
+        for (int j = 0; j < N; ++j) r.v[j] = k * N + j < Lattice<D>::Q ? T(f[k * N + j < Lattice<D>::Q ? k * N + j : 0]) : T(0);
+        row[k] = r;
+    }
+}
+
 template <typename T>
 struct BrickLevel {
     int64_t nbrick;
@@ -104,7 +144,7 @@ struct BrickLevel {
     const uint64_t *auxmask;  // [nbrick] nodes whose post-stream values go to the aux array
     const uint64_t *defmask;  // [nbrick] of those, the nodes whose collision waits for the aux collision
     const int32_t *auxbase;   // [nbrick]
-    const uint32_t *aux_missing;  // [naux]
+    const uint32_t *aux_missing;  // [naux] the node's absent sources << 6 | its lane
     const int32_t *aux_slot;  // [naux]
     BoundaryPull bnd;         // brick null: no resolved boundary nodes
 };
@@ -497,7 +537,7 @@ struct FusedRun {
 // rho and u of the nodes flagged in macro_flag
 template <typename T>
 struct AuxRun {
-    int64_t naux, nlist;
+    int64_t nlist;
     const int32_t *list, *aux_slot;
     const T *aux_f;
     const double *aux_force;
@@ -618,7 +658,7 @@ __device__ __forceinline__ void stream_collide_brick(const BrickLevel<T> &lv, co
     uint32_t missing = 0;
     if (is_aux) {
         ai = base + __popcll(am & ((1ull << lane) - 1ull));
-        missing = lv.aux_missing[ai];
+        missing = lv.aux_missing[ai] >> 6;
     }
     C f[Q];
     // elements of fin to pull, then every load, then what no load gives: a branch or a use
@@ -651,11 +691,10 @@ __device__ __forceinline__ void stream_collide_brick(const BrickLevel<T> &lv, co
         // absent sources that no boundary condition sets keep the earlier values
 #pragma unroll
         for (int q = 1; q < Q; ++q)
-            if (missing & (1u << q)) f[q] = C(aux_f[q * lv.naux + ai]);
+            if (missing & (1u << q)) f[q] = C(aux_f[ai * aux_stride<D>() + q]);
     }
     if (is_aux) {
-#pragma unroll
-        for (int q = 0; q < Q; ++q) aux_f[q * lv.naux + ai] = T(f[q]);
+        store_row<D>(aux_f, ai, f);
         // a recorded node that nothing changes before its next collision collides here
         if (deferred) return;
     }
@@ -672,7 +711,7 @@ __device__ __forceinline__ void stream_collide_brick(const BrickLevel<T> &lv, co
 // four bricks per workgroup.
 template <int D, typename T, typename C, bool SHIFT, int COLL, int VAR>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(std::is_same<C, float>::value && !(VAR & 1) ? 8 : 1)))
+__attribute__((amdgpu_waves_per_eu(std::is_same<C, float>::value && !(VAR & 1) && VAR < 6 ? 8 : 1)))
 void k_stream_collide(Batch<FusedRun<T>> B) {
     const int k = B.find();
     const FusedRun<T> &R = B.run[k];
@@ -683,13 +722,17 @@ void k_stream_collide(Batch<FusedRun<T>> B) {
     stream_collide_brick<D, T, C, SHIFT, COLL, VAR>(R.lv, R.fin, R.fout, R.aux_f, R.p, b, nullptr);
 }
 
-// Pull of brick b (every lane, every direction) into a per-wave LDS buffer [Q][64] with one
+// the row stride of a staged brick in LDS: the five (three) units of an aux row, 4 strides apart, lie
+// 16 banks apart, so that 13 consecutive nodes' units are read without conflicts
+constexpr int kStageStride = 68;
+
+// Pull of brick b (every lane, every direction) into a per-wave LDS buffer [Q][kStageStride] with one
 // direct-to-LDS dword load per direction (gfx950 global_load_lds_dword: lane i lands at
 // buf + 4 i).  Every lane loads from a valid address of fin: an absent neighbour brick is
 // replaced by b, a deferred node's missing source loads whatever slot the stencil names, and a
 // lane without a node loads the slot its stencil names inside brick b; the consumer drops those values (a deferred node's
-// missing directions keep the boundary / transfer values already in the aux array).  Addresses are 32-bit byte offsets
-// from the direction's base fin + 64 q.  Returns the lane's missing-source mask (deferred nodes).
+// missing directions keep the boundary / transfer values already in its aux row).  Addresses are 32-bit byte offsets
+// from the direction's base fin + 64 q.  Returns the lane's aux_missing entry (recorded nodes).
 template <int D, typename T, bool BND>
 __device__ __forceinline__ uint32_t pull_to_lds(const BrickLevel<T> &t, const T *__restrict__ fin, int64_t b, int lane,
                                                 T *buf) {
@@ -698,8 +741,6 @@ __device__ __forceinline__ uint32_t pull_to_lds(const BrickLevel<T> &t, const T 
     constexpr int Q = L::Q;
     constexpr int NN = B::nnbr;
     static_assert(sizeof(T) == 4, "dword staging");
-    const uint64_t am = table_load(t.auxmask, b);
-    uint32_t missing = 0;
     // opaque per pull: the direction's LDS destinations are formed here, not hoisted out of the
     // caller's loop into 19 long-lived scalars
     asm volatile("" : "+s"(buf));
@@ -733,20 +774,21 @@ __device__ __forceinline__ uint32_t pull_to_lds(const BrickLevel<T> &t, const T 
 #pragma unroll
         for (int q = 0; q < Q; ++q)
             __builtin_amdgcn_global_load_lds((const void *)(reinterpret_cast<const char *>(fin) + o[q]),
-                                             (__attribute__((address_space(3))) void *)(buf + q * 64), 4, 0, 0);
-        if ((am >> lane) & 1ull) missing = t.aux_missing[table_load(t.auxbase, b) + __popcll(am & ((1ull << lane) - 1ull))];
-        return missing;
-    }
+                                             (__attribute__((address_space(3))) void *)(buf + q * kStageStride), 4, 0, 0);
+    } else {
     for_each_source<D>(P, has_node, nbo, self, [&](int q, uint32_t off) {
         // an opaque scalar base, so that the load takes the scalar-base + 32-bit-offset form
         const char *qbase = reinterpret_cast<const char *>(fin + q * 64);
         asm volatile("" : "+s"(qbase));
         const char *src = qbase + off;
-        __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)(buf + q * 64),
+        __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)(buf + q * kStageStride),
                                          4, 0, 0);
     });
-    if ((am >> lane) & 1ull) missing = t.aux_missing[table_load(t.auxbase, b) + __popcll(am & ((1ull << lane) - 1ull))];
-    return missing;
+    }
+    const uint64_t am = table_load(t.auxmask, b);
+    uint32_t entry = 0;
+    if ((am >> lane) & 1ull) entry = t.aux_missing[table_load(t.auxbase, b) + __popcll(am & ((1ull << lane) - 1ull))];
+    return entry;
 }
 
 // The same with the FP32 learned closure.  Each workgroup stages the network's operand images
@@ -770,11 +812,12 @@ void k_stream_collide_mlp(Batch<FusedRun<T>> B) {
     const T *fin = R.fin;
     T *fout = R.fout, *aux_f = R.aux_f;
     const StepParams &p = R.p;
-    const int64_t nbrick = t.nbrick, naux = t.naux;
+    const int64_t nbrick = t.nbrick;
     using L = Lattice<D>;
     constexpr int Q = L::Q;
     __shared__ MlpOps ops;
-    __shared__ T stage[4][Q * 64];
+    __shared__ T stage[4][Q * kStageStride];
+    __shared__ uint32_t who_s[4][64];        // aux_missing entries of the brick's recorded nodes, in order
     constexpr int64_t per_group = 4 * ROUNDS;
     const int64_t g = xcd_group((nbrick + per_group - 1) / per_group, blockIdx.x - B.first[run],
                                 B.first[run + 1] - B.first[run]);
@@ -783,8 +826,9 @@ void k_stream_collide_mlp(Batch<FusedRun<T>> B) {
     T *buf = stage[wave];
     int64_t b = g * per_group + wave;
     // the first pull goes out before the network is staged, so that their latencies overlap
-    uint32_t miss = 0;
-    if (b < nbrick) miss = pull_to_lds<D, T, BND>(t, fin, b, threadIdx.x & 63, buf);
+    uint32_t *who = who_s[wave];
+    uint32_t entry = 0;
+    if (b < nbrick) entry = pull_to_lds<D, T, BND>(t, fin, b, threadIdx.x & 63, buf);
     stage_mlp_ops<((VAR & 15) >> 1) == 4, mrt_on_mfma<C, VAR>()>(ops, p.mlp->ops);
     if (b >= nbrick) return;                 // uniform per wave; no barrier follows
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the first pull has landed
@@ -799,35 +843,37 @@ void k_stream_collide_mlp(Batch<FusedRun<T>> B) {
         asm volatile("" : "+v"(lane));
         C f[Q];
 #pragma unroll
-        for (int q = 0; q < Q; ++q) f[q] = C(buf[q * 64 + lane]);
+        for (int q = 0; q < Q; ++q) f[q] = C(buf[q * kStageStride + lane]);
         const bool has_node = (table_load(t.occ, b) >> lane) & 1ull;
         const uint64_t am = table_load(t.auxmask, b);
-        if ((am >> lane) & 1ull) {
-            // deferred node: post-stream values to the aux array, except the missing sources
-            // (their boundary / transfer values are there already): those go to the spare slot
-            // at index Q naux.  Stores take a uniform base and a 32-bit byte offset (the host
-            // keeps Q naux 4 below 2^32); a wavefront whose deferred lanes miss no source (a
-            // uniform branch) stores without the per-direction selection.
-            const uint32_t ai4 = 4u * (uint32_t)(table_load(t.auxbase, b) + __popcll(am & ((1ull << lane) - 1ull)));
-            using gchar = __attribute__((address_space(1))) char;
-            using gT = __attribute__((address_space(1))) T;
-            gchar *base = (gchar *)aux_f;
-            asm volatile("" : "+s"(base));
-            // (each offset is made opaque so that the store keeps the base + 32-bit offset form)
-            if (__builtin_amdgcn_ballot_w64(miss != 0u) == 0ull) {
+        if (am) {   // uniform
+            // recorded nodes: post-stream values to their aux rows, except the missing sources (their
+            // boundary / transfer values are there already).  The rows of a brick's nodes are one
+            // run of memory: the wavefront writes it in 16-byte units from the staged brick, so
+            // every store is whole lines (a row per lane took 147 us on a 3M-node level, this 134)
+            if ((am >> lane) & 1ull) who[__popcll(am & ((1ull << lane) - 1ull))] = entry;
+            wave_lds_sync();
+            const int64_t base = table_load(t.auxbase, b);
+            constexpr int U = aux_stride<D>() / 4;
+            const int units = (int)__popcll(am) * U;
+            for (int u0 = 0; u0 < units; u0 += 64) {
+                const int u = u0 + lane;
+                if (u < units) {
+                    const int j = u / U, q0 = 4 * (u - j * U);
+                    const uint32_t w = who[j];
+                    const T *v = buf + (w & 63u);
+                    RowUnit<T> x;
 #pragma unroll
-                for (int q = 0; q < Q; ++q) {
-                    uint32_t o = ai4 + (uint32_t)(4 * q * naux);
-                    asm volatile("" : "+v"(o));
-                    *(gT *)(base + o) = T(f[q]);
-                }
-            } else {
-                const uint32_t spare4 = (uint32_t)(4 * Q * naux);
+                    for (int k = 0; k < 4; ++k) x.v[k] = v[(q0 + k < Q ? q0 + k : 0) * kStageStride];
+                    T *dst = aux_f + (base + j) * aux_stride<D>() + q0;
+                    const uint32_t m = (w >> 6) >> q0 & 15u;
+                    if (m == 0u) {
+                        *reinterpret_cast<RowUnit<T> *>(dst) = x;
+                    } else {
 #pragma unroll
-                for (int q = 0; q < Q; ++q) {
-                    uint32_t o = ((miss >> q) & 1u) ? spare4 : ai4 + (uint32_t)(4 * q * naux);
-                    asm volatile("" : "+v"(o));
-                    *(gT *)(base + o) = T(f[q]);
+                        for (int k = 0; k < 4; ++k)
+                            if (!(m >> k & 1u)) dst[k] = x.v[k];
+                    }
                 }
             }
         }
@@ -835,8 +881,8 @@ void k_stream_collide_mlp(Batch<FusedRun<T>> B) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         const int64_t bn = b + 4;
         const bool more = r + 1 < ROUNDS && bn < nbrick;
-        uint32_t miss_next = 0;
-        if (more) miss_next = pull_to_lds<D, T, BND>(t, fin, bn, lane, buf);
+        uint32_t entry_next = 0;
+        if (more) entry_next = pull_to_lds<D, T, BND>(t, fin, bn, lane, buf);
         if (!has_node) {
 #pragma unroll
             for (int q = 0; q < Q; ++q) f[q] = C(0);          // rest state (shifted storage)
@@ -851,7 +897,7 @@ void k_stream_collide_mlp(Batch<FusedRun<T>> B) {
         for (int q = 0; q < Q; ++q) store_nt(T(f[q]), dst + q * 64);
         if (!more) break;
         b = bn;
-        miss = miss_next;
+        entry = entry_next;
     }
 }
 
@@ -866,7 +912,7 @@ void k_aux_collide(Batch<AuxRun<T>> B) {
     const int run = B.find();
     const AuxRun<T> &R = B.run[run];
     const int32_t *__restrict__ list = R.list;
-    const int64_t nlist = R.nlist, naux = R.naux;
+    const int64_t nlist = R.nlist;
     const T *__restrict__ aux_f = R.aux_f;
     const double *__restrict__ aux_force = R.aux_force;
     const StepParams &p = R.p;
@@ -881,7 +927,8 @@ void k_aux_collide(Batch<AuxRun<T>> B) {
     if (!kWave && !active) return;
     C f[Q];
 #pragma unroll
-    for (int q = 0; q < Q; ++q) f[q] = active ? C(aux_f[q * naux + i]) : C(SHIFT ? 0. : Lattice<D>::w[q]);
+    for (int q = 0; q < Q; ++q) f[q] = C(SHIFT ? 0. : Lattice<D>::w[q]);
+    if (active) load_row<D>(aux_f, i, f);
     // the network is staged after the node's loads are out, so that their latencies overlap
     const MlpOps *ops = nullptr;
     if constexpr (kWave) {

@@ -52,13 +52,14 @@ struct TransferTables {
     size_t lds_bytes = 0;       // rows plus contributor words of the largest group
     DevBuf groups;              // [n_groups] GatherGroup
     DevBuf group_rows;          // rows of src_f each group stages, first use order
+    DevBuf group_aux;           // the same as aux rows: of the coarse level, or ~(of the fine level)
     int64_t n_fb = 0;           // fine nodes standing in for missing coarse sources
     DevBuf src_coarse_ai;       // [n_src] coarse aux index of each source row (ascending)
     DevBuf fb_fine_ai;          // [n_fb] fine aux index of each fallback row (ascending)
-    DevBuf src_f;               // [n_src + n_fb][Q] rescaled coarse rows, then fallback copies
-                                // (storage form), as of the last synchronised transfer
-    DevBuf src_mid;             // the same rows of a time-interpolated refill (coarse rows: mean
-                                // of src_f and the current ones)
+    // time interpolation only (allocated when it is on): the rescaled coarse rows, then fallback
+    // copies, [n_src + n_fb][S] in storage form, as of the last synchronised transfer, and the rows
+    // of a time-interpolated refill (coarse rows: mean of src_f and the current ones)
+    DevBuf src_f, src_mid;
     DevBuf f2c_coarse_ai;       // [n_f2c]
     DevBuf f2c_fine_ai;         // [n_f2c] fine aux index of the coincident node
     bool f2c_apart = false;     // no fine node is both a gather target and a fine-to-coarse

@@ -228,10 +228,7 @@ __global__ void k_upload(BrickLevel<T> lv, const double *f_in, int64_t n, const 
     for (int q = 0; q < Q; ++q)
         f[q] = active ? C(f_in[i * Q + q] - (SHIFT ? Lattice<D>::w[q] : 0.)) : C(SHIFT ? 0. : Lattice<D>::w[q]);
     const int32_t ai = active ? node_aux[i] : -1;
-    if (ai >= 0) {
-#pragma unroll
-        for (int q = 0; q < Q; ++q) aux_f[q * lv.naux + ai] = T(f[q]);
-    }
+    if (ai >= 0) store_row<D>(aux_f, ai, f);
     // a boundary node's first collision starts from the stored form of the values, as an aux node's
     if (ai == kResolvedBoundary) {
 #pragma unroll
@@ -262,7 +259,7 @@ __device__ __forceinline__ double post_stream_value(const BrickLevel<T> &lv, int
     constexpr int Q = L::Q;
     double v;
     if (ai >= 0) {
-        v = double(aux_f[q * lv.naux + ai]);
+        v = double(aux_f[(int64_t)ai * aux_stride<D>() + q]);
     } else if (fresh || q == 0) {
         v = double(last[pop_at<Q>(q, slot)]);
     } else if (lv.bnd.brick && (lv.bnd.brick[slot >> 6].y >> q & 1)) {
@@ -386,7 +383,7 @@ struct BcIdx {
 // BoundaryBounceBack{2D,3D} (lbm_bounce_back.cpp:29-91): f[in] = f_collide[out] - 6 rho0 w (c.u_w)
 template <int D, typename T>
 __global__ void k_bc_bounce_back(int64_t nb, const int32_t *node_ai, const int32_t *node_slot, const T *fa,
-                                 int64_t nslot, T *aux_f, int64_t naux, BcIdx idx, double rho0, double ux,
+                                 T *aux_f, BcIdx idx, double rho0, double ux,
                                  double uy, double uz) {
     using L = Lattice<D>;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -395,25 +392,25 @@ __global__ void k_bc_bounce_back(int64_t nb, const int32_t *node_ai, const int32
     for (int k = 0; k < idx.n; ++k) {
         const int o = idx.inv[k];
         const double cu = L::cx[o] * ux + L::cy[o] * uy + (D == 3 ? L::cz[o] * uz : 0.);
-        aux_f[idx.ind[k] * naux + ai] = T(double(fa[pop_at<L::Q>(o, slot)]) - 6. * rho0 * L::w[o] * cu);
+        aux_f[ai * aux_stride<D>() + idx.ind[k]] = T(double(fa[pop_at<L::Q>(o, slot)]) - 6. * rho0 * L::w[o] * cu);
     }
 }
 
 // BoundaryPeriodic{2D,3D} (lbm_periodic.cpp:22-133): incoming directions copied from the twin
-template <typename T>
-__global__ void k_bc_periodic(int64_t nb, const int32_t *node_ai, const int32_t *twin_ai, T *aux_f,
-                              int64_t naux, BcIdx idx) {
+template <int D, typename T>
+__global__ void k_bc_periodic(int64_t nb, const int32_t *node_ai, const int32_t *twin_ai, T *aux_f, BcIdx idx) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nb) return;
     const int64_t ai = node_ai[t], tj = twin_ai[t];
     if (tj < 0) return;
-    for (int k = 0; k < idx.n; ++k) aux_f[idx.ind[k] * naux + ai] = aux_f[idx.ind[k] * naux + tj];
+    constexpr int S = aux_stride<D>();
+    for (int k = 0; k < idx.n; ++k) aux_f[ai * S + idx.ind[k]] = aux_f[tj * S + idx.ind[k]];
 }
 
 // BoundaryNonEqExtrapolation{2D,3D} (lbm_noneq_extrapolation.cpp:29-144):
 // f = feq(rho0, u_b) + f(inner) - feq(rho, u of inner)
 template <int D, typename T, typename C, bool SHIFT>
-__global__ void k_bc_nee(int64_t nb, const int32_t *node_ai, const int32_t *inner_ai, T *aux_f, int64_t naux,
+__global__ void k_bc_nee(int64_t nb, const int32_t *node_ai, const int32_t *inner_ai, T *aux_f,
                          const double *aux_force, StepParams p, double rho0, double ux, double uy, double uz,
                          const double *ub_node) {
     constexpr int Q = Lattice<D>::Q;
@@ -422,7 +419,7 @@ __global__ void k_bc_nee(int64_t nb, const int32_t *node_ai, const int32_t *inne
     const int64_t ai = node_ai[t], j = inner_ai[t];
     if (j < 0) return;
     C f[Q];
-    for (int q = 0; q < Q; ++q) f[q] = C(aux_f[q * naux + j]);
+    load_row<D>(aux_f, j, f);
     C F[3] = {C(p.const_force[0]), C(p.const_force[1]), C(p.const_force[2])};
     if (p.has_force && aux_force) {
         F[0] += C(aux_force[j * 3]); F[1] += C(aux_force[j * 3 + 1]); F[2] += C(aux_force[j * 3 + 2]);
@@ -435,11 +432,13 @@ __global__ void k_bc_nee(int64_t nb, const int32_t *node_ai, const int32_t *inne
     const C ubx = C(ub_node ? ub_node[t * 3] : ux), uby = C(ub_node ? ub_node[t * 3 + 1] : uy);
     const C ubz = C(D == 3 ? (ub_node ? ub_node[t * 3 + 2] : uz) : 0.);
     const C ubsq = ubx * ubx + uby * uby + ubz * ubz;
+#pragma unroll
     for (int q = 0; q < Q; ++q) {
         const C fb = feq_stored<D, SHIFT, C>(q, rb, drb, ubx, uby, ubz, ubsq, p.compressible);
         const C fi = feq_stored<D, SHIFT, C>(q, rho, drho, u[0], u[1], u[2], usq, p.compressible);
-        aux_f[q * naux + ai] = T(fb + f[q] - fi);
+        f[q] = fb + f[q] - fi;
     }
+    store_row<D>(aux_f, ai, f);
 }
 
 
@@ -827,7 +826,7 @@ zlh_status launch_step_kernels(zlh_ctx *ctx, const int *levels, int n, int coll)
     for (int i = 0; i < n; ++i) {
         LevelState &L = ctx->lv[levels[i]];
         T *fa = L.f_d[L.cur].as<T>(), *fb = L.f_d[L.cur ^ 1].as<T>();
-        AuxRun<T> a{L.naux, L.naux, nullptr, L.aux_slot_d.as<int32_t>(), L.aux_f_d.as<T>(), L.aux_force_d.as<double>(), fa,
+        AuxRun<T> a{L.naux, nullptr, L.aux_slot_d.as<int32_t>(), L.aux_f_d.as<T>(), L.aux_force_d.as<double>(), fa,
                     L.aux_macro_d.as<double>(), L.aux_macro_flag_d.as<uint8_t>(), L.sp};
         if (L.pending != kPendingAll) {
             const int pk = L.pending == kPendingTransfer ? 1 : 0;
@@ -881,17 +880,17 @@ zlh_status launch_step_kernels(zlh_ctx *ctx, const int *levels, int n, int coll)
                 case ZLH_BC_BOUNCE_BACK:
                     hipLaunchKernelGGL((k_bc_bounce_back<D, T>), dim3(blocks(L.bc_n[dir])), dim3(256), 0, ctx->stream,
                                        L.bc_n[dir], L.bc_ai_d[dir].as<int32_t>(), L.bc_slot_d[dir].as<int32_t>(), fa,
-                                       L.nbrick * 64, aux_f, L.naux, idx, ctx->d.rho0, bv[0], bv[1], bv[2]);
+                                       aux_f, idx, ctx->d.rho0, bv[0], bv[1], bv[2]);
                     break;
                 case ZLH_BC_PERIODIC:
-                    hipLaunchKernelGGL((k_bc_periodic<T>), dim3(blocks(L.bc_n[dir])), dim3(256), 0, ctx->stream,
+                    hipLaunchKernelGGL((k_bc_periodic<D, T>), dim3(blocks(L.bc_n[dir])), dim3(256), 0, ctx->stream,
                                        L.bc_n[dir], L.bc_ai_d[dir].as<int32_t>(), L.bc_partner_d[dir].as<int32_t>(),
-                                       aux_f, L.naux, idx);
+                                       aux_f, idx);
                     break;
                 case ZLH_BC_NEE:
                     hipLaunchKernelGGL((k_bc_nee<D, T, C, SHIFT>), dim3(blocks(L.bc_n[dir])), dim3(256), 0, ctx->stream,
                                        L.bc_n[dir], L.bc_ai_d[dir].as<int32_t>(), L.bc_partner_d[dir].as<int32_t>(),
-                                       aux_f, L.naux, aux_force, L.sp, ctx->d.rho0, bv[0], bv[1], bv[2],
+                                       aux_f, aux_force, L.sp, ctx->d.rho0, bv[0], bv[1], bv[2],
                                        L.bc_u_d[dir].p ? L.bc_u_d[dir].as<double>() : nullptr);
                     break;
                 default:
@@ -1321,7 +1320,7 @@ zlh_status build_level_aux(zlh_ctx *ctx, int level) {
         const int32_t slot = L.node_slot_h[i];
         auxmask[slot >> 6] |= 1ull << (slot & 63);
         aux_slot[k] = slot;
-        aux_missing[k] = L.missing_h[i];
+        aux_missing[k] = L.missing_h[i] << 6 | (uint32_t)(slot & 63);
         L.node_aux_h[i] = (int32_t)k;
     }
     int32_t acc = 0;
@@ -1393,10 +1392,8 @@ zlh_status build_level_aux(zlh_ctx *ctx, int level) {
     const size_t ts = ctx->tsize();
     if ((s = dalloc(ctx, L.f_d[0], ts * Q * nslot))) return s;
     if ((s = dalloc(ctx, L.f_d[1], ts * Q * nslot))) return s;
-    // one spare element past [Q][naux]: the learned-closure kernel parks a deferred node's
-    // missing directions there instead of branching around their stores
-    if ((int64_t)Q * L.naux + 1 >= ((int64_t)1 << 31)) return ctx->fail(ZLH_ENOMEM, "level %d: aux array too large", level);
-    if ((s = dalloc(ctx, L.aux_f_d, ts * (Q * std::max<int64_t>(L.naux, 1) + 1)))) return s;
+    const int64_t stride = dims == 2 ? aux_stride<2>() : aux_stride<3>();
+    if ((s = dalloc(ctx, L.aux_f_d, ts * stride * std::max<int64_t>(L.naux, 1)))) return s;
     if ((s = dalloc(ctx, L.aux_macro_d, sizeof(double) * 4 * std::max<int64_t>(L.naux, 1)))) return s;
     if ((s = dalloc(ctx, L.aux_macro_flag_d, std::max<int64_t>(L.naux, 1)))) return s;
     if ((s = dalloc(ctx, L.aux_force_d, sizeof(double) * 3 * std::max<int64_t>(L.naux, 1)))) return s;
