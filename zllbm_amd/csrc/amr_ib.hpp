@@ -338,41 +338,22 @@ __global__ __launch_bounds__(256) void k_c2f_gather_f2c(int64_t nb_gather, int64
     }
 }
 
-// immersed boundary, step 1: zero the force of every supported node and recompute its velocity
-// with the remaining (constant) force (the lazy reset, immersed_boundary.cpp:76-85, 284-296)
-template <int D, typename T, typename C, bool SHIFT>
-__global__ void k_ib_reset(int64_t n, const int32_t *reset_ai, const T *aux_f, double *aux_force,
-                           double *node_u, StepParams p) {
-    constexpr int Q = Lattice<D>::Q;
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const int64_t ai = reset_ai[k];
-    aux_force[ai * 3] = 0.;
-    aux_force[ai * 3 + 1] = 0.;
-    aux_force[ai * 3 + 2] = 0.;
-    C f[Q];
-    load_row<D>(aux_f, ai, f);
-    C F[3] = {C(p.const_force[0]), C(p.const_force[1]), C(p.const_force[2])};
-    C rho, drho, u[3];
-    macro<D, SHIFT, C>(f, F, C(p.dt), 1, p.compressible, rho, drho, u);
-    node_u[ai * 3] = double(u[0]);
-    node_u[ai * 3 + 1] = double(u[1]);
-    node_u[ai * 3 + 2] = double(u[2]);
-}
-
 __device__ __forceinline__ double wave_sum(double v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
 }
 
-// immersed boundary, step 2: one wavefront per marker; lanes hold the stencil nodes.  Velocity
-// interpolation by a wavefront reduction and the Lagrangian force F = k (U - u_ref)
-// (DirectForcingScheme{2D,3D}, immersed_boundary.cpp:108-364)
-template <int D>
+// immersed boundary, step 1: one wavefront per marker; lanes hold the stencil nodes.  Each lane
+// recomputes its node's velocity with the remaining (constant) force (the lazy reset,
+// immersed_boundary.cpp:76-85, 284-296), then interpolation by a wavefront reduction and the
+// Lagrangian force F = k (U - u_ref) (DirectForcingScheme{2D,3D}, immersed_boundary.cpp:108-364).
+// A node lies in about eleven markers' stencils, so its velocity is computed as often; its row is
+// five vector loads, and a launch over the nodes that stored the velocities took 4.8 us beside the
+// markers' 4.7 (1,810 markers).
+template <int D, typename T, typename C, bool SHIFT>
 __global__ __launch_bounds__(256) void k_ib_markers(int64_t n_markers, int support, const int32_t *node_ai,
-                                                    const double *weight, const double *node_u,
-                                                    const double *marker_vel, double stiffness,
-                                                    double *marker_force) {
+                                                    const double *weight, const T *aux_f, const double *marker_vel,
+                                                    double stiffness, double *marker_force, StepParams p) {
     const int64_t m = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int lane = threadIdx.x & 63;
     if (m >= n_markers) return;
@@ -383,8 +364,14 @@ __global__ __launch_bounds__(256) void k_ib_markers(int64_t n_markers, int suppo
         w = weight[m * support + lane];
     }
     double u[3] = {0., 0., 0.};
-    if (ai >= 0)
-        for (int a = 0; a < D; ++a) u[a] = node_u[(int64_t)ai * 3 + a] * w;
+    if (ai >= 0) {
+        C f[Lattice<D>::Q];
+        load_row<D>(aux_f, ai, f);
+        C F[3] = {C(p.const_force[0]), C(p.const_force[1]), C(p.const_force[2])};
+        C rho, drho, v[3];
+        macro<D, SHIFT, C>(f, F, C(p.dt), 1, p.compressible, rho, drho, v);
+        for (int a = 0; a < D; ++a) u[a] = double(v[a]) * w;
+    }
     double fm[3] = {0., 0., 0.};
     for (int a = 0; a < D; ++a) {
         const double ur = wave_sum(u[a]);
@@ -394,7 +381,7 @@ __global__ __launch_bounds__(256) void k_ib_markers(int64_t n_markers, int suppo
         for (int a = 0; a < 3; ++a) marker_force[m * 3 + a] = fm[a];
 }
 
-// immersed boundary, step 3: the spread F delta area / (dt dx^(d-1)) of every marker onto its
+// immersed boundary, step 2: the spread F delta area / (dt dx^(d-1)) of every marker onto its
 // stencil nodes (immersed_boundary.cpp:108-364), as a gather: one thread per supported node sums
 // its markers' terms in FP64, in ascending marker order, and stores the node force.  Neighbouring
 // markers share most of their stencil nodes, so a per-marker scatter would serialise on atomics.
@@ -965,7 +952,6 @@ inline zlh_status upload_ib(zlh_ctx *ctx, int level) {
     if ((s = upload(ctx, T.reset_ai, reset))) return s;
     if ((s = upload(ctx, T.marker_vel, L.ib.vel))) return s;
     if ((s = dalloc(ctx, T.marker_force, sizeof(double) * 3 * T.n_markers))) return s;
-    if ((s = dalloc(ctx, T.node_u, sizeof(double) * 3 * std::max<int64_t>(L.naux, 1)))) return s;
     return ZLH_OK;
 }
 
@@ -1052,12 +1038,9 @@ template <int D, typename T, typename Cc, bool SHIFT>
 zlh_status launch_ib_t(zlh_ctx *ctx, int level) {
     LevelState &L = ctx->lv[level];
     IbTables &B = L.ibt;
-    hipLaunchKernelGGL((k_ib_reset<D, T, Cc, SHIFT>), dim3(blocks(B.n_reset)), dim3(256), 0, ctx->stream, B.n_reset,
-                       B.reset_ai.as<int32_t>(), L.aux_f_d.as<T>(), L.aux_force_d.as<double>(),
-                       B.node_u.as<double>(), L.sp);
-    hipLaunchKernelGGL((k_ib_markers<D>), dim3(blocks(B.n_markers * 64)), dim3(256), 0, ctx->stream, B.n_markers,
-                       B.support, B.node_ai.as<int32_t>(), B.weight.as<double>(), B.node_u.as<double>(),
-                       B.marker_vel.as<double>(), B.stiffness, B.marker_force.as<double>());
+    hipLaunchKernelGGL((k_ib_markers<D, T, Cc, SHIFT>), dim3(blocks(B.n_markers * 64)), dim3(256), 0, ctx->stream,
+                       B.n_markers, B.support, B.node_ai.as<int32_t>(), B.weight.as<double>(), L.aux_f_d.as<T>(),
+                       B.marker_vel.as<double>(), B.stiffness, B.marker_force.as<double>(), L.sp);
     hipLaunchKernelGGL((k_ib_spread<D>), dim3(blocks(B.n_reset)), dim3(256), 0, ctx->stream, B.n_reset,
                        B.reset_ai.as<int32_t>(), B.spread_begin.as<int32_t>(), B.spread_marker.as<int32_t>(),
                        B.spread_weight.as<double>(), B.marker_force.as<double>(), L.aux_force_d.as<double>());

@@ -78,7 +78,6 @@ struct IbTables {
     DevBuf spread_begin;        // [n_reset + 1] offsets into the spread arrays per supported node
     DevBuf spread_marker;       // marker of each spread term, ascending per node
     DevBuf spread_weight;       // its delta weight times the marker's area / (dt dx^(dims-1))
-    DevBuf node_u;              // [naux][3] velocity recomputed at the reset (double)
     DevBuf marker_vel;          // [n_markers][3]
     DevBuf marker_force;        // [n_markers][3] Lagrangian force
     double stiffness = 2.;
