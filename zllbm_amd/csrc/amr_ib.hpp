@@ -343,7 +343,7 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// immersed boundary, step 1: one wavefront per marker; lanes hold the stencil nodes.  Each lane
+// immersed boundary: one wavefront per marker; lanes hold the stencil nodes.  Each lane
 // recomputes its node's velocity with the remaining (constant) force (the lazy reset,
 // immersed_boundary.cpp:76-85, 284-296), then interpolation by a wavefront reduction and the
 // Lagrangian force F = k (U - u_ref) (DirectForcingScheme{2D,3D}, immersed_boundary.cpp:108-364).
@@ -379,30 +379,6 @@ __global__ __launch_bounds__(256) void k_ib_markers(int64_t n_markers, int suppo
     }
     if (lane == 0)
         for (int a = 0; a < 3; ++a) marker_force[m * 3 + a] = fm[a];
-}
-
-// immersed boundary, step 2: the spread F delta area / (dt dx^(d-1)) of every marker onto its
-// stencil nodes (immersed_boundary.cpp:108-364), as a gather: one thread per supported node sums
-// its markers' terms in FP64, in ascending marker order, and stores the node force.  Neighbouring
-// markers share most of their stencil nodes, so a per-marker scatter would serialise on atomics.
-template <int D>
-__global__ __launch_bounds__(256) void k_ib_spread(int64_t n_reset, const int32_t *__restrict__ reset_ai,
-                                                   const int32_t *__restrict__ begin,
-                                                   const int32_t *__restrict__ marker,
-                                                   const double *__restrict__ coef,
-                                                   const double *__restrict__ marker_force,
-                                                   double *__restrict__ aux_force) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_reset) return;
-    double acc[3] = {0., 0., 0.};
-#pragma unroll 4
-    for (int32_t e = begin[r]; e < begin[r + 1]; ++e) {
-        const int64_t m = marker[e];
-        const double s = coef[e];
-        for (int a = 0; a < D; ++a) acc[a] += marker_force[m * 3 + a] * s;
-    }
-    const int64_t ai = reset_ai[r];
-    for (int a = 0; a < D; ++a) aux_force[ai * 3 + a] = acc[a];
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -949,7 +925,7 @@ inline zlh_status upload_ib(zlh_ctx *ctx, int level) {
     if ((s = upload(ctx, T.spread_weight, coef))) return s;
     if ((s = upload(ctx, T.node_ai, ai))) return s;
     if ((s = upload(ctx, T.weight, P.weight))) return s;
-    if ((s = upload(ctx, T.reset_ai, reset))) return s;
+    if ((s = upload(ctx, T.spread_row, pos))) return s;
     if ((s = upload(ctx, T.marker_vel, L.ib.vel))) return s;
     if ((s = dalloc(ctx, T.marker_force, sizeof(double) * 3 * T.n_markers))) return s;
     return ZLH_OK;
@@ -1041,9 +1017,6 @@ zlh_status launch_ib_t(zlh_ctx *ctx, int level) {
     hipLaunchKernelGGL((k_ib_markers<D, T, Cc, SHIFT>), dim3(blocks(B.n_markers * 64)), dim3(256), 0, ctx->stream,
                        B.n_markers, B.support, B.node_ai.as<int32_t>(), B.weight.as<double>(), L.aux_f_d.as<T>(),
                        B.marker_vel.as<double>(), B.stiffness, B.marker_force.as<double>(), L.sp);
-    hipLaunchKernelGGL((k_ib_spread<D>), dim3(blocks(B.n_reset)), dim3(256), 0, ctx->stream, B.n_reset,
-                       B.reset_ai.as<int32_t>(), B.spread_begin.as<int32_t>(), B.spread_marker.as<int32_t>(),
-                       B.spread_weight.as<double>(), B.marker_force.as<double>(), L.aux_force_d.as<double>());
     ZLH_TRY(hipGetLastError());
     return ZLH_OK;
 }

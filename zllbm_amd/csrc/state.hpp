@@ -74,7 +74,7 @@ struct IbTables {
     int64_t n_reset = 0;
     DevBuf node_ai;             // [n_markers][support] aux index, -1 for unused entries
     DevBuf weight;              // [n_markers][support] delta weight (double)
-    DevBuf reset_ai;            // [n_reset] aux indices of every supported node, ascending
+    DevBuf spread_row;          // [naux] place of a supported node in spread_begin, else -1
     DevBuf spread_begin;        // [n_reset + 1] offsets into the spread arrays per supported node
     DevBuf spread_marker;       // marker of each spread term, ascending per node
     DevBuf spread_weight;       // its delta weight times the marker's area / (dt dx^(dims-1))

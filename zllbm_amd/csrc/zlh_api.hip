@@ -826,7 +826,11 @@ zlh_status launch_step_kernels(zlh_ctx *ctx, const int *levels, int n, int coll)
     for (int i = 0; i < n; ++i) {
         LevelState &L = ctx->lv[levels[i]];
         T *fa = L.f_d[L.cur].as<T>(), *fb = L.f_d[L.cur ^ 1].as<T>();
-        AuxRun<T> a{L.naux, nullptr, L.aux_slot_d.as<int32_t>(), L.aux_f_d.as<T>(), L.aux_force_d.as<double>(), fa,
+        IbForce ib{};
+        if (L.ibt.n_markers > 0)
+            ib = IbForce{L.ibt.spread_row.as<int32_t>(), L.ibt.spread_begin.as<int32_t>(), L.ibt.spread_marker.as<int32_t>(),
+                         L.ibt.spread_weight.as<double>(), L.ibt.marker_force.as<double>(), L.aux_force_d.as<double>()};
+        AuxRun<T> a{L.naux, nullptr, L.aux_slot_d.as<int32_t>(), L.aux_f_d.as<T>(), ib, fa,
                     L.aux_macro_d.as<double>(), L.aux_macro_flag_d.as<uint8_t>(), L.sp};
         if (L.pending != kPendingAll) {
             const int pk = L.pending == kPendingTransfer ? 1 : 0;
