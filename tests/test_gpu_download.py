@@ -1,6 +1,6 @@
-"""Downloads of populations and macroscopic variables at sizes around a staging chunk (4 MiB of
-output: 27,594 nodes of D3Q19 populations, 174,762 nodes of 2D macros), against the uploaded
-values and the oracle."""
+"""Downloads of populations and macroscopic variables at sizes from one node row to many staging
+chunks (1 MiB of output: 6,898 nodes of D3Q19 populations, 43,690 nodes of 2D macros), against the
+uploaded values and the oracle."""
 import numpy as np
 import pytest
 

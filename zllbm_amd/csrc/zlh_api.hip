@@ -7,6 +7,7 @@
 // boundary / transfer / forcing tables that address them.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <initializer_list>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -322,8 +323,8 @@ __global__ __launch_bounds__(128) void k_rows_out(BrickLevel<T> lv, const int32_
 // Density and velocity (rho [m], then u [m][D]) of the post-stream populations of the same nodes,
 // into pinned host memory, summed in double in direction order as the reference sums them
 // (CalMacro*, lbm_solver_interface.cpp:477-592).  (1 + D) 8 bytes of a node cross the host link
-// where its populations are 8 Q: the 3.29M nodes of a four-level D3Q19 grid take 8.6 ms, host
-// copy included (12 GB/s, bound by the page faults of a fresh destination), where downloading the
+// where its populations are 8 Q: the 3.29M nodes of a four-level D3Q19 grid take 7.5 ms, host
+// copy included (14 GB/s, bound by the page faults of a fresh destination), where downloading the
 // populations and summing them on the host took 269 ms.
 template <int D, typename T, bool SHIFT>
 __global__ __launch_bounds__(256) void k_macros_out(BrickLevel<T> lv, const int32_t *node_slot, const int32_t *node_aux,
@@ -531,6 +532,11 @@ struct zlh_ctx {
     DevBuf lattice_d;
     // pinned staging of the downloads (download_nodes): two halves, grown to what a call needs up
     // to 2 kStageBytes, freed with the context
+    // device workspace of the closure's gradient, training and evaluation, kept between calls up to
+    // kWorkBytes and freed with the context
+    DevBuf work;
+    // held by the calls that use stage or work: callers on several threads take turns
+    std::mutex scratch_m;
     char *stage = nullptr;
     size_t stage_bytes = 0;
     hipEvent_t ev_stage[2] = {nullptr, nullptr};
@@ -988,10 +994,11 @@ zlh_status do_materialize(zlh_ctx *ctx, int level, double *out_dev) {
 
 // Downloads of a level's nodes: a kernel writes a chunk of nodes into one half of a pinned buffer
 // while the host copies the other half into the caller's array, so that no device workspace is
-// allocated and the only bytes over the host link are those returned.  kStageBytes: chunks of
-// 4 MiB keep both sides busy and the buffer small.  A 33^2 macros call takes 28 us where
-// allocating, copying and freeing device memory took 82.
-constexpr size_t kStageBytes = 4u << 20;
+// allocated and the only bytes over the host link are those returned.  kStageBytes: macros of 3.2M
+// nodes took 9.1 / 7.3 / 7.0 / 8.6 ms with chunks of 0.5 / 1 / 2 / 4 MiB, and a solver's first call
+// pays for pinning the buffer (1.8 ms at 4 MiB).  A 33^2 macros call takes 22 us where allocating,
+// copying and freeing device memory took 82.
+constexpr size_t kStageBytes = (size_t)1 << 20;
 
 zlh_status stage_reserve(zlh_ctx *ctx, size_t bytes) {
     if (ctx->stage_bytes >= bytes) return ZLH_OK;
@@ -1011,6 +1018,7 @@ zlh_status stage_reserve(zlh_ctx *ctx, size_t bytes) {
 
 template <int D, typename T, bool SHIFT>
 zlh_status download_nodes_t(zlh_ctx *ctx, int level, double *f, double *rho, double *u) {
+    std::lock_guard<std::mutex> hold(ctx->scratch_m);
     LevelState &L = ctx->lv[level];
     BrickLevel<T> v = view<T>(L);
     // the buffer read by the last fused kernel (or, before any step, the uploaded populations)
@@ -1021,7 +1029,11 @@ zlh_status download_nodes_t(zlh_ctx *ctx, int level, double *f, double *rho, dou
     const int64_t chunk = std::min<int64_t>(L.n, (int64_t)(kStageBytes / 8) / per);
     const size_t half = ((size_t)(chunk * per) * 8 + 255) & ~(size_t)255;
     const int64_t nchunk = (L.n + chunk - 1) / chunk;
-    zlh_status s = stage_reserve(ctx, nchunk > 1 ? 2 * half : half);
+    // both halves for the largest level and the larger rows at once: one allocation per solver
+    int64_t largest = 0;
+    for (const LevelState &l : ctx->lv) largest = std::max(largest, l.n);
+    const size_t most = (size_t)std::min<int64_t>((int64_t)kStageBytes, largest * Q * 8);
+    zlh_status s = stage_reserve(ctx, 2 * ((most + 255) & ~(size_t)255));
     if (s) return s;
     auto fill = [&](int64_t c) -> hipError_t {
         const int64_t i0 = c * chunk, m = std::min(chunk, L.n - i0);
@@ -2053,6 +2065,33 @@ zlh_status zlh_mlp_set(zlh_ctx *ctx, const float *params, const float *mean, con
     return ZLH_OK;
 }
 
+// Device memory of one closure call: the context's workspace, or for a call that needs more than
+// kWorkBytes its own allocation, freed on return.  take() hands out 256-byte aligned parts of it.
+constexpr size_t kWorkBytes = (size_t)64 << 20;
+struct ClosureWork {
+    DevBuf own;
+    char *at = nullptr;
+    std::unique_lock<std::mutex> hold;
+    zlh_status reserve(zlh_ctx *ctx, std::initializer_list<size_t> floats) {
+        size_t bytes = 0;
+        for (size_t n : floats) bytes += (n * sizeof(float) + 255) & ~(size_t)255;
+        const bool kept = bytes <= kWorkBytes;
+        if (kept) hold = std::unique_lock<std::mutex>(ctx->scratch_m);
+        DevBuf &b = kept ? ctx->work : own;
+        if (!b.p || b.bytes < bytes) {
+            const zlh_status s = dalloc(ctx, b, bytes, false);
+            if (s) return s;
+        }
+        at = b.as<char>();
+        return ZLH_OK;
+    }
+    float *take(size_t floats) {
+        float *p = reinterpret_cast<float *>(at);
+        at += (floats * sizeof(float) + 255) & ~(size_t)255;
+        return p;
+    }
+};
+
 // gradient kernel of the selected training form (128 samples per workgroup trip in FP32, 256 with
 // BF16 operands; a grid of at most kGradMaxBlocks workgroups that loop over the batch): returns
 // the rows of part it writes
@@ -2087,23 +2126,23 @@ zlh_status zlh_mlp_gradient(zlh_ctx *ctx, const float *params, const float *x, c
                             float *loss) {
     if (!ctx) return ZLH_EINVAL;
     if (!params || !x || !t || !grad || n < 1 || n > (1 << 26)) return ctx->fail(ZLH_EINVAL, "bad gradient arguments");
-    DevBuf dp, dx, dt, dg, dr;
-    zlh_status s;
-    if ((s = dalloc(ctx, dp, sizeof(float) * kMlpParams, false))) return s;
-    if ((s = dalloc(ctx, dx, sizeof(float) * kMlpF * n, false))) return s;
-    if ((s = dalloc(ctx, dt, sizeof(float) * n, false))) return s;
-    if ((s = dalloc(ctx, dg, sizeof(float) * (kMlpParams + 1), false))) return s;
-    if ((s = dalloc(ctx, dr, sizeof(float) * kGradMaxBlocks * kGradRow, false))) return s;
-    ZLH_TRY(hipMemcpyAsync(dp.p, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice, ctx->stream));
-    ZLH_TRY(hipMemcpyAsync(dx.p, x, sizeof(float) * kMlpF * n, hipMemcpyHostToDevice, ctx->stream));
-    ZLH_TRY(hipMemcpyAsync(dt.p, t, sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
-    launch_full_gradient(ctx, dp.as<float>(), dx.as<float>(), dt.as<float>(), n, dr.as<float>(), dg.as<float>(),
-                         dg.as<float>() + kMlpParams);
+    // (five allocations and frees a call took 60 us of a 70,000-sample gradient's 216)
+    constexpr size_t np = kMlpParams, ng = kMlpParams + 1, nr = (size_t)kGradMaxBlocks * kGradRow;
+    ClosureWork w;
+    zlh_status s = w.reserve(ctx, {np, (size_t)n * kMlpF, (size_t)n, ng, nr});
+    if (s) return s;
+    float *dp = w.take(np), *dx = w.take((size_t)n * kMlpF), *dt = w.take((size_t)n), *dg = w.take(ng), *dr = w.take(nr);
+    ZLH_TRY(hipMemcpyAsync(dp, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice, ctx->stream));
+    ZLH_TRY(hipMemcpyAsync(dx, x, sizeof(float) * kMlpF * n, hipMemcpyHostToDevice, ctx->stream));
+    ZLH_TRY(hipMemcpyAsync(dt, t, sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
+    launch_full_gradient(ctx, dp, dx, dt, n, dr, dg, dg + kMlpParams);
     ZLH_TRY(hipGetLastError());
-    ZLH_TRY(hipMemcpyAsync(grad, dg.p, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, ctx->stream));
-    if (loss)
-        ZLH_TRY(hipMemcpyAsync(loss, dg.as<float>() + kMlpParams, sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
+    // gradient and loss in one copy
+    float out[kMlpParams + 1];
+    ZLH_TRY(hipMemcpyAsync(out, dg, sizeof(out), hipMemcpyDeviceToHost, ctx->stream));
     ZLH_TRY(hipStreamSynchronize(ctx->stream));
+    std::memcpy(grad, out, sizeof(float) * kMlpParams);
+    if (loss) *loss = out[kMlpParams];
     return ZLH_OK;
 }
 
@@ -2133,32 +2172,30 @@ zlh_status zlh_mlp_train(zlh_ctx *ctx, const float *x, const float *t, int64_t n
     if (!ctx) return ZLH_EINVAL;
     if (!params || !x || !t || n < 1 || n > (1 << 26) || steps < 1 || batch < 1 || batch > (1 << 20) || !(lr > 0.))
         return ctx->fail(ZLH_EINVAL, "bad training arguments");
-    DevBuf dp, dx, dt, dr, dm, dv, dl;
-    zlh_status s;
-    if ((s = dalloc(ctx, dp, sizeof(float) * kMlpParams, false))) return s;
-    if ((s = dalloc(ctx, dx, sizeof(float) * kMlpF * n, false))) return s;
-    if ((s = dalloc(ctx, dt, sizeof(float) * n, false))) return s;
-    if ((s = dalloc(ctx, dr, sizeof(float) * kGradMaxBlocks * kGradRow, false))) return s;
-    if ((s = dalloc(ctx, dm, sizeof(float) * kMlpParams))) return s;
-    if ((s = dalloc(ctx, dv, sizeof(float) * kMlpParams))) return s;
-    if ((s = dalloc(ctx, dl, sizeof(float) * steps, false))) return s;
-    ZLH_TRY(hipMemcpyAsync(dp.p, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice, ctx->stream));
-    ZLH_TRY(hipMemcpyAsync(dx.p, x, sizeof(float) * kMlpF * n, hipMemcpyHostToDevice, ctx->stream));
-    ZLH_TRY(hipMemcpyAsync(dt.p, t, sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
+    constexpr size_t np = kMlpParams, nr = (size_t)kGradMaxBlocks * kGradRow;
+    ClosureWork w;
+    zlh_status s = w.reserve(ctx, {np, (size_t)n * kMlpF, (size_t)n, nr, np, np, (size_t)steps});
+    if (s) return s;
+    float *dp = w.take(np), *dx = w.take((size_t)n * kMlpF), *dt = w.take((size_t)n), *dr = w.take(nr);
+    float *dm = w.take(np), *dv = w.take(np), *dl = w.take((size_t)steps);
+    ZLH_TRY(hipMemsetAsync(dm, 0, sizeof(float) * np, ctx->stream));
+    ZLH_TRY(hipMemsetAsync(dv, 0, sizeof(float) * np, ctx->stream));
+    ZLH_TRY(hipMemcpyAsync(dp, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice, ctx->stream));
+    ZLH_TRY(hipMemcpyAsync(dx, x, sizeof(float) * kMlpF * n, hipMemcpyHostToDevice, ctx->stream));
+    ZLH_TRY(hipMemcpyAsync(dt, t, sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
     // a batch of at least n samples is the full set in order (plain full-batch Adam); smaller
     // batches are drawn with replacement from a per-step hash
     const int full = (int64_t)batch >= n;
     const int nb = full ? (int)n : batch;
     for (int it = 1; it <= steps; ++it) {
-        const int rows = launch_mlp_grad(ctx, dp.as<float>(), dx.as<float>(), dt.as<float>(), n, nb,
-                                         (uint32_t)(seed * 1000003ull + (uint64_t)it), full ? 0 : 1, dr.as<float>());
+        const int rows = launch_mlp_grad(ctx, dp, dx, dt, n, nb, (uint32_t)(seed * 1000003ull + (uint64_t)it),
+                                         full ? 0 : 1, dr);
         hipLaunchKernelGGL(k_grad_reduce<true>, dim3(blocks(kMlpParams + 1, 32)), dim3(256), 0, ctx->stream,
-                           dr.as<float>(), rows, nullptr, dl.as<float>() + (it - 1), dp.as<float>(), dm.as<float>(),
-                           dv.as<float>(), (float)lr, 0.9f, 0.999f, 1e-8f, it);
+                           dr, rows, nullptr, dl + (it - 1), dp, dm, dv, (float)lr, 0.9f, 0.999f, 1e-8f, it);
     }
     ZLH_TRY(hipGetLastError());
-    ZLH_TRY(hipMemcpyAsync(params, dp.p, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, ctx->stream));
-    if (loss_history) ZLH_TRY(hipMemcpyAsync(loss_history, dl.p, sizeof(float) * steps, hipMemcpyDeviceToHost, ctx->stream));
+    ZLH_TRY(hipMemcpyAsync(params, dp, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, ctx->stream));
+    if (loss_history) ZLH_TRY(hipMemcpyAsync(loss_history, dl, sizeof(float) * steps, hipMemcpyDeviceToHost, ctx->stream));
     ZLH_TRY(hipStreamSynchronize(ctx->stream));
     return ZLH_OK;
 }
@@ -2168,22 +2205,22 @@ zlh_status zlh_mlp_eval(zlh_ctx *ctx, const float *x, int64_t n, int form, float
     if (!ctx->mlp_set) return ctx->fail(ZLH_ESTATE, "learned closure not set");
     if (!x || !y || n < 1 || form < ZLH_MLP_FP32 || form > ZLH_MLP_FP16_MFMA)
         return ctx->fail(ZLH_EINVAL, "bad evaluation arguments");
-    DevBuf dx, dy;
-    zlh_status s;
-    if ((s = dalloc(ctx, dx, sizeof(float) * kMlpF * n, false))) return s;
-    if ((s = dalloc(ctx, dy, sizeof(float) * n, false))) return s;
-    ZLH_TRY(hipMemcpyAsync(dx.p, x, sizeof(float) * kMlpF * n, hipMemcpyHostToDevice, ctx->stream));
+    ClosureWork w;
+    zlh_status s = w.reserve(ctx, {(size_t)n * kMlpF, (size_t)n});
+    if (s) return s;
+    float *dx = w.take((size_t)n * kMlpF), *dy = w.take((size_t)n);
+    ZLH_TRY(hipMemcpyAsync(dx, x, sizeof(float) * kMlpF * n, hipMemcpyHostToDevice, ctx->stream));
     if (form == ZLH_MLP_BF16_MFMA)
         hipLaunchKernelGGL(k_mlp_eval_wave<OperandsBf16>, dim3(blocks(n)), dim3(256), 0, ctx->stream,
-                           ctx->mlp_d.as<MlpDev>(), dx.as<float>(), n, dy.as<float>());
+                           ctx->mlp_d.as<MlpDev>(), dx, n, dy);
     else if (form == ZLH_MLP_FP16_MFMA)
         hipLaunchKernelGGL(k_mlp_eval_wave<OperandsF16>, dim3(blocks(n)), dim3(256), 0, ctx->stream,
-                           ctx->mlp_d.as<MlpDev>(), dx.as<float>(), n, dy.as<float>());
+                           ctx->mlp_d.as<MlpDev>(), dx, n, dy);
     else
         hipLaunchKernelGGL(k_mlp_eval, dim3(blocks(n)), dim3(256), 0, ctx->stream, ctx->mlp_d.as<MlpDev>(),
-                           dx.as<float>(), n, dy.as<float>());
+                           dx, n, dy);
     ZLH_TRY(hipGetLastError());
-    ZLH_TRY(hipMemcpyAsync(y, dy.p, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
+    ZLH_TRY(hipMemcpyAsync(y, dy, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
     ZLH_TRY(hipStreamSynchronize(ctx->stream));
     return ZLH_OK;
 }
