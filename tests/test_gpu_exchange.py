@@ -1,0 +1,83 @@
+"""The coarse/fine exchange, which stages and rescales aux rows itself, at boxes whose interfaces
+start at odd and even nodes of a brick, with thin and wide boxes and both interpolations, against
+the oracle; and the closure's workspace over calls of growing and shrinking size."""
+import threading
+
+import numpy as np
+import pytest
+
+from oracle.zlbm_oracle import Oracle
+from zllbm_amd import closure, grid as g
+from zllbm_amd import hip
+from tests import scenarios as sc
+from tests.test_gpu_mlp import _ctx, _data
+from tests.test_gpu_parity import assert_close
+
+pytestmark = pytest.mark.gpu
+
+BOXES = {
+    "2d even": (2, (24, 20), [((8, 6), (16, 14))]),
+    "2d odd": (2, (27, 23), [((5, 5), (16, 15)), ((15, 14), (23, 25))]),
+    "3d even": (3, (16, 16, 16), [((6, 6, 6), (12, 12, 12))]),
+    "3d odd": (3, (17, 19, 16), [((5, 5, 5), (12, 13, 12)), ((14, 15, 14), (20, 21, 20))]),
+}
+
+
+# FP64: rounding of sums in another order than the oracle's, 1e-12 of the largest population as the
+# other substep tests.  FP32 shifted: a few 2^-24 of |f - w| < 0.05 a step over 6 steps of collision
+# and exchange, far below 2e-6; populations are up to 1/3.
+@pytest.mark.parametrize("precision,tol", [(hip.FP64, 1e-12), (hip.FP32_SHIFTED, 2e-6)])
+@pytest.mark.parametrize("interp", [hip.INTERP_LAGRANGIAN, hip.INTERP_LINEAR])
+@pytest.mark.parametrize("box", sorted(BOXES))
+def test_exchange_against_oracle(box, interp, precision, tol):
+    dims, cells, boxes = BOXES[box]
+    grid = g.refined_box_grid(dims, cells, boxes)
+    kw = dict(nu0=0.01, bc=sc.all_bc(dims, sc.PER), collision=(hip.MRT,), interp_method=interp)
+    o, s = Oracle(grid, **kw), hip.Solver(grid, precision=precision, **kw).build()
+    for l in range(grid.max_level + 1):
+        rho, u = sc.level_fields(grid, l, 0.05, noise=1e-3)
+        o.init_macro(l, rho, u)
+        s.init_macro(l, rho, u)
+    o.time_marching(6)
+    s.time_marching(6)
+    for l in range(grid.max_level + 1):
+        assert_close(s.f(l), o.f(l), rtol=0 if tol > 1e-10 else tol, atol=tol)
+
+
+def test_closure_workspace_sizes():
+    """Each call's result is that of a new solver, whatever the sizes before it: the sizes grow,
+    shrink and pass the largest workspace that is kept (64 MiB, 1.67M samples)."""
+    s = _ctx()
+    p = closure.init_params(3)
+    X, T = _data(1_700_000, seed=9)
+    for n in (100, 5000, 33, 1_700_000, 70000, 1):
+        loss, grad = s.mlp_gradient(p, X[:n], T[:n])
+        lref, gref = _ctx().mlp_gradient(p, X[:n], T[:n])
+        assert loss == lref
+        np.testing.assert_array_equal(grad, gref)
+        q, h = s.mlp_train(p, X[:n], T[:n], 2, 64, 1e-3, seed=5)
+        qr, hr = _ctx().mlp_train(p, X[:n], T[:n], 2, 64, 1e-3, seed=5)
+        np.testing.assert_array_equal(h, hr)
+        np.testing.assert_array_equal(q, qr)
+
+
+def test_calls_from_two_threads():
+    """Gradients and downloads of one solver from two threads at once take turns."""
+    s = _ctx()
+    p = closure.init_params(3)
+    X, T = _data(6000, seed=4)
+    want = {n: s.mlp_gradient(p, X[:n], T[:n]) for n in (500, 6000)}
+    bad = []
+
+    def run(n):
+        for _ in range(20):
+            loss, grad = s.mlp_gradient(p, X[:n], T[:n])
+            if loss != want[n][0] or not np.array_equal(grad, want[n][1]):
+                bad.append(n)
+
+    threads = [threading.Thread(target=run, args=(n,)) for n in want]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
