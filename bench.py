@@ -201,7 +201,7 @@ def main():
     ap.add_argument("--l2-every", type=int, default=100)
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--one-stream", action="store_true",
-                    help="time marching on one stream (levels do not overlap; for per-kernel traces)")
+                    help="accepted without effect (every launch is on one stream)")
     ap.add_argument("--no-graphs", action="store_true",
                     help="direct launches instead of replayed graphs of two background steps")
     ap.add_argument("--calibrate-copy", type=int, default=0, metavar="MIB",

@@ -103,9 +103,9 @@ __global__ __launch_bounds__(256) void k_c2f_sources(int64_t n_src, int64_t n_fb
 // a row) or of the fine level (~index: a fallback node); rows that several groups stage are
 // rescaled by each, a few hundred operations against a launch over all rows (4.8 us on small
 // levels, 10.8 on a 3M-node one) and their round trip through memory.  Otherwise (time
-// interpolation) a row of the table src_f.  A contributor is one 32-bit word {LDS row offset, FP16 weight}: the tensor-product
-// Lagrange weights are products of -1/16, 9/16, 1/2 and 1, dyadic rationals exact in FP16 (the
-// host checks every one).
+// interpolation) a row of the table src_f.  A contributor is one 32-bit word {LDS row offset, FP16
+// weight}: the tensor-product Lagrange weights are products of -1/16, 9/16, 1/2 and 1, dyadic
+// rationals exact in FP16 (the host checks every one).
 constexpr int kGatherDirs = 5;
 constexpr size_t kGatherLdsBudget = 20 * 1024;
 constexpr int kGatherMaxRows = 768;   // staged rows of one group (row offsets fit the word's 16 bits)

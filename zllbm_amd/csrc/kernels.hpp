@@ -80,8 +80,10 @@ __device__ __forceinline__ void store_nt(T v, T *dst) {
 // lbm_bounce_back.cpp:29-91).
 // Rows of 64 lanes for the directions that some lane's conditions set: one coalesced load per such
 // direction and no selection per lane, 5 of 19 directions (1.3 KB beside 4.9 KB of FP32
-// populations) in a brick on one face.  It replaces a launch per face (4.2-4.6 us each) and the
-// deferred collision of the boundary nodes (4-9 us): see k_stream_collide.
+// populations) in a brick on one face.  It replaces a launch per face and the deferred collision of
+// the boundary nodes.  One step's launches, before and with it: FP64 cavity 128^2 25.5 -> 4.7 us,
+// 97x80x66 FP32 Smagorinsky 57 -> 22.4 us, 128^3 BF16 82.7 -> 47.5 us.  A dense table of Q rows a
+// brick and a branch per direction in the pull measured 26.4 and 64.3 us for the last two.
 struct BoundaryPull {
     const int2 *brick;
     const int32_t *src;
@@ -802,18 +804,16 @@ __device__ __forceinline__ uint32_t pull_to_lds(const BrickLevel<T> &t, const T 
     return entry;
 }
 
-// The same with the FP32 learned closure.  Each workgroup stages the network's operand images
-// in LDS once (after its waves' first pulls are out); its four waves then take ROUNDS rounds of
-// four adjacent bricks (the host picks 1 or 2), and each wave pulls its next brick into LDS
-// while it collides the current one, so the pull's latency hides behind the network's
-// arithmetic at the occupancy its registers allow.  Within
-// a round the order is: read the staged brick, write deferred nodes' post-stream values, issue
-// the next pull, collide, store; the store group is unconditional so that the next round's wait
-// (in-order vector memory counter) covers the pull and not these stores.
-// Register budget: 4 waves per SIMD unforced, 3 forced (whose Guo terms would spill at 4).
+// The same with the FP32 learned closure.  Each workgroup stages the network's operand images in LDS
+// after its four waves' pulls are out, so that their latencies overlap; each wave then takes one
+// brick.  A wave that took a second brick, pulled while it collided the first, needed 13 more registers
+// and a workgroup twice as long: 37.2 against 33.6 us on 80^3 nodes, 88.5 / 83.7 on 120^3, 137.3 /
+// 137.0 on 144^3; 4 and 8 bricks were slower still.
+// Registers: 115-123 without forcing and 120-146 with it in D3Q19, 4 or 3 waves per SIMD (the Guo
+// terms would spill where 4 are forced).
 // BND: the level has resolved boundary nodes (its own variant: on the other levels the table's two
-// pointers would cost the loop scalar spills, 130.1 against 128.9 us on a 3M-node level).
-template <int D, typename T, typename C, bool SHIFT, int COLL, int VAR, int ROUNDS, bool BND>
+// pointers cost scalar registers, 130.1 against 128.9 us on a 3M-node level).
+template <int D, typename T, typename C, bool SHIFT, int COLL, int VAR, bool BND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((VAR & 1) ? 3 : 4)))
 void k_stream_collide_mlp(Batch<FusedRun<T>> B) {
     static_assert(mlp_on_mfma<C, VAR>(), "kernel of the FP32 learned closure");
@@ -829,87 +829,65 @@ void k_stream_collide_mlp(Batch<FusedRun<T>> B) {
     __shared__ MlpOps ops;
     __shared__ T stage[4][Q * kStageStride];
     __shared__ uint32_t who_s[4][64];        // aux_missing entries of the brick's recorded nodes, in order
-    constexpr int64_t per_group = 4 * ROUNDS;
-    const int64_t g = xcd_group((nbrick + per_group - 1) / per_group, blockIdx.x - B.first[run],
-                                B.first[run + 1] - B.first[run]);
+    const int64_t g = xcd_group((nbrick + 3) / 4, blockIdx.x - B.first[run], B.first[run + 1] - B.first[run]);
     if (g < 0) return;                       // uniform per workgroup: before the barrier
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     T *buf = stage[wave];
-    int64_t b = g * per_group + wave;
-    // the first pull goes out before the network is staged, so that their latencies overlap
+    const int64_t b = g * 4 + wave;
     uint32_t *who = who_s[wave];
     uint32_t entry = 0;
-    if (b < nbrick) entry = pull_to_lds<D, T, BND>(t, fin, b, threadIdx.x & 63, buf);
+    if (b < nbrick) entry = pull_to_lds<D, T, BND>(t, fin, b, lane, buf);
     stage_mlp_ops<((VAR & 15) >> 1) == 4, mrt_on_mfma<C, VAR>()>(ops, p.mlp->ops);
     if (b >= nbrick) return;                 // uniform per wave; no barrier follows
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the first pull has landed
-#pragma unroll 1
-    for (int r = 0; r < ROUNDS; ++r) {
-        // the pull into buf has landed: the compiler does not order LDS reads after direct-to-LDS
-        // loads of an earlier iteration.  In-order counter: the last Q vector memory operations
-        // before this point are the previous round's stores, which may stay in flight.
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Q) : "memory");
-        int lane = threadIdx.x & 63;
-        // opaque per brick: keeps the lane's stencil offsets from being hoisted out of the loop
-        asm volatile("" : "+v"(lane));
-        C f[Q];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the pull has landed
+    C f[Q];
 #pragma unroll
-        for (int q = 0; q < Q; ++q) f[q] = C(buf[q * kStageStride + lane]);
-        const bool has_node = (table_load(t.occ, b) >> lane) & 1ull;
-        const uint64_t am = table_load(t.auxmask, b);
-        if (am) {   // uniform
-            // recorded nodes: post-stream values to their aux rows, except the missing sources (their
-            // boundary / transfer values are there already).  The rows of a brick's nodes are one
-            // run of memory: the wavefront writes it in 16-byte units from the staged brick, so
-            // every store is whole lines (a row per lane took 147 us on a 3M-node level, this 134)
-            if ((am >> lane) & 1ull) who[__popcll(am & ((1ull << lane) - 1ull))] = entry;
-            wave_lds_sync();
-            const int64_t base = table_load(t.auxbase, b);
-            constexpr int U = aux_stride<D>() / 4;
-            const int units = (int)__popcll(am) * U;
-            for (int u0 = 0; u0 < units; u0 += 64) {
-                const int u = u0 + lane;
-                if (u < units) {
-                    const int j = u / U, q0 = 4 * (u - j * U);
-                    const uint32_t w = who[j];
-                    const T *v = buf + (w & 63u);
-                    RowUnit<T> x;
+    for (int q = 0; q < Q; ++q) f[q] = C(buf[q * kStageStride + lane]);
+    const bool has_node = (table_load(t.occ, b) >> lane) & 1ull;
+    const uint64_t am = table_load(t.auxmask, b);
+    if (am) {   // uniform
+        // recorded nodes: post-stream values to their aux rows, except the missing sources (their
+        // boundary / transfer values are there already).  The rows of a brick's nodes are one
+        // run of memory: the wavefront writes it in 16-byte units from the staged brick, so
+        // every store is whole lines (a row per lane took 147 us on a 3M-node level, this 134)
+        if ((am >> lane) & 1ull) who[__popcll(am & ((1ull << lane) - 1ull))] = entry;
+        wave_lds_sync();
+        const int64_t base = table_load(t.auxbase, b);
+        constexpr int U = aux_stride<D>() / 4;
+        const int units = (int)__popcll(am) * U;
+        for (int u0 = 0; u0 < units; u0 += 64) {
+            const int u = u0 + lane;
+            if (u < units) {
+                const int j = u / U, q0 = 4 * (u - j * U);
+                const uint32_t w = who[j];
+                const T *v = buf + (w & 63u);
+                RowUnit<T> x;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) x.v[k] = v[(q0 + k < Q ? q0 + k : 0) * kStageStride];
-                    T *dst = aux_f + (base + j) * aux_stride<D>() + q0;
-                    const uint32_t m = (w >> 6) >> q0 & 15u;
-                    if (m == 0u) {
-                        *reinterpret_cast<RowUnit<T> *>(dst) = x;
-                    } else {
+                for (int k = 0; k < 4; ++k) x.v[k] = v[(q0 + k < Q ? q0 + k : 0) * kStageStride];
+                T *dst = aux_f + (base + j) * aux_stride<D>() + q0;
+                const uint32_t m = (w >> 6) >> q0 & 15u;
+                if (m == 0u) {
+                    *reinterpret_cast<RowUnit<T> *>(dst) = x;
+                } else {
 #pragma unroll
-                        for (int k = 0; k < 4; ++k)
-                            if (!(m >> k & 1u)) dst[k] = x.v[k];
-                    }
+                    for (int k = 0; k < 4; ++k)
+                        if (!(m >> k & 1u)) dst[k] = x.v[k];
                 }
             }
         }
-        // the buffer's reads have returned before it is refilled
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        const int64_t bn = b + 4;
-        const bool more = r + 1 < ROUNDS && bn < nbrick;
-        uint32_t entry_next = 0;
-        if (more) entry_next = pull_to_lds<D, T, BND>(t, fin, bn, lane, buf);
-        if (!has_node) {
-#pragma unroll
-            for (int q = 0; q < Q; ++q) f[q] = C(0);          // rest state (shifted storage)
-        }
-        C F[3] = {C(p.const_force[0]), C(p.const_force[1]), C(p.const_force[2])};
-        C rho, u[3];
-        collide<D, SHIFT, COLL, C, VAR>(f, F, p, rho, u, &ops);
-        // every lane stores: empty slots are never read, and deferred slots are rewritten by the
-        // next substep's aux collision before the fused kernel reads them
-        T *__restrict__ dst = fout + b * Q * 64 + lane;
-#pragma unroll
-        for (int q = 0; q < Q; ++q) store_nt(T(f[q]), dst + q * 64);
-        if (!more) break;
-        b = bn;
-        entry = entry_next;
     }
+    if (!has_node) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) f[q] = C(0);          // rest state (shifted storage)
+    }
+    C F[3] = {C(p.const_force[0]), C(p.const_force[1]), C(p.const_force[2])};
+    C rho, u[3];
+    collide<D, SHIFT, COLL, C, VAR>(f, F, p, rho, u, &ops);
+    // every lane stores: empty slots are never read, and deferred slots are rewritten by the
+    // next substep's aux collision before the fused kernel reads them
+    T *__restrict__ dst = fout + b * Q * 64 + lane;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) store_nt(T(f[q]), dst + q * 64);
 }
 
 // Collision of the aux nodes of the levels of a batch (deferred from the previous substep), writing post-collision

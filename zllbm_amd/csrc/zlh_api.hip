@@ -543,7 +543,6 @@ struct zlh_ctx {
     DevBuf mlp_d;           // MlpDev of the learned closure
     bool mlp_set = false;
     int mlp_train_form = ZLH_MLP_FP32;   // kernel of zlh_mlp_gradient / zlh_mlp_train
-    int n_cu = 0;           // compute units of the context's device
     int device = 0;         // the device the context was created on
     float *scratch_addr = nullptr;   // that device's address of the static no-allocation array
     // two background steps captured as one graph, per combination of the levels' buffer
@@ -735,41 +734,16 @@ unsigned lay_out(Batch<FusedRun<T>> &B, int per) {
     return B.first[B.n];
 }
 
-// learned-closure kernel with R rounds of four bricks per workgroup
-template <int D, typename T, typename C, bool SHIFT, int COLL, int V, int R, bool BND>
-void launch_mlp_rounds(zlh_ctx *ctx, Batch<FusedRun<T>> &B) {
-    const unsigned grid = lay_out(B, 4 * R);
-    hipLaunchKernelGGL((k_stream_collide_mlp<D, T, C, SHIFT, COLL, V, R, BND>), dim3(grid), dim3(256), 0, ctx->stream, B);
-}
-
-// one round per workgroup while the grid is at most two waves of resident workgroups (the
-// latency of a short grid is one brick's), two on larger levels (each wave's second pull then
-// overlaps its first brick's network; more rounds measured slower on a 3M-node level)
+// learned-closure kernel
 template <int D, typename T, typename C, bool SHIFT, int COLL, int V>
 void launch_mlp(zlh_ctx *ctx, Batch<FusedRun<T>> &B) {
-    static int per_cu = [] {
-        int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_stream_collide_mlp<D, T, C, SHIFT, COLL, V, 1, false>, 256, 0) !=
-                hipSuccess || n < 1)
-            n = 1;
-        return n;
-    }();
-    const int64_t resident = (int64_t)per_cu * ctx->n_cu;
     bool bnd = false;
-    int64_t groups = 0;
-    for (int i = 0; i < B.n; ++i) {
-        bnd |= B.run[i].lv.bnd.brick != nullptr;
-        groups += (B.run[i].lv.nbrick + 3) / 4;
-    }
-    const bool one = groups <= 2 * resident;
-    if (bnd) {
-        if (one) launch_mlp_rounds<D, T, C, SHIFT, COLL, V, 1, true>(ctx, B);
-        else launch_mlp_rounds<D, T, C, SHIFT, COLL, V, 2, true>(ctx, B);
-    } else if (one) {
-        launch_mlp_rounds<D, T, C, SHIFT, COLL, V, 1, false>(ctx, B);
-    } else {
-        launch_mlp_rounds<D, T, C, SHIFT, COLL, V, 2, false>(ctx, B);
-    }
+    for (int i = 0; i < B.n; ++i) bnd |= B.run[i].lv.bnd.brick != nullptr;
+    const unsigned grid = lay_out(B, 4);
+    if (bnd)
+        hipLaunchKernelGGL((k_stream_collide_mlp<D, T, C, SHIFT, COLL, V, true>), dim3(grid), dim3(256), 0, ctx->stream, B);
+    else
+        hipLaunchKernelGGL((k_stream_collide_mlp<D, T, C, SHIFT, COLL, V, false>), dim3(grid), dim3(256), 0, ctx->stream, B);
 }
 
 // bulk kernel variant: collision operator x (sub-grid model, forcing)
@@ -1456,9 +1430,7 @@ zlh_status zlh_create(const zlh_solver_desc *desc, zlh_ctx **out) {
     for (hipEvent_t &e : ctx->ev_stage)
         if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return ZLH_EDEVICE;
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&ctx->n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ctx->n_cu < 1)
-        return ZLH_EDEVICE;
+    if (hipGetDevice(&dev) != hipSuccess) return ZLH_EDEVICE;
     ctx->device = dev;
     if (scratch_setup(ctx.get())) return ZLH_EDEVICE;
     if (dalloc(ctx.get(), ctx->mlp_d, sizeof(MlpDev))) return ZLH_ENOMEM;
@@ -1487,8 +1459,7 @@ zlh_status zlh_max_level_bricks(const zlh_solver_desc *desc, int64_t *max_bricks
     // slot and aux indices are 32-bit: 64 nbrick 19 < 2^31
     int64_t m = (((int64_t)1 << 31) / 19 - 1) / 64;
     // the FP32 learned closure's fused kernel pulls through 32-bit byte offsets
-    // nbrick Q 64 4 (pull_to_lds in kernels.hpp) and stores deferred nodes through 32-bit byte
-    // offsets up to Q naux 4 <= nbrick Q 256: nbrick Q 256 < 2^32
+    // (pull_to_lds in kernels.hpp): nbrick Q 256 < 2^32
     if (desc->les == ZLH_LES_MLP && desc->precision == ZLH_FP32_SHIFTED) {
         const int64_t q = desc->dims == 2 ? 9 : 19;
         m = std::min<int64_t>(m, (((int64_t)1 << 32) - 1) / (q * 64 * 4));
