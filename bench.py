@@ -46,10 +46,10 @@ MLP_OPERANDS = "fp16"
 # what they read for a plain 1 GiB copy (bytes = 2.0 x FETCH_SIZE + 1.0 x WRITE_SIZE); the
 # summaries, with their commands, are the named files under profiles/
 PROFILED_TRAFFIC = {
-    ("amr4", "mrt", "fp32", "fp16"): (580.5e6, "profiles/k_stream_collide_mlp_amr4.md"),
-    ("tgv256", "mrt", "fp32", None): (2884.4e6, "profiles/k_stream_collide_tgv256.md"),
-    ("tgv256", "mrt", "bf16", None): (1492.6e6, "profiles/k_stream_collide_bf16_tgv256.md"),
-    ("sphere5", "mrt", "fp32", "fp16"): (82.8e6, "profiles/k_ib_sphere5.md"),
+    ("amr4", "mrt", "fp32", "fp16"): (555.0e6, "profiles/k_stream_collide_mlp_amr4.md"),
+    ("tgv256", "mrt", "fp32", None): (2946.5e6, "profiles/k_stream_collide_tgv256.md"),
+    ("tgv256", "mrt", "bf16", None): (1539.8e6, "profiles/k_stream_collide_bf16_tgv256.md"),
+    ("sphere5", "mrt", "fp32", "fp16"): (83.3e6, "profiles/k_ib_sphere5.md"),
 }
 
 
