@@ -60,7 +60,7 @@ __device__ __forceinline__ void rescale_row(T *row, double tau_ratio, int compre
     }
 }
 
-// Time interpolation only: the rows of the interpolation as a table, [n_src + n_fb][S], the
+// Where row_table says so: the rows of the interpolation as a table, [n_src + n_fb][S], the
 // rescaled coarse sources and then plain copies of the fine nodes that stand in for missing coarse
 // ones.  MID (after an odd fine substep): each coarse row is the mean of the row computed now and
 // the row `prev` of the last synchronised transfer, i.e. of the coarse state before and after the
@@ -102,8 +102,8 @@ __global__ __launch_bounds__(256) void k_c2f_sources(int64_t n_src, int64_t n_fb
 // DIRECT: a staged row is an aux row, of the coarse level (index >= 0; rescaled in LDS, one thread
 // a row) or of the fine level (~index: a fallback node); rows that several groups stage are
 // rescaled by each, a few hundred operations against a launch over all rows (4.8 us on small
-// levels, 10.8 on a 3M-node one) and their round trip through memory.  Otherwise (time
-// interpolation) a row of the table src_f.  A contributor is one 32-bit word {LDS row offset, FP16
+// levels, 10.8 on a 3M-node one) and their round trip through memory.  Otherwise
+// (row_table) a row of the table src_f.  A contributor is one 32-bit word {LDS row offset, FP16
 // weight}: the tensor-product Lagrange weights are products of -1/16, 9/16, 1/2 and 1, dyadic
 // rationals exact in FP16 (the host checks every one).
 constexpr int kGatherDirs = 5;
@@ -690,14 +690,23 @@ inline bool exact_half_bits(double w, uint16_t *bits) {
     return true;
 }
 
-// the row tables of time interpolation (when it is switched on after the build: by the rows computed
-// then, before any step)
+// Whether an exchange forms its rows as a table in a launch of its own (k_c2f_sources) instead of in
+// the gather.  Time interpolation does, as the table keeps the earlier rows.  Of large exchanges FP64
+// does: its LDS holds half as many rows a group, so more are staged and rescaled twice.  Gather
+// (and table) in FP64: 147k rows 138 against 92 + 21 us, 37k rows 40.0 against 30.0 + 8.9, 13k rows
+// 18.6 against 14.4 + 6.7; FP32 on 147k rows 47 against 49 + 11.
+inline bool row_table(const zlh_ctx *ctx, const TransferTables &X) {
+    return ctx->time_interp || (ctx->fp64() && X.n_src + X.n_fb > 32768);
+}
+
+// the row tables (for time interpolation switched on after the build: by the rows computed then,
+// before any step)
 inline zlh_status reserve_row_tables(zlh_ctx *ctx, TransferTables &X) {
     const int64_t stride = ctx->d.dims == 2 ? aux_stride<2>() : aux_stride<3>();
     const size_t bytes = ctx->tsize() * stride * std::max<int64_t>(X.n_src + X.n_fb, 1);
     zlh_status s;
     if (!X.src_f.p && (s = dalloc(ctx, X.src_f, bytes))) return s;
-    if (!X.src_mid.p && (s = dalloc(ctx, X.src_mid, bytes))) return s;
+    if (ctx->time_interp && !X.src_mid.p && (s = dalloc(ctx, X.src_mid, bytes))) return s;
     return ZLH_OK;
 }
 
@@ -832,7 +841,7 @@ inline zlh_status upload_transfer(zlh_ctx *ctx, int level) {
     if ((s = upload(ctx, X.fb_fine_ai, fb_ai))) return s;
     X.src_f = DevBuf();
     X.src_mid = DevBuf();
-    if (ctx->time_interp && (s = reserve_row_tables(ctx, X))) return s;
+    if (row_table(ctx, X) && (s = reserve_row_tables(ctx, X))) return s;
     if ((s = upload(ctx, X.f2c_coarse_ai, f2c_c))) return s;
     if ((s = upload(ctx, X.f2c_fine_ai, f2c_f))) return s;
     {
@@ -951,8 +960,7 @@ zlh_status launch_transfers_t(zlh_ctx *ctx, int level, int parts) {
     const double dtc = 1. / (double)(1u << (level - 1)), dtf = 1. / (double)(1u << level);
     const double c2f = 0.5 * (nu * 3. / dtc * 2. + 0.5) / (nu * 3. / dtc + 0.5);
     const double f2c = 2. * (nu * 3. / dtf / 2 + 0.5) / (nu * 3. / dtf + 0.5);
-    // with time interpolation the rows go through a table, which keeps the earlier ones
-    const bool table = ctx->time_interp;
+    const bool table = row_table(ctx, X);
     const bool mid = (parts & kTransferMid) != 0;
     if (table && (parts & (kTransferC2F | kTransferRows)) && X.n_src + X.n_fb > 0) {
         const zlh_status s = reserve_row_tables(ctx, X);
