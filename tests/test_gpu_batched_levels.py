@@ -85,3 +85,18 @@ def test_marching_equals_substeps_3d_forced(les, precision):
     for l in range(2):
         np.testing.assert_array_equal(runs[0].f(l), runs[1].f(l))
     np.testing.assert_array_equal(runs[0].ib_force(1), runs[1].ib_force(1))
+
+
+@pytest.mark.parametrize("levels", [1, 2])
+@pytest.mark.parametrize("graphs", [True, False])
+def test_no_steps_without_a_closure(levels, graphs):
+    """Marching no step asks for nothing: it succeeds before the learned closure is set, on one
+    level and on several, and any step before that is refused."""
+    grid = g.uniform_grid(3, (6, 6, 6)) if levels == 1 else sc.amr3d()[0]
+    s = hip.Solver(grid, nu0=0.01, bc=sc.all_bc(3, sc.PER), collision=(hip.MRT,), les=hip.LES_MLP,
+                   precision=hip.FP32_SHIFTED).build()
+    s.graphs_enable(graphs)
+    s.time_marching(0)
+    with pytest.raises(RuntimeError, match="learned closure not set"):
+        s.time_marching(1)
+    s.time_marching(0)

@@ -1663,7 +1663,6 @@ namespace {
 // chain of launches.
 zlh_status march_launches(zlh_ctx *ctx, int nsteps) {
     const int top = ctx->d.max_level;
-    if (ctx->d.les == ZLH_LES_MLP && !ctx->mlp_set) return ctx->fail(ZLH_ESTATE, "learned closure not set (zlh_mlp_set)");
     zlh_status s;
     for (int t = 0; t < nsteps; ++t)
         for (int64_t sub = 0; sub < (int64_t)1 << top; ++sub) {
@@ -1710,6 +1709,8 @@ zlh_status zlh_time_marching(zlh_ctx *ctx, int nsteps) {
     if (!ctx) return ZLH_EINVAL;
     if (!ctx->built) return ctx->fail(ZLH_ESTATE, "not built");
     if (nsteps < 0) return ctx->fail(ZLH_EINVAL, "negative step count");
+    if (nsteps > 0 && ctx->d.les == ZLH_LES_MLP && !ctx->mlp_set)
+        return ctx->fail(ZLH_ESTATE, "learned closure not set (zlh_mlp_set)");
     // launch-bound multi-level steps replay captured graphs: of two background steps while two
     // remain (level 0's buffer index comes back to where it was), of one step for an odd last
     // one.  Timing (per-launch events) runs the launches directly, and so does a single level: its
