@@ -68,6 +68,14 @@ def test_small_and_ragged_2d(cells, names):
     _compare(g.uniform_grid(2, cells), names, 10)
 
 
+@pytest.mark.parametrize("cells", [62, 63, 64, 127, 128])
+@pytest.mark.parametrize("names", [("channel", "walls"), ("walls", "channel"), ("channel", "periodic")])
+def test_face_kernel_workgroups(cells, names):
+    """Faces of one node less, as many and one more than one and two workgroups of 64 (a face of
+    `cells` cells has cells + 1 nodes), in the launches per face."""
+    _compare(g.uniform_grid(2, (cells, cells)), names, 10, collision=(hip.MRT,))
+
+
 @pytest.mark.parametrize("precision", [hip.FP64, hip.FP32_SHIFTED])
 @pytest.mark.parametrize("names", [("periodic", "periodic", "periodic"), ("walls", "periodic", "walls"),
                                    ("periodic", "lid", "walls")])

@@ -381,11 +381,19 @@ struct BcIdx {
     int inv[8];
 };
 
+// The kernels of one face take a node per thread, and a wavefront's access to 64 rows is as many
+// lines as rows, so they are bound by how many lines a CU looks up: one wavefront a workgroup puts a
+// face of a few thousand nodes on 4 times as many CUs.  k_bc_nee in FP64, workgroups of 256 and of 64:
+// 65^2 nodes in 3D 6.3 and 4.8 us, 33^2 5.4 and 4.6; the steps around them (64^3 cells, six
+// such faces; 48 x 32 x 32, two) 70.5 and 60.8, 40.0 and 35.4 us.
+constexpr int kBcThreads = 64;
+
 // BoundaryBounceBack{2D,3D} (lbm_bounce_back.cpp:29-91): f[in] = f_collide[out] - 6 rho0 w (c.u_w)
 template <int D, typename T>
-__global__ void k_bc_bounce_back(int64_t nb, const int32_t *node_ai, const int32_t *node_slot, const T *fa,
-                                 T *aux_f, BcIdx idx, double rho0, double ux,
-                                 double uy, double uz) {
+__global__ __launch_bounds__(kBcThreads) void k_bc_bounce_back(int64_t nb, const int32_t *node_ai,
+                                                               const int32_t *node_slot, const T *fa, T *aux_f,
+                                                               BcIdx idx, double rho0, double ux, double uy,
+                                                               double uz) {
     using L = Lattice<D>;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nb) return;
@@ -399,7 +407,8 @@ __global__ void k_bc_bounce_back(int64_t nb, const int32_t *node_ai, const int32
 
 // BoundaryPeriodic{2D,3D} (lbm_periodic.cpp:22-133): incoming directions copied from the twin
 template <int D, typename T>
-__global__ void k_bc_periodic(int64_t nb, const int32_t *node_ai, const int32_t *twin_ai, T *aux_f, BcIdx idx) {
+__global__ __launch_bounds__(kBcThreads) void k_bc_periodic(int64_t nb, const int32_t *node_ai, const int32_t *twin_ai,
+                                                            T *aux_f, BcIdx idx) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nb) return;
     const int64_t ai = node_ai[t], tj = twin_ai[t];
@@ -411,9 +420,9 @@ __global__ void k_bc_periodic(int64_t nb, const int32_t *node_ai, const int32_t 
 // BoundaryNonEqExtrapolation{2D,3D} (lbm_noneq_extrapolation.cpp:29-144):
 // f = feq(rho0, u_b) + f(inner) - feq(rho, u of inner)
 template <int D, typename T, typename C, bool SHIFT>
-__global__ void k_bc_nee(int64_t nb, const int32_t *node_ai, const int32_t *inner_ai, T *aux_f,
-                         const double *aux_force, StepParams p, double rho0, double ux, double uy, double uz,
-                         const double *ub_node) {
+__global__ __launch_bounds__(kBcThreads) void k_bc_nee(int64_t nb, const int32_t *node_ai, const int32_t *inner_ai,
+                                                       T *aux_f, const double *aux_force, StepParams p, double rho0,
+                                                       double ux, double uy, double uz, const double *ub_node) {
     constexpr int Q = Lattice<D>::Q;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nb) return;
@@ -860,21 +869,21 @@ zlh_status launch_step_kernels(zlh_ctx *ctx, const int *levels, int n, int coll)
             if (L.bc_n[dir] == 0) continue;
             const BcIdx idx = bc_indices(dims, dir);
             const double *bv = ctx->d.bc_value[dir];
+            const dim3 grid(blocks(L.bc_n[dir], kBcThreads)), block(kBcThreads);
             switch (ctx->d.bc_scheme[dir]) {
                 case ZLH_BC_BOUNCE_BACK:
-                    hipLaunchKernelGGL((k_bc_bounce_back<D, T>), dim3(blocks(L.bc_n[dir])), dim3(256), 0, ctx->stream,
-                                       L.bc_n[dir], L.bc_ai_d[dir].as<int32_t>(), L.bc_slot_d[dir].as<int32_t>(), fa,
-                                       aux_f, idx, ctx->d.rho0, bv[0], bv[1], bv[2]);
+                    hipLaunchKernelGGL((k_bc_bounce_back<D, T>), grid, block, 0, ctx->stream, L.bc_n[dir],
+                                       L.bc_ai_d[dir].as<int32_t>(), L.bc_slot_d[dir].as<int32_t>(), fa, aux_f, idx,
+                                       ctx->d.rho0, bv[0], bv[1], bv[2]);
                     break;
                 case ZLH_BC_PERIODIC:
-                    hipLaunchKernelGGL((k_bc_periodic<D, T>), dim3(blocks(L.bc_n[dir])), dim3(256), 0, ctx->stream,
-                                       L.bc_n[dir], L.bc_ai_d[dir].as<int32_t>(), L.bc_partner_d[dir].as<int32_t>(),
-                                       aux_f, idx);
+                    hipLaunchKernelGGL((k_bc_periodic<D, T>), grid, block, 0, ctx->stream, L.bc_n[dir],
+                                       L.bc_ai_d[dir].as<int32_t>(), L.bc_partner_d[dir].as<int32_t>(), aux_f, idx);
                     break;
                 case ZLH_BC_NEE:
-                    hipLaunchKernelGGL((k_bc_nee<D, T, C, SHIFT>), dim3(blocks(L.bc_n[dir])), dim3(256), 0, ctx->stream,
-                                       L.bc_n[dir], L.bc_ai_d[dir].as<int32_t>(), L.bc_partner_d[dir].as<int32_t>(),
-                                       aux_f, aux_force, L.sp, ctx->d.rho0, bv[0], bv[1], bv[2],
+                    hipLaunchKernelGGL((k_bc_nee<D, T, C, SHIFT>), grid, block, 0, ctx->stream, L.bc_n[dir],
+                                       L.bc_ai_d[dir].as<int32_t>(), L.bc_partner_d[dir].as<int32_t>(), aux_f, aux_force,
+                                       L.sp, ctx->d.rho0, bv[0], bv[1], bv[2],
                                        L.bc_u_d[dir].p ? L.bc_u_d[dir].as<double>() : nullptr);
                     break;
                 default:
