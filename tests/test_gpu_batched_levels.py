@@ -100,3 +100,21 @@ def test_no_steps_without_a_closure(levels, graphs):
     with pytest.raises(RuntimeError, match="learned closure not set"):
         s.time_marching(1)
     s.time_marching(0)
+
+
+# a single level with launches per face: replayed graphs below 32 MiB of populations, launches above
+# (512 x 511 nodes of 9 FP64 values are 18 MiB, 705 x 706 are 35 with the padding of their bricks)
+@pytest.mark.parametrize("cells", [(7, 9), (511, 510), (704, 705)])
+def test_single_level_channel_as_graphs_and_launches(cells):
+    grid = g.uniform_grid(2, cells)
+    bc = {g.XMIN: (sc.NEE, (0.03, 0.)), g.XMAX: (sc.NEE, (0.03, 0.)), g.YMIN: (sc.BB, (0., 0.)), g.YMAX: (sc.BB, (0.02, 0.))}
+    runs = []
+    for graphs in (True, False):
+        s = hip.Solver(grid, nu0=0.02, bc=bc, collision=(hip.MRT,)).build()
+        s.graphs_enable(graphs)
+        s.init_macro(0, *sc.level_fields(grid, 0, u0=0.02))
+        runs.append(s)
+    for n in (1, 2, 5, 4, 1, 3, 2):
+        for s in runs:
+            s.time_marching(n)
+        np.testing.assert_array_equal(runs[0].f(0), runs[1].f(0))

@@ -1710,6 +1710,27 @@ zlh_status capture_steps(zlh_ctx *ctx, int nsteps, hipGraphExec_t *exec) {
     return ZLH_OK;
 }
 
+// Whether a single level's steps go out as launches instead of as graphs.  The host takes 3 to 4 us
+// a launch; a graph launch of two steps takes it 16 us, and the device starts each of its kernels
+// sooner.
+//  * Without launches per face a step is one to three launches: a 128^2 FP64 cavity takes 5.8 us a
+//    step directly and 8.2 as graphs, one step waited for 15 and 36.
+//  * With them it is six (D2Q9) or eight.  The host is the slower side up to about 64 MB of
+//    populations in both buffers; us a step, directly / as graphs: 48 x 24 FP32 24 / 17.2, 512^2 FP64
+//    (38 MB) 29.8 / 28.2, 64^3 FP32 (42 MB) 46.0 / 43.6, 96 x 64^2 FP32 (62 MB) 49.5 / 48.6, 1024^2 FP32
+//    (75 MB) 36.0 / 36.5, 64^3 FP64 (84 MB) 55.2 / 56.5, 1024^2 FP64 47.2 / 50.1, 128 x 96^2 BF16 (92 MB)
+//    60.0 / 62.1.
+//  * A call of one step has no second launch to hide behind: at six launches 28.6 / 34, at eight 46 to
+//    64 / 42.8.
+bool launch_directly(const zlh_ctx *ctx, int nsteps) {
+    if (ctx->d.max_level > 0) return false;   // refined: 83 / 74 us for 7 substeps of three small levels
+    const LevelState &L = ctx->lv[0];
+    int faces = 0;
+    if (!L.resolved)
+        for (int dir = 1; dir <= 2 * ctx->d.dims; ++dir) faces += L.bc_n[dir] > 0;
+    return faces == 0 || L.f_d[0].bytes >= (size_t)32 << 20 || (nsteps == 1 && faces <= 4);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1720,14 +1741,10 @@ zlh_status zlh_time_marching(zlh_ctx *ctx, int nsteps) {
     if (nsteps < 0) return ctx->fail(ZLH_EINVAL, "negative step count");
     if (nsteps > 0 && ctx->d.les == ZLH_LES_MLP && !ctx->mlp_set)
         return ctx->fail(ZLH_ESTATE, "learned closure not set (zlh_mlp_set)");
-    // launch-bound multi-level steps replay captured graphs: of two background steps while two
-    // remain (level 0's buffer index comes back to where it was), of one step for an odd last
-    // one.  Timing (per-launch events) runs the launches directly, and so does a single level: its
-    // few launches take the host less time each (about 4.8 us a step with resolved boundaries) than
-    // the device, while a graph launch takes 16 us for two steps (a 128^2 FP64 cavity: 5.8 against
-    // 8.2 us a step; one step waited for: 15 against 36 us).  A 7-substep step of three small levels
-    // takes 83 us launched directly and 74 as a graph.
-    if (!ctx->use_graphs || ctx->timing || ctx->d.max_level == 0) return march_launches(ctx, nsteps);
+    // launch-bound steps replay captured graphs: of two background steps while two remain (level
+    // 0's buffer index comes back to where it was), of one step for an odd last one.  Timing
+    // (per-launch events) runs the launches directly.
+    if (!ctx->use_graphs || ctx->timing || launch_directly(ctx, nsteps)) return march_launches(ctx, nsteps);
     int t = 0;
     while (t < nsteps) {
         const int n = nsteps - t >= 2 ? 2 : 1;
