@@ -81,3 +81,38 @@ def test_calls_from_two_threads():
     for t in threads:
         t.join()
     assert not bad
+
+
+# rows of more than 32,768 nodes: FP64 in 3D forms them as a table in a launch of its own (k_c2f_sources),
+# in 2D the gather stages them itself, as every smaller exchange does
+LARGE = {
+    "3d": lambda: g.refined_box_grid(3, (62, 62, 62), [((5, 5, 5), (57, 57, 57))]),
+    "2d": lambda: g.refined_mask_grid(2, (400, 400), 2, lambda k, c: np.floor(c / 14).sum(1) % 2 == 0, buffer=0),
+}
+
+
+@pytest.mark.parametrize("name", sorted(LARGE))
+def test_large_fp64_exchange(name):
+    """Against the oracle; then time interpolation on and off again (its second table is made at the
+    switch), each against a solver that was built so and starts from the same populations."""
+    grid = LARGE[name]()
+    kw = dict(nu0=0.01, bc=sc.all_bc(grid.dims, sc.PER), collision=(hip.MRT,))
+    o, s = Oracle(grid, **kw), hip.Solver(grid, **kw).build()
+    assert s.transfer_info(1)["source_rows"] > 32768
+    for l in range(2):
+        rho, u = sc.level_fields(grid, l, 0.05, noise=1e-3)
+        o.init_macro(l, rho, u)
+        s.init_macro(l, rho, u)
+    o.time_marching(3)
+    s.time_marching(3)
+    for l in range(2):
+        assert_close(s.f(l), o.f(l))
+    for on in (True, False):
+        s.set_time_interpolation(on)
+        r = hip.Solver(grid, time_interp=on, **kw).build()
+        for l in range(2):
+            r.set_f(l, s.f(l))
+        s.time_marching(2)
+        r.time_marching(2)
+        for l in range(2):
+            np.testing.assert_array_equal(r.f(l), s.f(l))

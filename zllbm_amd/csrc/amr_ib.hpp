@@ -691,12 +691,14 @@ inline bool exact_half_bits(double w, uint16_t *bits) {
 }
 
 // Whether an exchange forms its rows as a table in a launch of its own (k_c2f_sources) instead of in
-// the gather.  Time interpolation does, as the table keeps the earlier rows.  Of large exchanges FP64
-// does: its LDS holds half as many rows a group, so more are staged and rescaled twice.  Gather
+// the gather.  Time interpolation does, as the table keeps the earlier rows.  Of large D3Q19 exchanges
+// FP64 does: its LDS holds half as many rows a group, so more are staged and rescaled twice.  Gather
 // (and table) in FP64: 147k rows 138 against 92 + 21 us, 37k rows 40.0 against 30.0 + 8.9, 13k rows
-// 18.6 against 14.4 + 6.7; FP32 on 147k rows 47 against 49 + 11.
+// 18.6 against 14.4 + 6.7; FP32 on 147k rows 47 against 49 + 11.  D2Q9 rows are 96 bytes and few are
+// shared: a step of 4M fine nodes around 613 refined squares (190k source rows) takes 446 us without the
+// table and 466 with it, three nested boxes of a 256 x 192 channel 64 and 70.
 inline bool row_table(const zlh_ctx *ctx, const TransferTables &X) {
-    return ctx->time_interp || (ctx->fp64() && X.n_src + X.n_fb > 32768);
+    return ctx->time_interp || (ctx->fp64() && ctx->d.dims == 3 && X.n_src + X.n_fb > 32768);
 }
 
 // the row tables (for time interpolation switched on after the build: by the rows computed then,

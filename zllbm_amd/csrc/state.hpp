@@ -56,9 +56,9 @@ struct TransferTables {
     int64_t n_fb = 0;           // fine nodes standing in for missing coarse sources
     DevBuf src_coarse_ai;       // [n_src] coarse aux index of each source row (ascending)
     DevBuf fb_fine_ai;          // [n_fb] fine aux index of each fallback row (ascending)
-    // time interpolation only (allocated when it is on): the rescaled coarse rows, then fallback
-    // copies, [n_src + n_fb][S] in storage form, as of the last synchronised transfer, and the rows
-    // of a time-interpolated refill (coarse rows: mean of src_f and the current ones)
+    // where row_table says so: the rescaled coarse rows, then fallback copies, [n_src + n_fb][S] in
+    // storage form, as of the last synchronised transfer; with time interpolation also the rows of a
+    // time-interpolated refill (coarse rows: mean of src_f and the current ones)
     DevBuf src_f, src_mid;
     DevBuf f2c_coarse_ai;       // [n_f2c]
     DevBuf f2c_fine_ai;         // [n_f2c] fine aux index of the coincident node
