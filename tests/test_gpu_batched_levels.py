@@ -118,3 +118,50 @@ def test_single_level_channel_as_graphs_and_launches(cells):
         for s in runs:
             s.time_marching(n)
         np.testing.assert_array_equal(runs[0].f(0), runs[1].f(0))
+
+
+def _every_substep_order(s, top):
+    """The reference's order with time interpolation: an exchange after every substep."""
+    count = [0] * (top + 1)
+
+    def step(l):
+        count[l] += 1
+        s.step_level(l, count[l])
+        if l > 0:
+            s.transfer_levels(l)
+        if l < top:
+            step(l + 1)
+            step(l + 1)
+    step(0)
+
+
+# the finest region keeps only the 3 cells to level 1's edge that it needs, so the exchange with level 2
+# touches level-1 nodes that the exchange with level 1 touches
+def _overlapping():
+    return g.refined_mask_grid(2, (24, 24), 3, lambda k, c: np.ones(len(c), bool), margin=3, buffer=0)
+
+
+@pytest.mark.parametrize("graphs", [True, False])
+@pytest.mark.parametrize("precision", [hip.FP64, hip.FP32_SHIFTED, hip.BF16_SHIFTED])
+@pytest.mark.parametrize("time_interp", [False, True])
+@pytest.mark.parametrize("scheme", [sc.BB, sc.PER])
+@pytest.mark.parametrize("overlap", [True, False])
+def test_exchanges_keep_the_reference_order(overlap, scheme, time_interp, precision, graphs):
+    """Exchanges that share nodes, and (with time interpolation) several exchanges after one batch of
+    steps, against one launch per level in the reference's order."""
+    grid = _overlapping() if overlap else _nested(4)
+    top = grid.max_level
+    kw = dict(nu0=0.02, bc=sc.all_bc(2, scheme), collision=(hip.MRT,), precision=precision, time_interp=time_interp)
+    a, b = hip.Solver(grid, **kw).build(), hip.Solver(grid, **kw).build()
+    assert a.transfer_info(1)["overlaps_finer_transfer"] == overlap
+    a.graphs_enable(graphs)
+    for l in range(top + 1):
+        rho, u = sc.level_fields(grid, l, 0.05, noise=1e-3)
+        for s in (a, b):
+            s.init_macro(l, rho, u)
+    for n in (1, 3, 2):
+        a.time_marching(n)
+        for _ in range(n):
+            (_every_substep_order if time_interp else _reference_order)(b, top)
+        for l in range(top + 1):
+            np.testing.assert_array_equal(a.f(l), b.f(l))

@@ -4,7 +4,7 @@ uploaded values and the oracle."""
 import numpy as np
 import pytest
 
-from oracle.zlbm_oracle import Oracle
+from oracle.zlbm_oracle import Oracle, lattice
 from zllbm_amd import grid as g
 from zllbm_amd import hip
 from tests import scenarios as sc
@@ -57,5 +57,34 @@ def test_downloads_after_steps(precision):
         assert_close(f, o.f(0))
     rho_s, u_s = s.macros(0)
     rho_h, u_h = _macros(f, C2)
+    np.testing.assert_array_equal(rho_s, rho_h)
+    np.testing.assert_array_equal(u_s, u_h)
+
+
+# 2D: 231 x 225 nodes are 2 chunks of macros; 3D: 41 x 43 x 40 are 11 of populations and 3 of macros
+# (32,768 nodes), each with nodes whose pull the boundary conditions resolve in every chunk
+@pytest.mark.parametrize("precision", [hip.FP64, hip.FP32_SHIFTED, hip.BF16_SHIFTED])
+@pytest.mark.parametrize("cells", [(230, 224), (40, 42, 39)])
+def test_macros_of_many_chunks_after_steps(cells, precision):
+    """Macros are the sums of the populations, which (FP64) are the oracle's."""
+    dims = len(cells)
+    grid = g.uniform_grid(dims, cells)
+    bc = sc.all_bc(dims, sc.BB)
+    bc[g.XMIN] = bc[g.XMAX] = (sc.PER, (0., 0., 0.))
+    bc[g.YMAX] = (sc.BB, (0.03, 0., 0.))
+    kw = dict(nu0=0.02, bc=bc, collision=(hip.MRT,))
+    s = hip.Solver(grid, precision=precision, **kw).build()
+    rho, u = sc.level_fields(grid, 0, 0.05, noise=1e-3)
+    s.init_macro(0, rho, u)
+    s.time_marching(3)
+    f = s.f(0)
+    if precision == hip.FP64:
+        o = Oracle(grid, **kw)
+        o.init_macro(0, rho, u)
+        o.time_marching(3)
+        assert_close(f, o.f(0))
+    c = np.stack(lattice(dims)[:dims], 1)
+    rho_s, u_s = s.macros(0)
+    rho_h, u_h = _macros(f, c)
     np.testing.assert_array_equal(rho_s, rho_h)
     np.testing.assert_array_equal(u_s, u_h)

@@ -116,3 +116,56 @@ def test_large_fp64_exchange(name):
         r.time_marching(2)
         for l in range(2):
             np.testing.assert_array_equal(r.f(l), s.f(l))
+
+
+# BF16 rows are staged in units of 8 bytes.  A store rounds f - w by up to 2^-9 of itself; the bounds
+# are those of the refined BF16 runs of 10 and 12 steps
+@pytest.mark.parametrize("interp", [hip.INTERP_LAGRANGIAN, hip.INTERP_LINEAR])
+@pytest.mark.parametrize("box", sorted(BOXES))
+def test_exchange_bf16_tracks_fp64(box, interp):
+    dims, cells, boxes = BOXES[box]
+    grid = g.refined_box_grid(dims, cells, boxes)
+    kw = dict(nu0=0.01, bc=sc.all_bc(dims, sc.PER), collision=(hip.MRT,), interp_method=interp)
+    runs = [hip.Solver(grid, precision=p, **kw).build() for p in (hip.FP64, hip.BF16_SHIFTED)]
+    for s in runs:
+        for l in range(grid.max_level + 1):
+            s.init_macro(l, *sc.level_fields(grid, l, 0.05, noise=1e-3))
+        s.time_marching(6)
+    for l in range(grid.max_level + 1):
+        (rho, u), (rho_b, u_b) = (s.macros(l) for s in runs)
+        assert np.linalg.norm(u_b - u) < 6e-3 * np.linalg.norm(u)
+        assert np.sqrt(np.mean((rho_b - rho) ** 2)) < 2.5e-4
+
+
+def test_downloads_beside_gradients():
+    """Populations (7 staging chunks) and macros (2) from two threads while a third takes gradients:
+    the calls that share the staging buffer and the workspace take turns."""
+    grid = g.uniform_grid(3, (34, 35, 36))
+    s = hip.Solver(grid, nu0=0.02, bc=sc.all_bc(3, sc.PER), collision=(hip.MRT,)).build()
+    s.init_macro(0, *sc.level_fields(grid, 0, 0.05, noise=1e-3))
+    s.time_marching(3)
+    p = closure.init_params(3)
+    X, T = _data(6000, seed=4)
+    f, (rho, u), (loss, grad) = s.f(0), s.macros(0), s.mlp_gradient(p, X, T)
+    bad = []
+
+    def run(same):
+        for _ in range(15):
+            if not same():
+                bad.append(same)
+
+    def macros_same():
+        r, v = s.macros(0)
+        return np.array_equal(r, rho) and np.array_equal(v, u)
+
+    def gradient_same():
+        l, d = s.mlp_gradient(p, X, T)
+        return l == loss and np.array_equal(d, grad)
+
+    threads = [threading.Thread(target=run, args=(c,))
+               for c in (lambda: np.array_equal(s.f(0), f), macros_same, gradient_same)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
