@@ -193,7 +193,7 @@ __device__ __forceinline__ void gather_group(int64_t gi, unsigned char *lds_raw,
     }
     __syncthreads();
     if (!active) return;
-    // a contributor word is {row * QP (low 16 bits), FP16 weight (high 16 bits)}; the pad entry
+    // a contributor word is {row * S (low 16 bits), FP16 weight (high 16 bits)}; the pad entry
     // of the last part is summed like the others and never stored
     auto weight = [](uint32_t cw) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(cw >> 16)); };
     double acc[NQ];
@@ -859,18 +859,20 @@ inline zlh_status upload_transfer(zlh_ctx *ctx, int level) {
         std::set_intersection(src_ai.begin(), src_ai.end(), c.begin(), c.end(), std::back_inserter(common));
         X.f2c_apart &= common.empty();
     }
-    F.xfer_writes = tgt;
-    F.xfer_reads = fb_ai;
-    F.xfer_reads.insert(F.xfer_reads.end(), f2c_f.begin(), f2c_f.end());
     if (level - 1 >= 1) {
         // the coarse level's own transfer (from level - 2) against this one's coarse side: this
-        // one reads src_ai and writes f2c_c there
-        std::vector<uint8_t> mark(std::max<int64_t>(C.naux, 1), 0);   // 1 read, 2 written
-        for (int32_t i : C.xfer_reads) mark[i] |= 1;
-        for (int32_t i : C.xfer_writes) mark[i] |= 2;
+        // one reads its coarse sources and writes its fine-to-coarse targets there.  Only reported
+        // (zlh_transfer_info): every transfer runs in the reference's order
+        const TransferPlan &CP = C.xplan;
+        std::vector<uint8_t> mark(C.n, 0);   // 1 read, 2 written
+        for (int64_t c : CP.contrib)
+            if (c < 0) mark[-c - 1] |= 1;
+        for (int64_t i : CP.f2c_fine) mark[i] |= 1;
+        for (int64_t i : CP.tgt) mark[i] |= 2;
         C.xfer_overlap = false;
-        for (int32_t i : src_ai) C.xfer_overlap |= (mark[i] & 2) != 0;
-        for (int32_t i : f2c_c) C.xfer_overlap |= mark[i] != 0;
+        for (int64_t c : P.contrib)
+            if (c >= 0) C.xfer_overlap |= (mark[c] & 2) != 0;
+        for (int64_t j : P.f2c_coarse) C.xfer_overlap |= mark[j] != 0;
     }
     std::vector<uint8_t> macro_flag(std::max<int64_t>(F.naux, 1), 0);
     for (int32_t i : f2c_f) macro_flag[i] = 1;
@@ -887,31 +889,30 @@ inline zlh_status upload_ib(zlh_ctx *ctx, int level) {
     zlh_status s;
     T.support = P.support;
     T.stiffness = L.ib.stiffness;
-    std::vector<int32_t> ai(P.node.size(), -1), dup_ai(P.dup_node.size(), -1), reset;
+    std::vector<int32_t> ai(P.node.size(), -1), dup_ai(P.dup_node.size(), -1), supported;
     std::vector<uint8_t> seen(L.naux, 0);
     for (size_t k = 0; k < P.node.size(); ++k) {
         if (P.node[k] < 0) continue;
         ai[k] = L.node_aux_h[P.node[k]];
         if (ai[k] < 0) return ctx->fail(ZLH_EDEVICE, "immersed boundary node not deferred");
-        if (!seen[ai[k]]) { seen[ai[k]] = 1; reset.push_back(ai[k]); }
+        if (!seen[ai[k]]) { seen[ai[k]] = 1; supported.push_back(ai[k]); }
     }
-    // duplicates on periodic planes are reset and receive spread terms, but interpolate nothing
+    // duplicates on periodic planes receive spread terms, but interpolate nothing
     for (size_t k = 0; k < P.dup_node.size(); ++k) {
         dup_ai[k] = L.node_aux_h[P.dup_node[k]];
         if (dup_ai[k] < 0) return ctx->fail(ZLH_EDEVICE, "immersed boundary node not deferred");
-        if (!seen[dup_ai[k]]) { seen[dup_ai[k]] = 1; reset.push_back(dup_ai[k]); }
+        if (!seen[dup_ai[k]]) { seen[dup_ai[k]] = 1; supported.push_back(dup_ai[k]); }
     }
-    // supported nodes in aux order, so the reset's and the spread's row accesses coalesce
-    std::sort(reset.begin(), reset.end());
-    T.n_reset = (int64_t)reset.size();
+    // supported nodes in aux order, as the aux collision takes them
+    std::sort(supported.begin(), supported.end());
     // node-major view of the marker table for the spread: the entries naming each supported
     // node, in ascending entry (marker) order
     if (ai.size() >= ((size_t)1 << 31)) return ctx->fail(ZLH_ENOMEM, "immersed boundary table too large");
     // each term's marker and coefficient weight x area / (dt dx^(dims-1)) (the same double
     // product the marker-major form forms), in ascending marker order per node
-    std::vector<int32_t> pos(L.naux, -1), begin(reset.size() + 1, 0), marker;
+    std::vector<int32_t> pos(L.naux, -1), begin(supported.size() + 1, 0), marker;
     std::vector<double> coef;
-    for (size_t r = 0; r < reset.size(); ++r) pos[reset[r]] = (int32_t)r;
+    for (size_t r = 0; r < supported.size(); ++r) pos[supported[r]] = (int32_t)r;
     // terms: (node, marker, table entry) of every stencil entry and every duplicate, ordered by
     // marker per node (a node takes at most one term per marker)
     struct Term { int32_t a; int64_t m, k; };
@@ -922,7 +923,7 @@ inline zlh_status upload_ib(zlh_ctx *ctx, int level) {
         terms.push_back({dup_ai[k], P.dup_entry[k] / P.support, P.dup_entry[k]});
     std::stable_sort(terms.begin(), terms.end(), [](const Term &x, const Term &y) { return x.m < y.m; });
     for (const Term &t : terms) ++begin[pos[t.a] + 1];
-    for (size_t r = 0; r < reset.size(); ++r) begin[r + 1] += begin[r];
+    for (size_t r = 0; r < supported.size(); ++r) begin[r + 1] += begin[r];
     marker.resize(begin.back());
     coef.resize(begin.back());
     std::vector<int32_t> fill(begin.begin(), begin.end() - 1);

@@ -712,7 +712,7 @@ __device__ __forceinline__ void stream_collide_brick(const BrickLevel<T> &lv, co
             if (missing & (1u << q)) f[q] = C(aux_f[(int64_t)(base + row) * aux_stride<D>() + q]);
     }
     if (am) {   // uniform
-        // The rows of a brick's recorded nodes are one run of memory: kStageRows of them at a time
+        // The rows of a brick's recorded nodes are one run of memory: R of them at a time
         // go through LDS, and the lanes that hold nodes write the run in 16-byte units (8 in
         // BF16), so that a store is whole lines.  With a row per lane the four-level 3.3M-node
         // Smagorinsky step took 1.46 ms in FP32 and 2.89 in FP64, so 1.41 and 2.85

@@ -71,11 +71,10 @@ struct TransferTables {
 struct IbTables {
     int64_t n_markers = 0;
     int support = 0;            // (2 * stencil)^dims entries per marker
-    int64_t n_reset = 0;
     DevBuf node_ai;             // [n_markers][support] aux index, -1 for unused entries
     DevBuf weight;              // [n_markers][support] delta weight (double)
     DevBuf spread_row;          // [naux] place of a supported node in spread_begin, else -1
-    DevBuf spread_begin;        // [n_reset + 1] offsets into the spread arrays per supported node
+    DevBuf spread_begin;        // [supported nodes + 1] offsets of their terms in the spread arrays
     DevBuf spread_marker;       // marker of each spread term, ascending per node
     DevBuf spread_weight;       // its delta weight times the marker's area / (dt dx^(dims-1))
     DevBuf marker_vel;          // [n_markers][3]
@@ -135,16 +134,14 @@ struct LevelState {
     std::vector<int32_t> node_slot_h, node_aux_h;
     std::vector<uint32_t> missing_h;
     std::vector<uint8_t> aux_mark;   // kAux* roles per node (0: bulk)
-    // aux nodes of this level that the transfer from the coarser level writes (ghost targets) and
-    // reads (fallback rows, fine-to-coarse sources), and whether the transfer into the next finer
-    // level conflicts with them (writes a node the first touches, or reads a node it writes)
-    std::vector<int32_t> xfer_writes, xfer_reads;
+    // whether the transfer into the next finer level conflicts with the transfer from the coarser one
+    // on nodes of this level (writes a node that one touches, or reads a node it writes)
     bool xfer_overlap = false;
     // device
     DevBuf keys_d, bkeys_d, node_slot_d, slot_node_d, occ_d, nbr_d, auxmask_d, auxbase_d, aux_missing_d,
         aux_slot_d, node_aux_d, f_d[2], aux_f_d, aux_macro_d, aux_force_d,
         aux_macro_flag_d;   // [naux] 1: the aux collision records rho, u (fine-to-coarse sources)
-    // boundary tables per direction: aux index of node, partner aux index, slot
+    // tables of the launches per face, by direction: aux index of node, partner aux index, slot
     DevBuf bc_ai_d[7], bc_partner_d[7], bc_slot_d[7];
     DevBuf bc_u_d[7];   // [n][3] per-node boundary velocity of a profiled face (empty: uniform)
     int64_t bc_n[7] = {0, 0, 0, 0, 0, 0, 0};
@@ -153,7 +150,7 @@ struct LevelState {
     // 8 x (node whose pull or own population it is) + face (0: that node's pull; else its own
     // population of the opposite direction behind that face), -1: its own pull
     bool resolved = false;
-    std::vector<int64_t> res_node;    // boundary nodes, ascending
+    std::vector<int64_t> res_node;    // boundary nodes, ascending (both lists: during the build)
     std::vector<int64_t> res_code;    // [res_node][Q]
     DevBuf bnd_brick_d, bnd_src_d, bnd_face_d, bnd_wall_d;
     TransferTables xfer;

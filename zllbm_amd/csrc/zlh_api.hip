@@ -1204,6 +1204,7 @@ zlh_status upload_resolved(zlh_ctx *ctx, int level) {
     else build(k_bnd_regular<3>, k_bnd_entries<3>);
     ZLH_TRY(hipGetLastError());
     ZLH_TRY(hipStreamSynchronize(ctx->stream));   // the entries are freed on return
+    std::vector<int64_t>().swap(L.res_code);
     return ZLH_OK;
 }
 
@@ -1314,6 +1315,7 @@ zlh_status build_level_aux(zlh_ctx *ctx, int level) {
     std::vector<uint32_t> aux_missing(L.naux);
     L.node_aux_h.assign(L.n, -1);
     for (int64_t i : L.res_node) L.node_aux_h[i] = kResolvedBoundary;
+    std::vector<int64_t>().swap(L.res_node);
     for (int64_t k = 0; k < L.naux; ++k) {
         const int64_t i = aux_nodes[k];
         const int32_t slot = L.node_slot_h[i];
@@ -1354,13 +1356,7 @@ zlh_status build_level_aux(zlh_ctx *ctx, int level) {
     if ((s = upload(ctx, L.aux_missing_d, aux_missing))) return s;
     if ((s = upload(ctx, L.node_aux_d, L.node_aux_h))) return s;
     for (int dir = 1; dir <= 2 * dims; ++dir) {
-        std::vector<int32_t> ai, part, slot;
-        for (size_t k = 0; k < L.bnode[dir].size(); ++k) {
-            ai.push_back(L.node_aux_h[L.bnode[dir][k]]);
-            part.push_back(L.bpart[dir][k] >= 0 ? L.node_aux_h[L.bpart[dir][k]] : -1);
-            slot.push_back(L.node_slot_h[L.bnode[dir][k]]);
-        }
-        L.bc_n[dir] = (int64_t)ai.size();
+        L.bc_n[dir] = (int64_t)L.bnode[dir].size();
         const auto given = ctx->bc_node_u.find({level, dir});
         if (given != ctx->bc_node_u.end()) {
             if ((int64_t)given->second.size() != 3 * L.bc_n[dir])
@@ -1383,6 +1379,14 @@ zlh_status build_level_aux(zlh_ctx *ctx, int level) {
                 for (int c = 0; c < 3; ++c) ub.push_back(ctx->d.bc_value[dir][c] * fac);
             }
             if ((s = upload(ctx, L.bc_u_d[dir], ub))) return s;
+        }
+        for (DevBuf *d : {&L.bc_ai_d[dir], &L.bc_partner_d[dir], &L.bc_slot_d[dir]}) *d = DevBuf();
+        if (L.resolved) continue;   // no launches per face
+        std::vector<int32_t> ai, part, slot;
+        for (size_t k = 0; k < L.bnode[dir].size(); ++k) {
+            ai.push_back(L.node_aux_h[L.bnode[dir][k]]);
+            part.push_back(L.bpart[dir][k] >= 0 ? L.node_aux_h[L.bpart[dir][k]] : -1);
+            slot.push_back(L.node_slot_h[L.bnode[dir][k]]);
         }
         if ((s = upload(ctx, L.bc_ai_d[dir], ai))) return s;
         if ((s = upload(ctx, L.bc_partner_d[dir], part))) return s;
