@@ -1828,9 +1828,13 @@ zlh_status zlh_set_time_interpolation(zlh_ctx *ctx, int enable) {
     ctx->drop_graphs();   // captured graphs hold the other transfer schedule
     if (ctx->built) {
         // the synchronised rows from the state as it is now (after a whole background step, the
-        // rows the last transfers computed)
+        // rows the last transfers computed); without memory for them it stays off, as a step must
+        // not allocate
         zlh_status s = refresh_transfer_rows(ctx, -1);
-        if (s) return s;
+        if (s) {
+            ctx->time_interp = false;
+            return s;
+        }
         ZLH_TRY(hipStreamSynchronize(ctx->stream));
     }
     return ZLH_OK;
