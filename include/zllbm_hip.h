@@ -165,8 +165,10 @@ zlh_status zlh_transfer_to_coarse(zlh_ctx *ctx, int fine_level);
 /* background steps in the coarse-to-fine multi time stepping order (AmrManager::TimeMarching,
  * amr_manager.cpp:279-300; MultiTimeSteppingC2F, grid/grid_manager.cpp:997-1024) */
 zlh_status zlh_time_marching(zlh_ctx *ctx, int nsteps);
-/* zlh_time_marching replays pairs of background steps of refined grids as captured HIP graphs
- * (default on); off launches every kernel directly (no reference counterpart) */
+/* zlh_time_marching replays pairs of background steps as captured HIP graphs where that is faster
+ * (refined grids, and small single levels whose boundary conditions take launches of their own;
+ * default on); off launches every kernel directly (no reference counterpart).  Results are the
+ * same either way. */
 zlh_status zlh_graphs_enable(zlh_ctx *ctx, int enable);
 /* accepted from earlier callers, without effect: zlh_time_marching once ran each level's substeps
  * on a stream of its own; now the levels that step at the same time share a launch on the

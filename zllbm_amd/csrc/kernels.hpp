@@ -870,7 +870,8 @@ void k_stream_collide_mlp(Batch<FusedRun<T>> B) {
         // recorded nodes: post-stream values to their aux rows, except the missing sources (their
         // boundary / transfer values are there already).  The rows of a brick's nodes are one
         // run of memory: the wavefront writes it in 16-byte units from the staged brick, so
-        // every store is whole lines (a row per lane took 147 us on a 3M-node level, this 134)
+        // every store is whole lines (when a wave took two bricks, a row per lane took 147 us on a
+        // 3M-node level and this 134; with one brick a wave it is 129)
         if ((am >> lane) & 1ull) who[__popcll(am & ((1ull << lane) - 1ull))] = entry;
         wave_lds_sync();
         const int64_t base = table_load(t.auxbase, b);

@@ -404,7 +404,11 @@ __global__ __launch_bounds__(256) void k_mlp_eval_wave(const MlpDev *m, const fl
 // accumulator has to be cleared first.
 // ---------------------------------------------------------------------------------------------
 constexpr int kGradRow = 1412;       // kMlpParams + 1, rounded up to 16 bytes
-constexpr int kGradMaxBlocks = 256;  // rows: one workgroup per CU loops over a larger batch
+// Rows: one workgroup per CU, which loops over a larger batch.  The gradient kernels' registers (291 and
+// 323 of a SIMD's 512) leave one wavefront per SIMD, so a second workgroup would only queue behind the
+// first.  256 rows against 512, us: FP32 17.2 / 21.6 on 65,536 samples, 27.9 / 31.9 on 131,072, 174.7 / 178.7
+// on 2^20; BF16 operands 15.3 / 15.5, 21.0 / 27.8, 94.7 / 100.2.
+constexpr int kGradMaxBlocks = 256;
 static_assert(kGradRow >= kMlpParams + 1, "a row holds the gradient and the loss");
 
 __device__ __forceinline__ float wave_sum_f(float v) {
@@ -443,10 +447,11 @@ __device__ __forceinline__ void wave_lds_sync() {
 //              operands are turned around through a per-wavefront LDS tile (row stride 36 floats:
 //              16-byte reads of a row's half); the bias and output-weight gradients are the row
 //              sums of the same reads
-// 69 products of 64 cycles per 32 samples.  A batch of 4,096 takes 11.2 us (32 workgroups, bound by
-// the latency of one tile) and 2^20 samples 0.25 ms (4.1 G samples/s, bound by the matrix pipe and
-// its dependent chains at one wavefront per SIMD); one sample per lane with a wavefront reduction
-// and an atomic per parameter (1,409 of each) took 403 us and 8.4 ms.
+// 69 products of 64 cycles per 32 samples.  A batch of 4,096 takes 10.8 us (32 workgroups, bound by
+// the latency of one tile) and 2^20 samples 175 us (6.0 G samples/s).  The products fill the matrix
+// pipe for a third of that; the SiLU arithmetic on the vector units and the turns through LDS take the
+// rest, which one wavefront per SIMD does not overlap.  One sample per lane with a wavefront reduction and
+// an atomic per parameter (1,409 of each) took 403 us and 8.4 ms.
 constexpr int kTileStride = 36;
 struct alignas(16) GradTilesF {
     float d[kMlpH][kTileStride];     // layer delta [hidden][sample]: D2, then D1
@@ -645,7 +650,7 @@ __global__ __launch_bounds__(256) void k_grad_reduce(const float *__restrict__ p
 // tile is its own, so only the closing sum over the workgroup's wavefronts takes a barrier.  Bound
 // by the latency of a tile at one wavefront per SIMD: 70,000 samples (two trips of the grid) take
 // 24 us, where four barriers a tile and LDS atomics of 32 lanes to one address in the closing sum
-// took 44.5; 2^20 samples 0.18 ms an Adam step.
+// took 44.5; 2^20 samples take 95 us (122.7).
 // ---------------------------------------------------------------------------------------------
 constexpr int kGradTileStride = 72;   // LDS row stride of the transposed tiles, BF16 elements (144 B)
 

@@ -539,16 +539,16 @@ struct zlh_ctx {
     double timing_ms[16] = {};       // per level
     int64_t timing_launches[16] = {};
     DevBuf lattice_d;
-    // pinned staging of the downloads (download_nodes): two halves, grown to what a call needs up
-    // to 2 kStageBytes, freed with the context
-    // device workspace of the closure's gradient, training and evaluation, kept between calls up to
-    // kWorkBytes and freed with the context
-    DevBuf work;
     // held by the calls that use stage or work: callers on several threads take turns
     std::mutex scratch_m;
+    // pinned staging of the downloads (download_nodes): two halves, for the largest level up to
+    // 2 kStageBytes, freed with the context
     char *stage = nullptr;
     size_t stage_bytes = 0;
     hipEvent_t ev_stage[2] = {nullptr, nullptr};
+    // device workspace of the closure's gradient, training and evaluation, kept between calls up to
+    // kWorkBytes and freed with the context
+    DevBuf work;
     DevBuf mlp_d;           // MlpDev of the learned closure
     bool mlp_set = false;
     int mlp_train_form = ZLH_MLP_FP32;   // kernel of zlh_mlp_gradient / zlh_mlp_train

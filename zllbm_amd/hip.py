@@ -312,8 +312,8 @@ class Solver:
                                     f(model.fmax), float(model.nu_scale)))
 
     def mlp_gradient(self, params, x, t, form=MLP_FP32):
-        """Mean-squared-error gradient over all samples; form MLP_FP32 (vector units) or
-        MLP_BF16_MFMA (matrix cores, BF16 operands)."""
+        """Mean-squared-error gradient over all samples; form MLP_FP32 (FP32
+        operands) or MLP_BF16_MFMA (BF16 operands)."""
         f = lambda v: np.ascontiguousarray(v, np.float32)
         g = np.zeros(len(params), np.float32)
         loss = np.zeros(1, np.float32)

@@ -36,7 +36,7 @@ def main(argv=None):
     ap.add_argument("--per-ratio", type=int, default=200000, help="samples kept per snapshot and ratio")
     ap.add_argument("--train-steps", type=int, default=4000)
     ap.add_argument("--form", choices=("fp32", "bf16-mfma"), default="fp32",
-                    help="gradient kernel: vector units (FP32) or matrix cores (BF16 operands)")
+                    help="gradient kernel: FP32 or BF16 operands")
     ap.add_argument("--out", required=True)
     args = ap.parse_args(argv)
     t0 = time.time()
