@@ -147,3 +147,19 @@ def test_learned_closure_walls():
             out.append(s.macros(0)[1])
             assert (s.info(0)[1] > 0) == (precision == hip.FP32_SHIFTED and "lid" in names)
         assert np.linalg.norm(out[0] - out[1]) < 1e-4 * np.linalg.norm(out[1])
+
+
+@pytest.mark.parametrize("precision", [hip.FP64, hip.FP32_SHIFTED, hip.BF16_SHIFTED])
+@pytest.mark.parametrize("names", [("lid", "periodic"), ("walls", "lids"), ("lids", "periodic", "walls")])
+def test_conservation_sums_the_populations(names, precision):
+    """The sums on the device take the resolved pull as the downloads do: FP64 sums in another order,
+    some 500 values of at most 1/2."""
+    grid = g.uniform_grid(len(names), (17, 19) if len(names) == 2 else (6, 5, 9))
+    s = hip.Solver(grid, nu0=0.05, bc=_bc(names), precision=precision, collision=(hip.MRT,)).build()
+    s.init_macro(0, *_random_state(grid.levels[0].n, len(names), 3))
+    s.time_marching(5)
+    rho, u = s.macros(0)
+    want = np.zeros(4)
+    want[0] = rho.sum()
+    want[1:1 + len(names)] = (rho[:, None] * u).sum(0)
+    np.testing.assert_allclose(s.conservation(0), want, rtol=0, atol=1e-11)

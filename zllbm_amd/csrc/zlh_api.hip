@@ -248,12 +248,19 @@ __global__ void k_upload(BrickLevel<T> lv, const double *f_in, int64_t n, const 
     for (int q = 0; q < Q; ++q) fa[pop_at<Q>(q, slot)] = T(f[q]);
 }
 
+// BoundaryPull::brick of a node's brick: no rows where the level has none
+template <typename T>
+__device__ __forceinline__ int2 brick_rows(const BrickLevel<T> &lv, int64_t slot) {
+    return lv.bnd.brick ? lv.bnd.brick[slot >> 6] : make_int2(0, 0);
+}
+
 // post-stream population q of one node (brick slot, aux index or -1), in double and unshifted:
 // deferred nodes hold it in the aux array; a bulk node's is the pull of the post-collision value
 // at x - c_q from the buffer the last fused kernel read (before the first step, the uploaded
 // value itself)
+// (bnd: brick_rows of the node, read once for its Q values)
 template <int D, typename T, bool SHIFT>
-__device__ __forceinline__ double post_stream_value(const BrickLevel<T> &lv, int64_t slot, int32_t ai, int q,
+__device__ __forceinline__ double post_stream_value(const BrickLevel<T> &lv, int64_t slot, int32_t ai, int2 bnd, int q,
                                                     const T *last, const T *aux_f, int fresh) {
     using L = Lattice<D>;
     using B = Brick<D>;
@@ -263,9 +270,9 @@ __device__ __forceinline__ double post_stream_value(const BrickLevel<T> &lv, int
         v = double(aux_f[(int64_t)ai * aux_stride<D>() + q]);
     } else if (fresh || q == 0) {
         v = double(last[pop_at<Q>(q, slot)]);
-    } else if (lv.bnd.brick && (lv.bnd.brick[slot >> 6].y >> q & 1)) {
+    } else if (bnd.y >> q & 1) {
         // what the fused kernel pulled: a brick with resolved boundary nodes
-        const int64_t e = (int64_t)bnd_row(lv.bnd.brick[slot >> 6], q) * 64 + (slot & 63);
+        const int64_t e = (int64_t)bnd_row(bnd, q) * 64 + (slot & 63);
         T f = last[lv.bnd.src[e]];
         if (lv.bnd.face && lv.bnd.face[e]) f = wall_value<Q, T>(lv.bnd.wall, lv.bnd.face[e], q, f);
         v = double(f);
@@ -294,7 +301,9 @@ __global__ void k_materialize(BrickLevel<T> lv, const int32_t *node_slot, const 
     if (i >= n) return;
     const int32_t ai = node_aux[i];
     const int64_t slot = node_slot[i];
-    for (int q = 0; q < Q; ++q) out[q * n + i] = post_stream_value<D, T, SHIFT>(lv, slot, ai, q, last, aux_f, fresh);
+    const int2 bnd = brick_rows(lv, slot);
+    for (int q = 0; q < Q; ++q)
+        out[q * n + i] = post_stream_value<D, T, SHIFT>(lv, slot, ai, bnd, q, last, aux_f, fresh);
 }
 
 // Post-stream populations of the nodes [i0, i0 + m), [m][Q] double in key order (unshifted), into
@@ -311,9 +320,10 @@ __global__ __launch_bounds__(128) void k_rows_out(BrickLevel<T> lv, const int32_
     if (r < m) {
         const int32_t ai = node_aux[i0 + r];
         const int64_t slot = node_slot[i0 + r];
+        const int2 bnd = brick_rows(lv, slot);
 #pragma unroll
         for (int q = 0; q < Q; ++q)
-            tile[threadIdx.x * Q + q] = post_stream_value<D, T, SHIFT>(lv, slot, ai, q, last, aux_f, fresh);
+            tile[threadIdx.x * Q + q] = post_stream_value<D, T, SHIFT>(lv, slot, ai, bnd, q, last, aux_f, fresh);
     }
     __syncthreads();
     const int ne = (int)(m - r0 < 128 ? m - r0 : 128) * Q;
@@ -335,11 +345,12 @@ __global__ __launch_bounds__(256) void k_macros_out(BrickLevel<T> lv, const int3
     if (r >= m) return;
     const int32_t ai = node_aux[i0 + r];
     const int64_t slot = node_slot[i0 + r];
-    double s = post_stream_value<D, T, SHIFT>(lv, slot, ai, 0, last, aux_f, fresh);
+    const int2 bnd = brick_rows(lv, slot);
+    double s = post_stream_value<D, T, SHIFT>(lv, slot, ai, bnd, 0, last, aux_f, fresh);
     double j[3] = {0., 0., 0.};
 #pragma unroll
     for (int q = 1; q < L::Q; ++q) {
-        const double v = post_stream_value<D, T, SHIFT>(lv, slot, ai, q, last, aux_f, fresh);
+        const double v = post_stream_value<D, T, SHIFT>(lv, slot, ai, bnd, q, last, aux_f, fresh);
         s += v;
         j[0] += L::cx[q] * v;
         j[1] += L::cy[q] * v;
