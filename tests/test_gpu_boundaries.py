@@ -149,6 +149,27 @@ def test_learned_closure_walls():
         assert np.linalg.norm(out[0] - out[1]) < 1e-4 * np.linalg.norm(out[1])
 
 
+@pytest.mark.parametrize("names", [("periodic", "walls"), ("walls", "walls"), ("periodic", "lid"), ("channel", "walls")])
+def test_learned_closure_walls_2d(names):
+    """As above in 2D (its own kernels, with and without the table)."""
+    from tests.test_gpu_mlp import ROOT
+    import os
+    from zllbm_amd import closure
+    model = closure.ClosureModel.load(os.path.join(ROOT, "zllbm_amd", "data", "closure_turbulence.npz"))
+    grid = g.uniform_grid(2, (21, 18))
+    out = []
+    for precision in (hip.FP32_SHIFTED, hip.FP64):
+        s = hip.Solver(grid, nu0=0.01, bc=_bc(names), precision=precision, collision=(hip.MRT,), les=hip.LES_MLP,
+                       cs=0.1, mlp_operands=hip.MLP_OPERANDS_FP16).build()
+        s.mlp_set(model)
+        rho, u = _random_state(grid.levels[0].n, 2, 2)
+        s.init_macro(0, rho, u)
+        s.time_marching(11)
+        out.append(s.macros(0)[1])
+        assert (s.info(0)[1] > 0) == ("channel" in names or (precision == hip.FP32_SHIFTED and "lid" in names))
+    assert np.linalg.norm(out[0] - out[1]) < 1e-4 * np.linalg.norm(out[1])
+
+
 @pytest.mark.parametrize("precision", [hip.FP64, hip.FP32_SHIFTED, hip.BF16_SHIFTED])
 @pytest.mark.parametrize("names", [("lid", "periodic"), ("walls", "lids"), ("lids", "periodic", "walls")])
 def test_conservation_sums_the_populations(names, precision):
